@@ -15,8 +15,7 @@
 //     the same as a plain launch of that tile configuration.
 // A plan object keeps the descriptors on the device and can replay the
 // launch as a captured HIP graph.
-#include "internal.hpp"
-#include "gemm_tile.hpp"
+#include "gemm_plan.hpp"
 
 #include <algorithm>
 #include <cstring>
@@ -29,7 +28,7 @@ using namespace dev;
 namespace detail_batch {
 
 enum : int32_t {
-    F_A_K = 1, F_B_K = 2, F_VEC_A = 4, F_VEC_B = 8, F_VEC_C = 16, F_SMALL = 32
+    F_A_K = 1, F_B_K = 2, F_SMALL = 4
 };
 
 struct BatchDesc {
@@ -76,10 +75,9 @@ struct XcdSegs {
 
 // Kernel modes (a schedule choice the batch autotuner times; every mode
 // computes bit-identical results):
-//   0: one slab in flight, guarded element loads on edge tiles;
-//   1: one slab in flight, precomputed edge addressing (EdgeState);
-//   2: two slabs in flight, precomputed edge addressing;
-//   3: two slabs in flight, guarded element loads;
+//   0, 1: one slab in flight (two names from when edge tiles had two ways to
+//      load; the kernels are the same);
+//   2, 3: two slabs in flight (likewise);
 //   4: wave tiles (gemm_batch_wave_kernel);
 //   5: as 0, with registers capped for four workgroups per CU, the C tile
 //      pulled into L2 one slab ahead and C written through LDS in whole
@@ -94,8 +92,9 @@ constexpr int WAVE_MODE = 4;
 // Mode used until the autotuner runs: the one measured fastest on uneven
 // batches of 10,000 problems (dims log-uniform in [8, 512]), for both types.
 constexpr int default_mode(Dt) { return 8; }
+// Modes whose kernels are the same as another's: run as, and timed with, it.
+constexpr int mode_kernel(int mode) { return mode == 1 ? 0 : mode == 2 ? 3 : mode; }
 constexpr int mode_pf(int mode) { return (mode == 2 || mode == 3) ? 2 : 1; }
-constexpr bool mode_edge(int mode) { return mode == 1 || mode == 2; }
 constexpr int mode_waves(int mode) { return mode == 7 ? 5 : mode == 8 ? 6 : (mode == 5 || mode == 6) ? 4 : 1; }
 // The C tile fits the half-k stages only for FP32 (64 x 68 floats = two stages).
 template <typename T> constexpr bool mode_lds_epi(int mode) {
@@ -134,11 +133,10 @@ __attribute__((amdgpu_waves_per_eu(mode_waves(MODE)))) void gemm_batch_kernel(co
         p.m = d.m; p.n = d.n; p.k = d.k;
         p.lda = d.lda; p.ldb = d.ldb; p.c_si = d.c_si; p.c_sj = d.c_sj;
         p.alpha = (T)d.alpha; p.beta = (T)d.beta;
-        p.vec_a = (d.flags & F_VEC_A) != 0;
-        p.vec_b = (d.flags & F_VEC_B) != 0;
-        p.vec_c = (d.flags & F_VEC_C) != 0;
+        p.vec_a = p.vec_b = 0;      // loads go through buffer descriptors
+        p.vec_c = d.c_si == 1;
         const int64_t tm = w.tile % d.tiles_m, tn = w.tile / d.tiles_m;
-        gemm_tile<T, TL, A_K, B_K, mode_pf(MODE), mode_edge(MODE), mode_lds_epi<T>(MODE),
+        gemm_tile<T, TL, A_K, B_K, true, mode_pf(MODE), mode_lds_epi<T>(MODE),
                   mode_c_pf<T>(MODE)>(p, tm, tn, smem, sink);
         __syncthreads();
         if (!has_next) break;
@@ -208,21 +206,20 @@ __attribute__((amdgpu_waves_per_eu(mode_waves(MODE)))) void gemm_batch_dyn_kerne
         p.m = d.m; p.n = d.n; p.k = d.k;
         p.lda = d.lda; p.ldb = d.ldb; p.c_si = d.c_si; p.c_sj = d.c_sj;
         p.alpha = (T)d.alpha; p.beta = (T)d.beta;
-        p.vec_a = (d.flags & F_VEC_A) != 0;
-        p.vec_b = (d.flags & F_VEC_B) != 0;
-        p.vec_c = (d.flags & F_VEC_C) != 0;
+        p.vec_a = p.vec_b = 0;      // loads go through buffer descriptors
+        p.vec_c = d.c_si == 1;
         const int64_t tm = w.tile % d.tiles_m, tn = w.tile / d.tiles_m;
         constexpr int PF = mode_pf(MODE);
-        constexpr bool EG = mode_edge(MODE), LE = mode_lds_epi<T>(MODE), CP = mode_c_pf<T>(MODE);
+        constexpr bool LE = mode_lds_epi<T>(MODE), CP = mode_c_pf<T>(MODE);
         switch (variant_of(d.flags)) {
-        case 0: gemm_tile<T, Big, false, false, PF, EG, LE, CP>(p, tm, tn, smem, sink); break;
-        case 1: gemm_tile<T, Big, false, true, PF, EG, LE, CP>(p, tm, tn, smem, sink); break;
-        case 2: gemm_tile<T, Big, true, false, PF, EG, LE, CP>(p, tm, tn, smem, sink); break;
-        case 3: gemm_tile<T, Big, true, true, PF, EG, LE, CP>(p, tm, tn, smem, sink); break;
-        case 4: gemm_tile<T, Small, false, false, PF, EG, LE, CP>(p, tm, tn, smem, sink); break;
-        case 5: gemm_tile<T, Small, false, true, PF, EG, LE, CP>(p, tm, tn, smem, sink); break;
-        case 6: gemm_tile<T, Small, true, false, PF, EG, LE, CP>(p, tm, tn, smem, sink); break;
-        default: gemm_tile<T, Small, true, true, PF, EG, LE, CP>(p, tm, tn, smem, sink); break;
+        case 0: gemm_tile<T, Big, false, false, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
+        case 1: gemm_tile<T, Big, false, true, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
+        case 2: gemm_tile<T, Big, true, false, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
+        case 3: gemm_tile<T, Big, true, true, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
+        case 4: gemm_tile<T, Small, false, false, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
+        case 5: gemm_tile<T, Small, false, true, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
+        case 6: gemm_tile<T, Small, true, false, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
+        default: gemm_tile<T, Small, true, true, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
         }
         if (threadIdx.x == 0) shared_idx[0] = nn;
         __syncthreads();   // smem free for the next tile; nn visible
@@ -369,10 +366,8 @@ inline void variant_info(int mode, int v, const void*& fn, int& threads) {
         }
         abort_with(BLIS_INVALID_UKR_ID, "batch: wave variant");
     }
-    switch (mode) {
+    switch (mode_kernel(mode)) {
     case 0: fn = variant_fn<T, 0>(v); return;
-    case 1: fn = variant_fn<T, 1>(v); return;
-    case 2: fn = variant_fn<T, 2>(v); return;
     case 3: fn = variant_fn<T, 3>(v); return;
     case 5: fn = variant_fn<T, 5>(v); return;
     case 6: fn = variant_fn<T, 6>(v); return;
@@ -384,10 +379,8 @@ inline void variant_info(int mode, int v, const void*& fn, int& threads) {
 
 template <typename T>
 inline const void* dyn_fn(int mode) {
-    switch (mode) {
+    switch (mode_kernel(mode)) {
     case 0: return (const void*)&gemm_batch_dyn_kernel<T, 0>;
-    case 1: return (const void*)&gemm_batch_dyn_kernel<T, 1>;
-    case 2: return (const void*)&gemm_batch_dyn_kernel<T, 2>;
     case 3: return (const void*)&gemm_batch_dyn_kernel<T, 3>;
     case 5: return (const void*)&gemm_batch_dyn_kernel<T, 5>;
     case 6: return (const void*)&gemm_batch_dyn_kernel<T, 6>;
@@ -416,8 +409,6 @@ __global__ void batch_c_copy_kernel(const BatchDesc* __restrict__ descs, int nde
         }
     }
 }
-
-inline bool al16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 int cu_count() {
     static int n = 0;
@@ -476,7 +467,6 @@ struct BatchPlan {
 };
 
 static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipStream_t st) {
-    const int V = dt == Dt::F64 ? 2 : 4;
     auto* plan = new BatchPlan();
     plan->dt = dt;
     std::vector<BatchDesc> descs;
@@ -505,6 +495,11 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
             if (q.b.rs == 1) { d.ldb = q.b.cs; flags |= F_B_K; }
             else if (q.b.cs == 1) { d.ldb = q.b.rs; }
             else general = true;
+            // The kernels read through buffer descriptors; strides that do
+            // not allow it run as plain GEMMs.
+            if (!general)
+                general = !buf_ok(d.lda, (flags & F_A_K) ? q.k : q.m, 64, dt) ||
+                          !buf_ok(d.ldb, (flags & F_B_K) ? q.k : q.n, 64, dt);
         } else {
             d.lda = 1; d.ldb = 1;
         }
@@ -516,9 +511,6 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
         d.c_si = q.c.rs; d.c_sj = q.c.cs;
         d.m = (int32_t)q.m; d.n = (int32_t)q.n; d.k = (int32_t)q.k;
         d.alpha = q.alpha; d.beta = q.beta;
-        if (al16(d.a) && d.lda % V == 0) flags |= F_VEC_A;
-        if (al16(d.b) && d.ldb % V == 0) flags |= F_VEC_B;
-        if (al16(d.c) && d.c_si == 1 && d.c_sj % V == 0) flags |= F_VEC_C;
         // 32 x 32 tiles where they cover the problem at lower cost: a 32 x 32
         // tile was measured at about 0.4 of a 64 x 64 tile's time at equal k
         // (both latency-bound at these sizes), so it wins where it cuts the
@@ -1027,7 +1019,7 @@ static void plan_tune(BatchPlan* plan, int reps) {
         vbest[v] = default_mode(plan->dt);   // never the wave mode (it spans variants)
         vbest_ms[v] = 0.f;
         for (int mode = 0; mode < NMODE; ++mode) {
-            if (mode == WAVE_MODE || plan->grid[mode][v] == 0) continue;
+            if (mode == WAVE_MODE || mode != mode_kernel(mode) || plan->grid[mode][v] == 0) continue;
             const float ms = time_ms([&] { launch_variant(plan, mode, v, st); });
             if (mode == 0 || ms < vbest_ms[v]) { vbest_ms[v] = ms; vbest[v] = mode; }
         }
@@ -1040,7 +1032,7 @@ static void plan_tune(BatchPlan* plan, int reps) {
     int dbest = default_mode(plan->dt);
     float dbest_ms = 0.f;
     for (int mode = 0; mode < NMODE; ++mode) {
-        if (mode == WAVE_MODE || plan->dgrid[mode] == 0) continue;
+        if (mode == WAVE_MODE || mode != mode_kernel(mode) || plan->dgrid[mode] == 0) continue;
         const float ms = time_ms([&] { launch_dyn(plan, mode, st); });
         if (dbest_ms == 0.f || ms < dbest_ms) { dbest_ms = ms; dbest = mode; }
     }

@@ -24,39 +24,35 @@ using namespace dev;
 // Kernels
 // ---------------------------------------------------------------------------
 
-template <typename T, class TL, bool A_K, bool B_K>
-__global__ __launch_bounds__(TL::NT) void gemm_kernel(TileProblem<T> p, GridInfo g) {
+// One tile per workgroup. With gridDim.y > 1 each blockIdx.y is a k partition
+// of a split-k product: partition z covers k in [z*kchunk, min(k,
+// (z+1)*kchunk)) and stores alpha * A_z * B_z, without reading anything
+// there first, into its own m x n column-major slice of `parts` (ld = m).
+// splitk_reduce_kernel then forms C.
+template <typename T, class TL, bool A_K, bool B_K, bool BUF>
+__global__ __launch_bounds__(TL::NT) void gemm_kernel(TileProblem<T> p, GridInfo g,
+                                                      int64_t kchunk, T* parts) {
     __shared__ T smem[2 * TL::STAGE];
+    if (gridDim.y > 1) {
+        const int64_t z = blockIdx.y, k0 = z * kchunk;
+        p.a += A_K ? k0 : k0 * p.lda;
+        p.b += B_K ? k0 : k0 * p.ldb;
+        p.k = min(kchunk, p.k - k0);
+        p.c = parts + z * p.m * p.n;
+        p.c_si = 1;
+        p.c_sj = p.m;
+        p.vec_c = 1;
+        p.beta = T(0);
+    }
     int tm, tn;
     tile_coords(blockIdx.x, gridDim.x, g, tm, tn);
-    gemm_tile<T, TL, A_K, B_K>(p, tm, tn, smem);
-}
-
-// One k partition of a split-k product per blockIdx.y: partition z covers
-// k in [z*kchunk, min(k, (z+1)*kchunk)) and stores alpha * A_z * B_z, without
-// reading anything there first, into its own m x n column-major slice of
-// `parts` (ld = m). splitk_reduce_kernel then forms C.
-template <typename T, class TL, bool A_K, bool B_K>
-__global__ __launch_bounds__(TL::NT) void gemm_splitk_kernel(TileProblem<T> p, GridInfo g,
-                                                             int64_t kchunk, T* parts) {
-    __shared__ T smem[2 * TL::STAGE];
-    const int64_t z = blockIdx.y, k0 = z * kchunk;
-    p.a += A_K ? k0 : k0 * p.lda;
-    p.b += B_K ? k0 : k0 * p.ldb;
-    p.k = min(kchunk, p.k - k0);
-    p.c = parts + z * p.m * p.n;
-    p.c_si = 1;
-    p.c_sj = p.m;
-    p.beta = T(0);
-    int tm, tn;
-    tile_coords(blockIdx.x, gridDim.x, g, tm, tn);
-    gemm_tile<T, TL, A_K, B_K>(p, tm, tn, smem);
+    gemm_tile<T, TL, A_K, B_K, BUF>(p, tm, tn, smem);
 }
 
 // count products at fixed element strides, one per blockIdx.y:
 // C_z := beta*C_z + alpha*A_z*B_z with A_z = A + z*sa, B_z = B + z*sb,
 // C_z = C + z*sc.
-template <typename T, class TL, bool A_K, bool B_K>
+template <typename T, class TL, bool A_K, bool B_K, bool BUF>
 __global__ __launch_bounds__(TL::NT) void gemm_strided_kernel(TileProblem<T> p, GridInfo g,
                                                               int64_t sa, int64_t sb, int64_t sc) {
     __shared__ T smem[2 * TL::STAGE];
@@ -66,7 +62,7 @@ __global__ __launch_bounds__(TL::NT) void gemm_strided_kernel(TileProblem<T> p, 
     p.c += z * sc;
     int tm, tn;
     tile_coords(blockIdx.x, gridDim.x, g, tm, tn);
-    gemm_tile<T, TL, A_K, B_K>(p, tm, tn, smem);
+    gemm_tile<T, TL, A_K, B_K, BUF>(p, tm, tn, smem);
 }
 
 // C := beta*C + sum_z parts_z, partitions added in ascending z (a fixed
@@ -181,62 +177,52 @@ struct SplitK {
     void* ws = nullptr;
 };
 
-template <typename T, class TL>
-static void launch_tl(const TileProblem<T>& p, bool a_k, bool b_k, const GridInfo& g,
-                      int nblocks, const SplitK& sk, hipStream_t st) {
-    dim3 grid(nblocks), block(TL::NT);
-    if (sk.parts > 1) {
-        const dim3 grid2(nblocks, sk.parts);
-        T* ws = (T*)sk.ws;
-        if (!a_k && !b_k)
-            hipLaunchKernelGGL((gemm_splitk_kernel<T, TL, false, false>), grid2, block, 0, st, p, g,
-                               sk.kchunk, ws);
-        else if (!a_k && b_k)
-            hipLaunchKernelGGL((gemm_splitk_kernel<T, TL, false, true>), grid2, block, 0, st, p, g,
-                               sk.kchunk, ws);
-        else if (a_k && !b_k)
-            hipLaunchKernelGGL((gemm_splitk_kernel<T, TL, true, false>), grid2, block, 0, st, p, g,
-                               sk.kchunk, ws);
-        else
-            hipLaunchKernelGGL((gemm_splitk_kernel<T, TL, true, true>), grid2, block, 0, st, p, g,
-                               sk.kchunk, ws);
-        HIP_CHECK(hipGetLastError());
-        return;
-    }
+template <typename T, class TL, bool BUF>
+static void launch_tl(const TileProblem<T>& p, bool a_k, bool b_k, GridInfo g, const SplitK& sk,
+                      hipStream_t st) {
+    g.grid_m = (int)((p.m + TL::BM - 1) / TL::BM);
+    g.grid_n = (int)((p.n + TL::BN - 1) / TL::BN);
+    if (g.group_m < 1) g.group_m = 1;
+    const dim3 grid(g.grid_m * g.grid_n, sk.parts), block(TL::NT);
+    T* ws = (T*)sk.ws;
     if (!a_k && !b_k)
-        hipLaunchKernelGGL((gemm_kernel<T, TL, false, false>), grid, block, 0, st, p, g);
+        hipLaunchKernelGGL((gemm_kernel<T, TL, false, false, BUF>), grid, block, 0, st, p, g,
+                           sk.kchunk, ws);
     else if (!a_k && b_k)
-        hipLaunchKernelGGL((gemm_kernel<T, TL, false, true>), grid, block, 0, st, p, g);
+        hipLaunchKernelGGL((gemm_kernel<T, TL, false, true, BUF>), grid, block, 0, st, p, g,
+                           sk.kchunk, ws);
     else if (a_k && !b_k)
-        hipLaunchKernelGGL((gemm_kernel<T, TL, true, false>), grid, block, 0, st, p, g);
+        hipLaunchKernelGGL((gemm_kernel<T, TL, true, false, BUF>), grid, block, 0, st, p, g,
+                           sk.kchunk, ws);
     else
-        hipLaunchKernelGGL((gemm_kernel<T, TL, true, true>), grid, block, 0, st, p, g);
+        hipLaunchKernelGGL((gemm_kernel<T, TL, true, true, BUF>), grid, block, 0, st, p, g,
+                           sk.kchunk, ws);
     HIP_CHECK(hipGetLastError());
 }
 
+// Every tile of the table reads its operands through buffer descriptors. A
+// problem whose strides do not allow that runs on one of two tiles built
+// without them, a large and a small one: the tile never changes the result.
 template <typename T>
 static void launch_tile(int tile, const TileProblem<T>& p, bool a_k, bool b_k,
-                        GridInfo g, const SplitK& sk, hipStream_t st) {
+                        const GridInfo& g, const SplitK& sk, hipStream_t st) {
     const TileShape& ts = tile_shape(dt_of<T>(), tile);
-    g.grid_m = (int)((p.m + ts.bm - 1) / ts.bm);
-    g.grid_n = (int)((p.n + ts.bn - 1) / ts.bn);
-    if (g.group_m < 1) g.group_m = 1;
-    const int nblocks = g.grid_m * g.grid_n;
-    if constexpr (std::is_same<T, double>::value) {
-        switch (tile) {
-#define BLIS_AMD_CASE(idx, BM, BN, BK, WM, WN) \
-        case idx: launch_tl<double, TileCfg<double, BM, BN, BK, WM, WN>>(p, a_k, b_k, g, nblocks, sk, st); return;
-        BLIS_AMD_TILES_F64(BLIS_AMD_CASE)
-#undef BLIS_AMD_CASE
-        }
-    } else {
-        switch (tile) {
-#define BLIS_AMD_CASE(idx, BM, BN, BK, WM, WN) \
-        case idx: launch_tl<float, TileCfg<float, BM, BN, BK, WM, WN>>(p, a_k, b_k, g, nblocks, sk, st); return;
-        BLIS_AMD_TILES_F32(BLIS_AMD_CASE)
-#undef BLIS_AMD_CASE
-        }
+    if (!buf_problem(p, a_k, b_k, ts.bm, ts.bn, ts.bk)) {
+        constexpr int BK = std::is_same<T, double>::value ? 16 : 32;
+        if (ts.bm >= 64)
+            launch_tl<T, TileCfg<T, 128, 64, BK, 32, 32>, false>(p, a_k, b_k, g, sk, st);
+        else
+            launch_tl<T, TileCfg<T, 32, 32, BK, 16, 16>, false>(p, a_k, b_k, g, sk, st);
+        return;
     }
+#define BLIS_AMD_CASE(idx, BM, BN, BK, WM, WN) \
+    case idx: launch_tl<T, TileCfg<T, BM, BN, BK, WM, WN>, true>(p, a_k, b_k, g, sk, st); return;
+    if constexpr (std::is_same<T, double>::value) {
+        switch (tile) { BLIS_AMD_TILES_F64(BLIS_AMD_CASE) }
+    } else {
+        switch (tile) { BLIS_AMD_TILES_F32(BLIS_AMD_CASE) }
+    }
+#undef BLIS_AMD_CASE
     abort_with(BLIS_INVALID_UKR_ID, "gemm: tile index out of range");
 }
 
@@ -377,20 +363,13 @@ static void launch_plan(Dt dt, Plan& pl, const GemmConfig& cfg, double alpha, do
     // Split-k: each partition a full product into its own m x n slice of
     // scratch, then one reduction into C.
     SplitK sk = split_params(pl.k, cfg.split_k);
-    if (gemm_sup_deep_k(tile, sk.parts, pl.k)) {
-        gemm_sup_run(dt, pl, alpha, beta, st);
-        return;
-    }
+    if (gemm_sup_deep_k(tile, sk.parts, pl.k) && gemm_sup_run(dt, pl, alpha, beta, st)) return;
     const size_t es = dt_size(dt);
     if (sk.parts > 1) sk.ws = sc.take((size_t)sk.parts * pl.m * pl.n * es, 17);
     if (dt == Dt::F64) {
-        TileProblem<double> p = make_problem<double>(pl, alpha, beta);
-        if (sk.parts > 1) p.vec_c = pl.m % Mma<double>::V == 0;
-        launch_tile<double>(tile, p, pl.a_k, pl.b_k, g, sk, st);
+        launch_tile<double>(tile, make_problem<double>(pl, alpha, beta), pl.a_k, pl.b_k, g, sk, st);
     } else {
-        TileProblem<float> p = make_problem<float>(pl, alpha, beta);
-        if (sk.parts > 1) p.vec_c = pl.m % Mma<float>::V == 0;
-        launch_tile<float>(tile, p, pl.a_k, pl.b_k, g, sk, st);
+        launch_tile<float>(tile, make_problem<float>(pl, alpha, beta), pl.a_k, pl.b_k, g, sk, st);
     }
     if (sk.parts > 1) {
         const int gr = grid_for(pl.m * pl.n);
@@ -419,10 +398,8 @@ void gemm_run(const GemmDesc& d, const GemmConfig* cfg, hipStream_t st) {
     // the table's tiles instead).
     if (cfg == &g_override && g_override.tile < 0 && g_override.split_k <= 1 &&
         !pl.a_packed && !pl.b_packed && gemm_sup_applies(pl.m, pl.n, pl.k) &&
-        selector_mode() != SELECT_EXHAUSTIVE) {
-        gemm_sup_run(d.dt, pl, d.alpha, d.beta, st);
+        selector_mode() != SELECT_EXHAUSTIVE && gemm_sup_run(d.dt, pl, d.alpha, d.beta, st))
         return;
-    }
     GemmConfig picked;
     if (cfg == &g_override && g_override.tile < 0) {
         // No configuration given: the selector (heuristic, learned or
@@ -445,23 +422,44 @@ void gemm_run(const GemmDesc& d, const GemmConfig* cfg, hipStream_t st) {
     launch_plan(d.dt, pl, *cfg, d.alpha, d.beta, sc, st);
 }
 
-template <typename T, class TL>
-static void launch_strided(const TileProblem<T>& p, bool a_k, bool b_k, const GridInfo& g,
-                           int count, int64_t sa, int64_t sb, int64_t sc, hipStream_t st) {
+template <typename T, class TL, bool BUF>
+static void launch_strided_tl(const TileProblem<T>& p, bool a_k, bool b_k, const GridInfo& g,
+                              int count, int64_t sa, int64_t sb, int64_t sc, hipStream_t st) {
     const dim3 grid(g.grid_m * g.grid_n, count), block(TL::NT);
     if (!a_k && !b_k)
-        hipLaunchKernelGGL((gemm_strided_kernel<T, TL, false, false>), grid, block, 0, st, p, g,
-                           sa, sb, sc);
+        hipLaunchKernelGGL((gemm_strided_kernel<T, TL, false, false, BUF>), grid, block, 0, st, p,
+                           g, sa, sb, sc);
     else if (!a_k && b_k)
-        hipLaunchKernelGGL((gemm_strided_kernel<T, TL, false, true>), grid, block, 0, st, p, g,
-                           sa, sb, sc);
+        hipLaunchKernelGGL((gemm_strided_kernel<T, TL, false, true, BUF>), grid, block, 0, st, p,
+                           g, sa, sb, sc);
     else if (a_k && !b_k)
-        hipLaunchKernelGGL((gemm_strided_kernel<T, TL, true, false>), grid, block, 0, st, p, g,
-                           sa, sb, sc);
+        hipLaunchKernelGGL((gemm_strided_kernel<T, TL, true, false, BUF>), grid, block, 0, st, p,
+                           g, sa, sb, sc);
     else
-        hipLaunchKernelGGL((gemm_strided_kernel<T, TL, true, true>), grid, block, 0, st, p, g,
+        hipLaunchKernelGGL((gemm_strided_kernel<T, TL, true, true, BUF>), grid, block, 0, st, p, g,
                            sa, sb, sc);
     HIP_CHECK(hipGetLastError());
+}
+
+// The 32x32 tile (tile 4 of both tables): these batches are of small
+// products, several hundred tiles in all.
+template <typename T>
+static void launch_strided(const Plan& pl, double alpha, double beta, int count, int64_t sa,
+                           int64_t sb, int64_t sc, hipStream_t st) {
+    constexpr int V = Mma<T>::V;
+    using TL = TileCfg<T, 32, 32, std::is_same<T, double>::value ? 16 : 32, 16, 16>;
+    GridInfo g{};
+    g.group_m = 8;
+    g.xcd_remap = 1;
+    g.grid_m = (int)((pl.m + TL::BM - 1) / TL::BM);
+    g.grid_n = (int)((pl.n + TL::BN - 1) / TL::BN);
+    TileProblem<T> p = make_problem<T>(pl, alpha, beta);
+    p.vec_a = p.vec_a && sa % V == 0;
+    p.vec_b = p.vec_b && sb % V == 0;
+    if (buf_problem(p, pl.a_k, pl.b_k, TL::BM, TL::BN, TL::BK))
+        launch_strided_tl<T, TL, true>(p, pl.a_k, pl.b_k, g, count, sa, sb, sc, st);
+    else
+        launch_strided_tl<T, TL, false>(p, pl.a_k, pl.b_k, g, count, sa, sb, sc, st);
 }
 
 void gemm_strided_run(const GemmDesc& d, int count, int64_t sa, int64_t sb, int64_t sc,
@@ -472,30 +470,8 @@ void gemm_strided_run(const GemmDesc& d, int count, int64_t sa, int64_t sb, int6
     Plan pl = layout(d);
     if (pl.a_packed || pl.b_packed)
         abort_with(BLIS_INVALID_UKR_ID, "gemm strided: operands need a unit stride");
-    // The 32x32 tile (tile 4 of both tables): these batches are of small
-    // products, several hundred tiles in all.
-    GridInfo g{};
-    g.group_m = 8;
-    g.xcd_remap = 1;
-    g.grid_m = (int)((pl.m + 31) / 32);
-    g.grid_n = (int)((pl.n + 31) / 32);
-    if (d.dt == Dt::F64) {
-        constexpr int V = Mma<double>::V;
-        TileProblem<double> p = make_problem<double>(pl, d.alpha, d.beta);
-        p.vec_a = p.vec_a && sa % V == 0;
-        p.vec_b = p.vec_b && sb % V == 0;
-        p.vec_c = p.vec_c && sc % V == 0;
-        launch_strided<double, TileCfg<double, 32, 32, 16, 16, 16>>(p, pl.a_k, pl.b_k, g, count,
-                                                                   sa, sb, sc, st);
-    } else {
-        constexpr int V = Mma<float>::V;
-        TileProblem<float> p = make_problem<float>(pl, d.alpha, d.beta);
-        p.vec_a = p.vec_a && sa % V == 0;
-        p.vec_b = p.vec_b && sb % V == 0;
-        p.vec_c = p.vec_c && sc % V == 0;
-        launch_strided<float, TileCfg<float, 32, 32, 32, 16, 16>>(p, pl.a_k, pl.b_k, g, count,
-                                                                 sa, sb, sc, st);
-    }
+    if (d.dt == Dt::F64) launch_strided<double>(pl, d.alpha, d.beta, count, sa, sb, sc, st);
+    else launch_strided<float>(pl, d.alpha, d.beta, count, sa, sb, sc, st);
 }
 
 // ---------------------------------------------------------------------------

@@ -117,6 +117,21 @@ inline bool vec_ok(const void* ptr, bool packed, int64_t ld, Dt dt) {
     return (packed || aligned16(ptr)) && ld % V == 0;
 }
 
+// Whether a tile kernel may read an operand (contiguous extent `run`, `ld`
+// between lines, `lines` of them in a slab) through a buffer descriptor:
+// lines that do not overlap or run backwards, so that everything past the
+// last element is past the descriptor's end, and 32-bit byte offsets.
+inline bool buf_ok(int64_t ld, int64_t run, int lines, Dt dt) {
+    return ld >= run && ld <= (((int64_t)1 << 32) - 65536) / (lines * (int64_t)dt_size(dt));
+}
+
+// The same for both operands of a problem on a bm x bn x bk tile.
+template <typename T>
+inline bool buf_problem(const TileProblem<T>& p, bool a_k, bool b_k, int bm, int bn, int bk) {
+    return buf_ok(p.lda, a_k ? p.k : p.m, a_k ? bm : bk, dt_of<T>()) &&
+           buf_ok(p.ldb, b_k ? p.k : p.n, b_k ? bn : bk, dt_of<T>());
+}
+
 template <typename T>
 inline TileProblem<T> make_problem(const Plan& pl, double alpha, double beta) {
     constexpr int V = Mma<T>::V;
@@ -128,17 +143,18 @@ inline TileProblem<T> make_problem(const Plan& pl, double alpha, double beta) {
     p.alpha = (T)alpha; p.beta = (T)beta;
     p.vec_a = aligned16(pl.a) && (pl.lda % V == 0);
     p.vec_b = aligned16(pl.b) && (pl.ldb % V == 0);
-    p.vec_c = aligned16(pl.c) && pl.c_si == 1 && (pl.c_sj % V == 0);
+    p.vec_c = pl.c_si == 1;
     return p;
 }
 
 // The single-call small-problem path (sup.hip): applies to m, n, k all at
 // most SMALL_GEMM_MAX_DIM with k > 64; the plan's operands must have a unit
 // stride. gemm_sup_deep_k: the 32 x 32 table tile over k > 64 in one
-// partition runs as the same kernel. BLIS_AMD_SUP=0 in the environment
-// turns both off (read once).
+// partition runs as the same kernel. gemm_sup_run returns false, having done
+// nothing, when the strides do not allow its loads. BLIS_AMD_SUP=0 in the
+// environment turns both off (read once).
 bool gemm_sup_applies(int64_t m, int64_t n, int64_t k);
 bool gemm_sup_deep_k(int tile, int parts, int64_t k);
-void gemm_sup_run(Dt dt, const Plan& pl, double alpha, double beta, hipStream_t st);
+bool gemm_sup_run(Dt dt, const Plan& pl, double alpha, double beta, hipStream_t st);
 
 } // namespace blis_amd

@@ -41,6 +41,10 @@ namespace dev {
 typedef double d2_t __attribute__((ext_vector_type(2)));
 typedef double d4_t __attribute__((ext_vector_type(4)));
 typedef float  f4_t __attribute__((ext_vector_type(4)));
+// 16-byte vectors at element alignment, for C: gfx950 takes vector accesses
+// at any dword address, so a column of C needs no 16-byte alignment.
+typedef d2_t d2u_t __attribute__((aligned(8)));
+typedef f4_t f4u_t __attribute__((aligned(4)));
 
 template <typename T> struct Mma;
 // Operand layout (both types, measured on gfx950): lane l supplies
@@ -51,6 +55,7 @@ template <typename T> struct Mma;
 template <> struct Mma<double> {
     using acc_t = d4_t;
     using vec_t = d2_t;             // 16-byte vector
+    using uvec_t = d2u_t;           // the same at element alignment
     static constexpr int V = 2;     // elements per 16-byte vector
     __device__ static inline acc_t mma(double a, double b, acc_t c) {
         return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
@@ -60,6 +65,7 @@ template <> struct Mma<double> {
 template <> struct Mma<float> {
     using acc_t = f4_t;
     using vec_t = f4_t;
+    using uvec_t = f4u_t;
     static constexpr int V = 4;
     __device__ static inline acc_t mma(float a, float b, acc_t c) {
         return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -81,7 +87,6 @@ struct TileCfg {
     // pad for FP64 was measured to raise bank conflicts: it costs the 16-byte
     // alignment of the fragment reads).
     static constexpr int PAD = V;
-    static constexpr bool LDS_VEC = (PAD % V) == 0;   // rows start 16-byte aligned
     static constexpr int LDA = BM + PAD;
     static constexpr int LDB = BN + PAD;
     static constexpr int A_ELEMS = BK * LDA;
@@ -110,259 +115,129 @@ struct TileProblem {
     int64_t  lda, ldb;
     int64_t  c_si, c_sj;
     T        alpha, beta;
-    int      vec_a, vec_b, vec_c;   // 16-byte vector access allowed
+    int      vec_a, vec_b;   // 16-byte alignment of A and B (loads without a descriptor)
+    int      vec_c;          // c_si == 1: C is stored in vectors
 };
 
-// Addressing of one operand in an edge tile (or a partial last k slab),
-// computed once per tile. The operand is X_eff, rows x K, with
-// X_eff(r, p) = x[p + r*ld] when K_CONTIG, else x[r + p*ld]; the tile covers
-// rows [row0, row0 + ROWS). Each thread owns NV 16-byte vectors of a slab,
-// in the same thread -> element order as the fast path and the LDS stores.
-// Elements outside the matrix are loaded from a clamped address and replaced
-// by zero, so no load sits behind a per-lane branch. A wave uses 16-byte
-// loads whenever none of its lanes straddles the matrix edge (a wave-uniform
-// vote), otherwise element loads.
-template <typename T, class TL, int ROWS, bool K_CONTIG, int NV>
-struct EdgeState {
+// One operand of a tile, read a k slab at a time. The operand is X_eff,
+// rows x K, with X_eff(r, p) = x[p + r*ld] when K_CONTIG, else x[r + p*ld];
+// the tile covers rows [row0, row0 + ROWS). Each thread owns NV 16-byte
+// vectors of a slab, between their load and their LDS store.
+//
+// BUF: the slab is read through a buffer descriptor whose base moves with
+// the slab (scalar arithmetic) and whose extent ends at the operand's last
+// element, so every lane of every tile issues the same 16-byte loads at the
+// same offsets, with no branch, no clamp and no 64-bit vector address: the
+// hardware returns zero past the end. What else an edge tile reads between
+// the operand's first and last element (the next column's rows, a row's
+// padding) lands in tile rows outside the matrix, which feed only outputs
+// that are never stored; the k positions past K of a K_CONTIG operand, which
+// every output sums over, are zeroed on the way to LDS. Buffer loads need
+// 4-byte alignment only, so odd leading dimensions take the same path. It
+// needs ld >= the contiguous extent and slab offsets below 2^32 bytes
+// (buf_ok in gemm_plan.hpp). Against 64-bit addresses with element loads on
+// edge and unaligned tiles (device time): 1999 x 1501 x 1003 T/N on odd
+// leading dimensions 150 against 170 us, 512^3 12.2 against 13.5 us, the
+// 10,000-problem FP64 batch 1546 against 1739 us (its 64 x 64 kernels no
+// longer spill); 8192^3, all interior, is unchanged.
+// Not BUF (negative, overlapping or very large strides): 16-byte loads for
+// slabs wholly inside an aligned operand, element loads behind bounds checks
+// otherwise.
+template <typename T, class TL, int ROWS, bool K_CONTIG, int NV, bool BUF>
+struct SlabLoader {
     using vec_t = typename Mma<T>::vec_t;
     static constexpr int V = TL::V;
+    static constexpr int LD = ROWS + TL::PAD;   // LDS row pitch
+    // Vectors along the contiguous direction, and slab lines between a
+    // thread's consecutive vectors.
+    static constexpr int CV = K_CONTIG ? TL::BK / V : ROWS / V;
+    static constexpr int LINES = TL::NT / CV;
+    static_assert(TL::NT % CV == 0, "a thread's vectors must be whole lines apart");
+    vec_t r[NV];
     const T* x;
-    int64_t ld, K, klast;          // klast = (K-1)*ld (R_CONTIG)
-    bool vec;                      // 16-byte access allowed (aligned x, ld % V == 0)
-    int64_t rows;
-    int64_t off[NV];               // K_CONTIG: clamped row * ld; R_CONTIG: kk * ld
-    int sub[NV];                   // K_CONTIG: k offset of the vector; R_CONTIG: kk
-    int r0[NV];                    // R_CONTIG: first row of the vector
-    unsigned rmask[NV];            // rows inside the matrix (bit e for element e)
-    bool vecw[NV];                 // R_CONTIG: the whole wave may use vector loads
+    int64_t ld, K, rows, row0;
+    int vec;
+    // BUF: start of the next slab to load, bytes from there to the operand's
+    // end, and the thread's first offset.
+    const char* base;
+    int64_t left;
+    uint32_t off0;
 
     __device__ inline void init(const T* x_, int64_t rows_, int64_t K_, int64_t ld_, int vec_,
-                                int64_t row0, int tid) {
-        x = x_; ld = ld_; K = K_; vec = vec_ != 0; rows = rows_;
-        klast = (K - 1) * ld;
+                                int64_t row0_, int tid) {
+        x = x_; ld = ld_; K = K_; rows = rows_; row0 = row0_; vec = vec_;
+        if constexpr (BUF) {
+            constexpr int ES = (int)sizeof(T);
+            const int c = tid % CV, l = tid / CV;
+            off0 = (uint32_t)l * ((uint32_t)ld * ES) + (uint32_t)(c * 16);
+            base = (const char*)(x + (K_CONTIG ? row0 * ld : row0));
+            left = (K_CONTIG ? (rows - 1 - row0) * ld + K : (K - 1) * ld + (rows - row0)) * ES;
+        }
+    }
+
+    // Load the slab at k0; BUF loaders are called for consecutive slabs.
+    __device__ inline void load(int64_t k0, int tid) {
+        if constexpr (BUF) {
+            const uint32_t n = left > 0xFFFFFFFFll ? 0xFFFFFFFFu : (uint32_t)left;
+            auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)n, 0x00020000);
+            const uint32_t step = (uint32_t)LINES * ((uint32_t)ld * (uint32_t)sizeof(T));
 #pragma unroll
-        for (int q = 0; q < NV; ++q) {
-            const int v = tid + q * TL::NT;
-            if constexpr (K_CONTIG) {
-                const int kc = v % (TL::BK / V), ii = v / (TL::BK / V);
-                const int64_t r = row0 + ii;
-                off[q] = (r < rows ? r : rows - 1) * ld;
-                sub[q] = kc * V;
-                rmask[q] = (r < rows) ? 0xFu : 0u;
-            } else {
-                const int ic = v % (ROWS / V), kk = v / (ROWS / V);
-                const int64_t r = row0 + (int64_t)ic * V;
-                off[q] = (int64_t)kk * ld;
-                sub[q] = kk;
-                unsigned m = 0;
+            for (int q = 0; q < NV; ++q) {
+                auto t = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(off0 + q * step), 0, 0);
+                r[q] = __builtin_bit_cast(vec_t, t);
+            }
+            const int64_t adv = (K_CONTIG ? (int64_t)TL::BK : TL::BK * ld) * (int64_t)sizeof(T);
+            base += adv;
+            left -= adv;
+        } else {
+            const bool whole = vec && row0 + ROWS <= rows && k0 + TL::BK <= K;   // uniform
 #pragma unroll
-                for (int e = 0; e < V; ++e) m |= (r + e < rows ? 1u : 0u) << e;
-                rmask[q] = m;
-                r0[q] = (int)r;
-                const bool full = r + V <= rows, none = r >= rows && rows >= V;
-                vecw[q] = __all((vec && (full || none)) ? 1 : 0) != 0;
+            for (int q = 0; q < NV; ++q) {
+                const int v = tid + q * TL::NT;
+                const int c = v % CV, l = v / CV;
+                const int64_t row = row0 + (K_CONTIG ? l : c * V), pk = k0 + (K_CONTIG ? c * V : l);
+                const T* src = K_CONTIG ? x + pk + row * ld : x + row + pk * ld;
+                if (whole) {
+                    r[q] = *reinterpret_cast<const vec_t*>(src);
+                    continue;
+                }
+                const int64_t run = K_CONTIG ? K - pk : rows - row;   // elements left along it
+                const bool line = K_CONTIG ? row < rows : pk < K;
+                if (vec && line && run >= V) {
+                    r[q] = *reinterpret_cast<const vec_t*>(src);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < V; ++e) {
+                        T val = T(0);
+                        if (line && e < run) val = src[e];
+                        r[q][e] = val;
+                    }
+                }
             }
         }
     }
 
-    template <int NR>
-    __device__ inline void load(vec_t (&r)[NR], int64_t k0) const {
-        static_assert(NR == NV, "register count");
+    // Store the slab at k0 into an LDS stage, k-major.
+    __device__ inline void store(T* S, int64_t k0, int tid) {
+        if constexpr (BUF && K_CONTIG) {
+            if (k0 + TL::BK > K) {
+                const int kleft = (int)(K - k0);
 #pragma unroll
-        for (int q = 0; q < NV; ++q) {
-            if constexpr (K_CONTIG) {
-                const int64_t pk = k0 + sub[q];
-                const T* row = x + off[q];
-                if (vec && k0 + TL::BK <= K) {
-                    const vec_t t = *reinterpret_cast<const vec_t*>(row + pk);
-#pragma unroll
-                    for (int e = 0; e < V; ++e) r[q][e] = rmask[q] ? t[e] : T(0);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < V; ++e) {
-                        const bool kin = pk + e < K;
-                        const T val = row[kin ? pk + e : K - 1];
-                        r[q][e] = (rmask[q] && kin) ? val : T(0);
-                    }
-                }
-            } else {
-                const bool kin = k0 + sub[q] < K;
-                const T* col = x + (kin ? k0 * ld + off[q] : klast);
-                if (vecw[q]) {
-                    // rows r0 .. r0+V-1 all inside (vector start r0), or all
-                    // outside (any aligned in-bounds vector: start 0)
-                    const int rb = (rmask[q] & 1u) ? r0[q] : 0;
-                    const vec_t t = *reinterpret_cast<const vec_t*>(col + rb);
+                for (int q = 0; q < NV; ++q)
 #pragma unroll
                     for (int e = 0; e < V; ++e)
-                        r[q][e] = (kin && ((rmask[q] >> e) & 1u)) ? t[e] : T(0);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < V; ++e) {
-                        const int64_t ri = r0[q] + e;
-                        const T val = col[ri < rows ? ri : rows - 1];
-                        r[q][e] = (kin && ((rmask[q] >> e) & 1u)) ? val : T(0);
-                    }
-                }
+                        if ((tid % CV) * V + e >= kleft) r[q][e] = T(0);
             }
         }
-    }
-};
-
-// Registers holding one slab of A between its global load and LDS store.
-template <typename T, class TL, bool A_K>
-struct ALoader {
-    using vec_t = typename Mma<T>::vec_t;
-    static constexpr int V = TL::V;
-    vec_t r[TL::NVA];
-
-    // Edge tile or partial slab, element by element behind bounds checks.
-    __device__ inline void load_guarded(const TileProblem<T>& p, int64_t m0, int64_t k0, int tid) {
 #pragma unroll
-        for (int q = 0; q < TL::NVA; ++q) {
+        for (int q = 0; q < NV; ++q) {
             const int v = tid + q * TL::NT;
-            if constexpr (!A_K) {
-                const int ic = v % (TL::BM / V), kk = v / (TL::BM / V);
-                const int64_t i = m0 + ic * V, pk = k0 + kk;
-                const T* src = p.a + i + pk * p.lda;
-                if (p.vec_a && pk < p.k && i + V <= p.m) {
-                    r[q] = *reinterpret_cast<const vec_t*>(src);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < V; ++e) {
-                        T x = T(0);
-                        if (pk < p.k && i + e < p.m) x = src[e];
-                        r[q][e] = x;
-                    }
-                }
+            const int c = v % CV, l = v / CV;
+            if constexpr (!K_CONTIG) {
+                *reinterpret_cast<vec_t*>(S + l * LD + c * V) = r[q];
             } else {
-                const int kc = v % (TL::BK / V), ii = v / (TL::BK / V);
-                const int64_t i = m0 + ii, pk = k0 + kc * V;
-                const T* src = p.a + pk + i * p.lda;
-                if (p.vec_a && i < p.m && pk + V <= p.k) {
-                    r[q] = *reinterpret_cast<const vec_t*>(src);
-                } else {
 #pragma unroll
-                    for (int e = 0; e < V; ++e) {
-                        T x = T(0);
-                        if (i < p.m && pk + e < p.k) x = src[e];
-                        r[q][e] = x;
-                    }
-                }
-            }
-        }
-    }
-
-    // Interior tile, full slab, vector access allowed: straight-line 16-byte
-    // loads with no per-lane conditions (so the loads issue back to back).
-    __device__ inline void load_fast(const TileProblem<T>& p, int64_t m0, int64_t k0, int tid) {
-#pragma unroll
-        for (int q = 0; q < TL::NVA; ++q) {
-            const int v = tid + q * TL::NT;
-            if constexpr (!A_K) {
-                const int ic = v % (TL::BM / V), kk = v / (TL::BM / V);
-                r[q] = *reinterpret_cast<const vec_t*>(p.a + (m0 + ic * V) + (k0 + kk) * p.lda);
-            } else {
-                const int kc = v % (TL::BK / V), ii = v / (TL::BK / V);
-                r[q] = *reinterpret_cast<const vec_t*>(p.a + (k0 + kc * V) + (m0 + ii) * p.lda);
-            }
-        }
-    }
-
-    __device__ inline void store(T* As, int tid) const {
-#pragma unroll
-        for (int q = 0; q < TL::NVA; ++q) {
-            const int v = tid + q * TL::NT;
-            if constexpr (!A_K) {
-                const int ic = v % (TL::BM / V), kk = v / (TL::BM / V);
-                if constexpr (TL::LDS_VEC) {
-                    *reinterpret_cast<vec_t*>(As + kk * TL::LDA + ic * V) = r[q];
-                } else {
-#pragma unroll
-                    for (int e = 0; e < V; ++e) As[kk * TL::LDA + ic * V + e] = r[q][e];
-                }
-            } else {
-                const int kc = v % (TL::BK / V), ii = v / (TL::BK / V);
-#pragma unroll
-                for (int e = 0; e < V; ++e) As[(kc * V + e) * TL::LDA + ii] = r[q][e];
-            }
-        }
-    }
-};
-
-template <typename T, class TL, bool B_K>
-struct BLoader {
-    using vec_t = typename Mma<T>::vec_t;
-    static constexpr int V = TL::V;
-    vec_t r[TL::NVB];
-
-    // Edge tile or partial slab, element by element behind bounds checks.
-    __device__ inline void load_guarded(const TileProblem<T>& p, int64_t n0, int64_t k0, int tid) {
-#pragma unroll
-        for (int q = 0; q < TL::NVB; ++q) {
-            const int v = tid + q * TL::NT;
-            if constexpr (B_K) {
-                const int kc = v % (TL::BK / V), jj = v / (TL::BK / V);
-                const int64_t j = n0 + jj, pk = k0 + kc * V;
-                const T* src = p.b + pk + j * p.ldb;
-                if (p.vec_b && j < p.n && pk + V <= p.k) {
-                    r[q] = *reinterpret_cast<const vec_t*>(src);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < V; ++e) {
-                        T x = T(0);
-                        if (j < p.n && pk + e < p.k) x = src[e];
-                        r[q][e] = x;
-                    }
-                }
-            } else {
-                const int jc = v % (TL::BN / V), kk = v / (TL::BN / V);
-                const int64_t j = n0 + jc * V, pk = k0 + kk;
-                const T* src = p.b + j + pk * p.ldb;
-                if (p.vec_b && pk < p.k && j + V <= p.n) {
-                    r[q] = *reinterpret_cast<const vec_t*>(src);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < V; ++e) {
-                        T x = T(0);
-                        if (pk < p.k && j + e < p.n) x = src[e];
-                        r[q][e] = x;
-                    }
-                }
-            }
-        }
-    }
-
-    __device__ inline void load_fast(const TileProblem<T>& p, int64_t n0, int64_t k0, int tid) {
-#pragma unroll
-        for (int q = 0; q < TL::NVB; ++q) {
-            const int v = tid + q * TL::NT;
-            if constexpr (B_K) {
-                const int kc = v % (TL::BK / V), jj = v / (TL::BK / V);
-                r[q] = *reinterpret_cast<const vec_t*>(p.b + (k0 + kc * V) + (n0 + jj) * p.ldb);
-            } else {
-                const int jc = v % (TL::BN / V), kk = v / (TL::BN / V);
-                r[q] = *reinterpret_cast<const vec_t*>(p.b + (n0 + jc * V) + (k0 + kk) * p.ldb);
-            }
-        }
-    }
-
-    __device__ inline void store(T* Bs, int tid) const {
-#pragma unroll
-        for (int q = 0; q < TL::NVB; ++q) {
-            const int v = tid + q * TL::NT;
-            if constexpr (B_K) {
-                const int kc = v % (TL::BK / V), jj = v / (TL::BK / V);
-#pragma unroll
-                for (int e = 0; e < V; ++e) Bs[(kc * V + e) * TL::LDB + jj] = r[q][e];
-            } else {
-                const int jc = v % (TL::BN / V), kk = v / (TL::BN / V);
-                if constexpr (TL::LDS_VEC) {
-                    *reinterpret_cast<vec_t*>(Bs + kk * TL::LDB + jc * V) = r[q];
-                } else {
-#pragma unroll
-                    for (int e = 0; e < V; ++e) Bs[kk * TL::LDB + jc * V + e] = r[q][e];
-                }
+                for (int e = 0; e < V; ++e) S[(c * V + e) * LD + l] = r[q][e];
             }
         }
     }
@@ -381,7 +256,7 @@ __device__ inline void mma_slab(const T* As, const T* Bs,
         const T* ap = As + (ks + lk) * TL::LDA + wm0 + TL::TM * lr;
         const T* bp = Bs + (ks + lk) * TL::LDB + wn0 + TL::TN * lr;
         T af[TL::TM], bf[TL::TN];
-        if constexpr (TL::TM % V == 0 && TL::LDS_VEC) {
+        if constexpr (TL::TM % V == 0) {
 #pragma unroll
             for (int q = 0; q < TL::TM / V; ++q) {
                 vec_t t = *reinterpret_cast<const vec_t*>(ap + q * V);
@@ -392,7 +267,7 @@ __device__ inline void mma_slab(const T* As, const T* Bs,
 #pragma unroll
             for (int i = 0; i < TL::TM; ++i) af[i] = ap[i];
         }
-        if constexpr (TL::TN % V == 0 && TL::LDS_VEC) {
+        if constexpr (TL::TN % V == 0) {
 #pragma unroll
             for (int q = 0; q < TL::TN / V; ++q) {
                 vec_t t = *reinterpret_cast<const vec_t*>(bp + q * V);
@@ -429,6 +304,7 @@ __device__ inline void store_tile(const TileProblem<T>& p,
                                   const typename Mma<T>::acc_t (&acc)[TL::TM][TL::TN],
                                   int64_t row0, int64_t col0, int lane) {
     using vec_t = typename Mma<T>::vec_t;
+    using uvec_t = typename Mma<T>::uvec_t;
     constexpr int V = TL::V;
     constexpr int TM = TL::TM;
     const int g = lane >> 4, lc = lane & 15;
@@ -450,12 +326,12 @@ __device__ inline void store_tile(const TileProblem<T>& p,
 #pragma unroll
                             for (int e = 0; e < V; ++e) o[e] = alpha * acc[q * V + e][j][r];
                         } else {
-                            const vec_t old = *reinterpret_cast<const vec_t*>(dst + q * V);
+                            const vec_t old = *reinterpret_cast<const uvec_t*>(dst + q * V);
 #pragma unroll
                             for (int e = 0; e < V; ++e)
                                 o[e] = epilogue(alpha, acc[q * V + e][j][r], beta, old[e]);
                         }
-                        *reinterpret_cast<vec_t*>(dst + q * V) = o;
+                        *reinterpret_cast<uvec_t*>(dst + q * V) = o;
                     }
                     continue;
                 }
@@ -491,6 +367,7 @@ __device__ inline void store_tile_masked(const TileProblem<T>& p,
                                          const typename Mma<T>::acc_t (&acc)[TL::TM][TL::TN],
                                          int64_t row0, int64_t col0, int lane, CMask cm) {
     using vec_t = typename Mma<T>::vec_t;
+    using uvec_t = typename Mma<T>::uvec_t;
     constexpr int V = TL::V;
     constexpr int TM = TL::TM;
     const int g = lane >> 4, lc = lane & 15;
@@ -516,12 +393,12 @@ __device__ inline void store_tile_masked(const TileProblem<T>& p,
 #pragma unroll
                             for (int e = 0; e < V; ++e) o[e] = alpha * acc[q * V + e][j][r];
                         } else {
-                            const vec_t old = *reinterpret_cast<const vec_t*>(dst + q * V);
+                            const vec_t old = *reinterpret_cast<const uvec_t*>(dst + q * V);
 #pragma unroll
                             for (int e = 0; e < V; ++e)
                                 o[e] = epilogue(alpha, acc[q * V + e][j][r], beta, old[e]);
                         }
-                        *reinterpret_cast<vec_t*>(dst + q * V) = o;
+                        *reinterpret_cast<uvec_t*>(dst + q * V) = o;
                     }
                     continue;
                 }
@@ -552,6 +429,7 @@ __device__ inline void store_tile_lds(const TileProblem<T>& p,
                                       const typename Mma<T>::acc_t (&acc)[TL::TM][TL::TN],
                                       int64_t m0, int64_t n0, int wm0, int wn0, T* smem) {
     using vec_t = typename Mma<T>::vec_t;
+    using uvec_t = typename Mma<T>::uvec_t;
     constexpr int V = TL::V;
     constexpr int TM = TL::TM;
     constexpr int LDC = TL::BM + V;
@@ -587,11 +465,11 @@ __device__ inline void store_tile_lds(const TileProblem<T>& p,
 #pragma unroll
                 for (int e = 0; e < V; ++e) o[e] = alpha * a[e];
             } else {
-                const vec_t old = *reinterpret_cast<const vec_t*>(dst);
+                const vec_t old = *reinterpret_cast<const uvec_t*>(dst);
 #pragma unroll
                 for (int e = 0; e < V; ++e) o[e] = epilogue(alpha, a[e], beta, old[e]);
             }
-            *reinterpret_cast<vec_t*>(dst) = o;
+            *reinterpret_cast<uvec_t*>(dst) = o;
         } else {
 #pragma unroll
             for (int e = 0; e < V; ++e) {
@@ -605,16 +483,10 @@ __device__ inline void store_tile_lds(const TileProblem<T>& p,
 
 // Compute one BM x BN tile (tile coordinates tm, tn) of one problem. smem
 // must hold 2*TL::STAGE elements. The caller synchronises before reusing smem.
-// FAST: the tile lies inside the matrix and A, B (and C) allow 16-byte access,
-// so every full k slab is loaded without bounds checks.
+// BUF: the operands are read through buffer descriptors (SlabLoader).
 // PF: k slabs whose global loads are in flight while a slab is multiplied
 // (1: one register buffer; 2: two, for tiles that stream their operands
 // from HBM, such as the small problems of a batch).
-// EDGE: how edge tiles load. false: element loads behind bounds checks
-// (fewest registers: the single-GEMM kernels, whose occupancy was tuned with
-// it); true: addressing precomputed once per tile (EdgeState) and 16-byte
-// loads wherever a whole wave is inside the matrix (fewer instructions per
-// slab: the batch kernels, where almost every tile is an edge tile).
 // The loaded values, and so the arithmetic, are the same in every variant.
 // Pull the C tile's cache lines into L2 ahead of the epilogue (beta != 0):
 // one 4-byte global->LDS load per 128-byte line of each tile column, into a
@@ -635,12 +507,14 @@ __device__ inline void prefetch_c(const TileProblem<T>& p, int64_t m0, int64_t n
     __builtin_amdgcn_global_load_lds((const void*)(p.c + r + c * p.c_sj), (lds_ptr_t)dst, 4, 0, 0);
 }
 
-template <typename T, class TL, bool A_K, bool B_K, bool FAST, int PF, bool EDGE, bool LDS_EPI,
+template <typename T, class TL, bool A_K, bool B_K, bool BUF, int PF, bool LDS_EPI,
           bool C_PF = false, bool MASK = false>
 __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64_t n0, T* smem,
                                       int* sink = nullptr, CMask cm = CMask{}) {
     static_assert(PF == 1 || PF == 2, "prefetch depth");
     using acc_t = typename Mma<T>::acc_t;
+    using Loader_A = SlabLoader<T, TL, TL::BM, A_K, TL::NVA, BUF>;
+    using Loader_B = SlabLoader<T, TL, TL::BN, B_K, TL::NVB, BUF>;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int wm = wave % TL::WGM, wn = wave / TL::WGM;
@@ -653,49 +527,19 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
         for (int j = 0; j < TL::TN; ++j) acc[i][j] = acc_t{};
 
     const int64_t nk = (p.k + TL::BK - 1) / TL::BK;
-    using EA = EdgeState<T, TL, TL::BM, A_K, TL::NVA>;
-    using EB = EdgeState<T, TL, TL::BN, B_K, TL::NVB>;
-    // With EDGE, edge tiles keep their addressing for every slab; interior
-    // (FAST) tiles build it only for a partial last slab, so it holds no
-    // registers during their main loop.
-    EA ea;
-    EB eb;
-    if constexpr (EDGE && !FAST) {
-        if (nk > 0) {
-            ea.init(p.a, p.m, p.k, p.lda, p.vec_a, m0, tid);
-            eb.init(p.b, p.n, p.k, p.ldb, p.vec_b, n0, tid);
-        }
-    }
-    auto load = [&](ALoader<T, TL, A_K>& al, BLoader<T, TL, B_K>& bl, int64_t k0) {
-        if (FAST && k0 + TL::BK <= p.k) {
-            al.load_fast(p, m0, k0, tid);
-            bl.load_fast(p, n0, k0, tid);
-        } else if constexpr (!EDGE) {
-            al.load_guarded(p, m0, k0, tid);
-            bl.load_guarded(p, n0, k0, tid);
-        } else if constexpr (FAST) {
-            EA ta;
-            EB tb;
-            ta.init(p.a, p.m, p.k, p.lda, p.vec_a, m0, tid);
-            tb.init(p.b, p.n, p.k, p.ldb, p.vec_b, n0, tid);
-            ta.load(al.r, k0);
-            tb.load(bl.r, k0);
-        } else {
-            ea.load(al.r, k0);
-            eb.load(bl.r, k0);
-        }
-    };
+    Loader_A al;
+    Loader_B bl;
+    al.init(p.a, p.m, p.k, p.lda, p.vec_a, m0, tid);
+    bl.init(p.b, p.n, p.k, p.ldb, p.vec_b, n0, tid);
 
+    // k == 0 (a batch problem with k == 0 or alpha == 0) touches neither A
+    // nor B.
     if constexpr (PF == 1) {
-        ALoader<T, TL, A_K> al;
-        BLoader<T, TL, B_K> bl;
-        // k == 0 (a batch problem with k == 0 or alpha == 0) touches neither
-        // A nor B: the loads clamp addresses to the last row/column, which
-        // exists only when k >= 1.
         if (nk > 0) {
-            load(al, bl, 0);
-            al.store(smem, tid);
-            bl.store(smem + TL::A_ELEMS, tid);
+            al.load(0, tid);
+            bl.load(0, tid);
+            al.store(smem, 0, tid);
+            bl.store(smem + TL::A_ELEMS, 0, tid);
         }
         __syncthreads();
         if constexpr (C_PF) {
@@ -705,14 +549,17 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
             T* cur = smem + (s & 1) * TL::STAGE;
             T* nxt = smem + ((s + 1) & 1) * TL::STAGE;
             const bool more = (s + 1) < nk;
-            if (more) load(al, bl, (s + 1) * TL::BK);
+            if (more) {
+                al.load((s + 1) * TL::BK, tid);
+                bl.load((s + 1) * TL::BK, tid);
+            }
             if constexpr (C_PF) {
                 if (s + 2 == nk) prefetch_c<T, TL>(p, m0, n0, sink);
             }
             mma_slab<T, TL>(cur, cur + TL::A_ELEMS, acc, wm0, wn0, lane);
             if (more) {
-                al.store(nxt, tid);
-                bl.store(nxt + TL::A_ELEMS, tid);
+                al.store(nxt, (s + 1) * TL::BK, tid);
+                bl.store(nxt + TL::A_ELEMS, (s + 1) * TL::BK, tid);
             }
             __syncthreads();
         }
@@ -721,34 +568,53 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
         // written to LDS and now receives slab s + 2; buffer ((s + 1) & 1)
         // holds slab s + 1 and is written to the other LDS stage after the
         // multiply. The loop is unrolled by two so that each buffer is a
-        // fixed set of registers.
-        ALoader<T, TL, A_K> a0, a1;
-        BLoader<T, TL, B_K> b0, b1;
+        // fixed set of registers; one loader walks the slabs and its loaded
+        // registers change places with the second buffer's.
+        typename Mma<T>::vec_t ra[TL::NVA], rb[TL::NVB];   // odd slabs
+        auto swap_in = [&](auto& l, auto& other, auto&& f) {
+            constexpr int N = sizeof(other) / sizeof(other[0]);
+#pragma unroll
+            for (int q = 0; q < N; ++q) { auto t = l.r[q]; l.r[q] = other[q]; other[q] = t; }
+            f();
+#pragma unroll
+            for (int q = 0; q < N; ++q) { auto t = l.r[q]; l.r[q] = other[q]; other[q] = t; }
+        };
+        auto load = [&](auto buf, int64_t k0) {
+            if constexpr (decltype(buf)::value == 0) { al.load(k0, tid); bl.load(k0, tid); }
+            else {
+                swap_in(al, ra, [&] { al.load(k0, tid); });
+                swap_in(bl, rb, [&] { bl.load(k0, tid); });
+            }
+        };
+        auto store = [&](auto buf, T* S, int64_t k0) {
+            if constexpr (decltype(buf)::value == 0) {
+                al.store(S, k0, tid);
+                bl.store(S + TL::A_ELEMS, k0, tid);
+            } else {
+                swap_in(al, ra, [&] { al.store(S, k0, tid); });
+                swap_in(bl, rb, [&] { bl.store(S + TL::A_ELEMS, k0, tid); });
+            }
+        };
+        using Even = std::integral_constant<int, 0>;
+        using Odd = std::integral_constant<int, 1>;
         if (nk > 0) {
-            load(a0, b0, 0);
-            if (nk > 1) load(a1, b1, TL::BK);
-            a0.store(smem, tid);
-            b0.store(smem + TL::A_ELEMS, tid);
+            load(Even{}, 0);
+            if (nk > 1) load(Odd{}, TL::BK);
+            store(Even{}, smem, 0);
         }
         __syncthreads();
         auto step = [&](auto buf, int64_t s) {
             constexpr int B = decltype(buf)::value;   // == s & 1
             T* cur = smem + B * TL::STAGE;
             T* nxt = smem + (1 - B) * TL::STAGE;
-            if (s + 2 < nk) {
-                if constexpr (B == 0) load(a0, b0, (s + 2) * TL::BK);
-                else load(a1, b1, (s + 2) * TL::BK);
-            }
+            if (s + 2 < nk) load(buf, (s + 2) * TL::BK);
             mma_slab<T, TL>(cur, cur + TL::A_ELEMS, acc, wm0, wn0, lane);
-            if (s + 1 < nk) {
-                if constexpr (B == 0) { a1.store(nxt, tid); b1.store(nxt + TL::A_ELEMS, tid); }
-                else { a0.store(nxt, tid); b0.store(nxt + TL::A_ELEMS, tid); }
-            }
+            if (s + 1 < nk) store(std::integral_constant<int, 1 - B>{}, nxt, (s + 1) * TL::BK);
             __syncthreads();
         };
         for (int64_t s = 0; s < nk; s += 2) {
-            step(std::integral_constant<int, 0>{}, s);
-            if (s + 1 < nk) step(std::integral_constant<int, 1>{}, s + 1);
+            step(Even{}, s);
+            if (s + 1 < nk) step(Odd{}, s + 1);
         }
     }
 
@@ -756,7 +622,7 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
         store_tile_masked<T, TL>(p, acc, m0 + wm0, n0 + wn0, lane, cm);
     else if constexpr (LDS_EPI)
         store_tile_lds<T, TL>(p, acc, m0, n0, wm0, wn0, smem);
-    else if (FAST && p.vec_c)
+    else if (p.vec_c && m0 + TL::BM <= p.m && n0 + TL::BN <= p.n)
         store_tile<T, TL, true>(p, acc, m0 + wm0, n0 + wn0, lane);
     else
         store_tile<T, TL, false>(p, acc, m0 + wm0, n0 + wn0, lane);
@@ -767,20 +633,14 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
 // slab before the epilogue (one-slab prefetch depth only), through `sink`
 // (NT ints of LDS nobody reads). MASK: write only the stored region `cm` of
 // a structured C (store_tile_masked).
-template <typename T, class TL, bool A_K, bool B_K, int PF = 1, bool EDGE = false,
-          bool LDS_EPI = false, bool C_PF = false, bool MASK = false>
+template <typename T, class TL, bool A_K, bool B_K, bool BUF, int PF = 1, bool LDS_EPI = false,
+          bool C_PF = false, bool MASK = false>
 __device__ inline void gemm_tile(const TileProblem<T>& p, int64_t tm, int64_t tn, T* smem,
                                  int* sink = nullptr, CMask cm = CMask{}) {
     static_assert(!C_PF || PF == 1, "C prefetch is placed for one slab in flight");
     static_assert(!MASK || !LDS_EPI, "masked stores go straight from the accumulators");
     const int64_t m0 = tm * TL::BM, n0 = tn * TL::BN;
-    const bool fast = p.vec_a && p.vec_b && m0 + TL::BM <= p.m && n0 + TL::BN <= p.n;
-    if (fast)
-        gemm_tile_impl<T, TL, A_K, B_K, true, PF, EDGE, LDS_EPI, C_PF, MASK>(p, m0, n0, smem, sink,
-                                                                            cm);
-    else
-        gemm_tile_impl<T, TL, A_K, B_K, false, PF, EDGE, LDS_EPI, C_PF, MASK>(p, m0, n0, smem,
-                                                                             sink, cm);
+    gemm_tile_impl<T, TL, A_K, B_K, BUF, PF, LDS_EPI, C_PF, MASK>(p, m0, n0, smem, sink, cm);
 }
 
 } // namespace dev

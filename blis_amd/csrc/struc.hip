@@ -65,7 +65,7 @@ StrucSpec transposed(const StrucSpec& s) {
 
 // One tile of a structured product. Workgroups are uniform in (tm, tn), so
 // the early return is taken by the whole workgroup before any barrier.
-template <typename T, class TL, bool A_K, bool B_K, bool MASK>
+template <typename T, class TL, bool A_K, bool B_K, bool BUF, bool MASK>
 __global__ __launch_bounds__(TL::NT) void gemm_struc_kernel(TileProblem<T> p, GridInfo g,
                                                             StrucSpec s) {
     __shared__ T smem[2 * TL::STAGE];
@@ -95,8 +95,8 @@ __global__ __launch_bounds__(TL::NT) void gemm_struc_kernel(TileProblem<T> p, Gr
     p.a += A_K ? kb : kb * p.lda;
     p.b += B_K ? kb : kb * p.ldb;
     p.k = ke - kb;
-    gemm_tile<T, TL, A_K, B_K, 1, false, false, false, MASK>(p, tm, tn, smem, nullptr,
-                                                             CMask{s.cmask, s.cdoff});
+    gemm_tile<T, TL, A_K, B_K, BUF, 1, false, false, MASK>(p, tm, tn, smem, nullptr,
+                                                           CMask{s.cmask, s.cdoff});
 }
 
 // Dense column-major copy (ld = ldd) of an n x n structured matrix stored
@@ -178,16 +178,18 @@ int grid_for(int64_t total) {
     return (int)std::max<int64_t>(1, std::min<int64_t>(g, 8192));
 }
 
-template <typename T, class TL>
-void launch_struc_tl(const TileProblem<T>& p, bool a_k, bool b_k, const GridInfo& g,
+template <typename T, class TL, bool BUF>
+void launch_struc_tl(const TileProblem<T>& p, bool a_k, bool b_k, GridInfo g,
                      const StrucSpec& s, hipStream_t st) {
+    g.grid_m = (int)((p.m + TL::BM - 1) / TL::BM);
+    g.grid_n = (int)((p.n + TL::BN - 1) / TL::BN);
     const dim3 grid(g.grid_m * g.grid_n), block(TL::NT);
 #define BLIS_AMD_STRUC_LAUNCH(AK, BK)                                                        \
     if (s.cmask)                                                                             \
-        hipLaunchKernelGGL((gemm_struc_kernel<T, TL, AK, BK, true>), grid, block, 0, st, p,  \
+        hipLaunchKernelGGL((gemm_struc_kernel<T, TL, AK, BK, BUF, true>), grid, block, 0, st, p,  \
                            g, s);                                                            \
     else                                                                                     \
-        hipLaunchKernelGGL((gemm_struc_kernel<T, TL, AK, BK, false>), grid, block, 0, st, p, \
+        hipLaunchKernelGGL((gemm_struc_kernel<T, TL, AK, BK, BUF, false>), grid, block, 0, st, p, \
                            g, s);
     if (!a_k && !b_k) { BLIS_AMD_STRUC_LAUNCH(false, false) }
     else if (!a_k && b_k) { BLIS_AMD_STRUC_LAUNCH(false, true) }
@@ -200,13 +202,20 @@ void launch_struc_tl(const TileProblem<T>& p, bool a_k, bool b_k, const GridInfo
 // The structured kernels are built for the tiles the size heuristic picks
 // (gemm_default_tile): FP64 6, 10, 3, 4 and FP32 1, 12, 9, 10, 3, 4.
 template <typename T>
-void launch_struc(int tile, const TileProblem<T>& p, bool a_k, bool b_k, GridInfo g,
+void launch_struc(int tile, const TileProblem<T>& p, bool a_k, bool b_k, const GridInfo& g,
                   const StrucSpec& s, hipStream_t st) {
     const TileShape& ts = tile_shape(dt_of<T>(), tile);
-    g.grid_m = (int)((p.m + ts.bm - 1) / ts.bm);
-    g.grid_n = (int)((p.n + ts.bn - 1) / ts.bn);
+    if (!buf_problem(p, a_k, b_k, ts.bm, ts.bn, ts.bk)) {
+        // Strides that buffer descriptors cannot take (gemm.hip).
+        constexpr int BK = std::is_same<T, double>::value ? 16 : 32;
+        if (ts.bm >= 64)
+            launch_struc_tl<T, TileCfg<T, 128, 64, BK, 32, 32>, false>(p, a_k, b_k, g, s, st);
+        else
+            launch_struc_tl<T, TileCfg<T, 32, 32, BK, 16, 16>, false>(p, a_k, b_k, g, s, st);
+        return;
+    }
 #define BLIS_AMD_STRUC_CASE(idx, BM, BN, BK, WM, WN) \
-    case idx: launch_struc_tl<T, TileCfg<T, BM, BN, BK, WM, WN>>(p, a_k, b_k, g, s, st); return;
+    case idx: launch_struc_tl<T, TileCfg<T, BM, BN, BK, WM, WN>, true>(p, a_k, b_k, g, s, st); return;
     if constexpr (std::is_same<T, double>::value) {
         switch (tile) {
         BLIS_AMD_STRUC_CASE(6, 128, 128, 16, 64, 32)

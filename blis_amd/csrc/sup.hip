@@ -32,15 +32,16 @@ __global__ __launch_bounds__(SUP_THREADS) void gemm_sup_kernel(TileProblem<T> p,
     static_assert(TL::NT == SUP_THREADS, "sup tile shape");
     __shared__ T smem[2 * TL::STAGE];
     const int tm = blockIdx.x % grid_m, tn = blockIdx.x / grid_m;
-    gemm_tile<T, TL, A_K, B_K, 2>(p, tm, tn, smem);
+    gemm_tile<T, TL, A_K, B_K, true, 2>(p, tm, tn, smem);
 }
 
 namespace {
 
 template <typename T, int BK>
-void launch_sup_bk(const Plan& pl, double alpha, double beta, hipStream_t st) {
+bool launch_sup_bk(const Plan& pl, double alpha, double beta, hipStream_t st) {
     using TL = SupTL<T, BK>;
     const TileProblem<T> p = make_problem<T>(pl, alpha, beta);
+    if (!buf_problem(p, pl.a_k, pl.b_k, TL::BM, TL::BN, TL::BK)) return false;
     const int gm = (int)((pl.m + TL::BM - 1) / TL::BM);
     const int gn = (int)((pl.n + TL::BN - 1) / TL::BN);
     const dim3 grid(gm * gn), block(TL::NT);
@@ -53,12 +54,13 @@ void launch_sup_bk(const Plan& pl, double alpha, double beta, hipStream_t st) {
     else
         hipLaunchKernelGGL((gemm_sup_kernel<T, BK, true, true>), grid, block, 0, st, p, gm);
     HIP_CHECK(hipGetLastError());
+    return true;
 }
 
 template <typename T>
-void launch_sup(const Plan& pl, double alpha, double beta, hipStream_t st) {
-    if (pl.k <= 256) launch_sup_bk<T, 32>(pl, alpha, beta, st);
-    else launch_sup_bk<T, 64>(pl, alpha, beta, st);
+bool launch_sup(const Plan& pl, double alpha, double beta, hipStream_t st) {
+    if (pl.k <= 256) return launch_sup_bk<T, 32>(pl, alpha, beta, st);
+    return launch_sup_bk<T, 64>(pl, alpha, beta, st);
 }
 
 } // namespace
@@ -89,9 +91,9 @@ bool gemm_sup_deep_k(int tile, int parts, int64_t k) {
     return sup_enabled() && tile == 4 && parts <= 1 && k > 64 && k <= SMALL_GEMM_MAX_DIM;
 }
 
-void gemm_sup_run(Dt dt, const Plan& pl, double alpha, double beta, hipStream_t st) {
-    if (dt == Dt::F64) launch_sup<double>(pl, alpha, beta, st);
-    else launch_sup<float>(pl, alpha, beta, st);
+bool gemm_sup_run(Dt dt, const Plan& pl, double alpha, double beta, hipStream_t st) {
+    if (dt == Dt::F64) return launch_sup<double>(pl, alpha, beta, st);
+    return launch_sup<float>(pl, alpha, beta, st);
 }
 
 } // namespace blis_amd

@@ -1,0 +1,106 @@
+"""How the GEMM tiles read their operands (SlabLoader, gemm_tile.hpp).
+
+Every tile reads A and B through buffer descriptors that end at the operand's
+last element; operands whose strides do not allow that (negative, overlapping
+or very large leading dimensions) take the loads behind bounds checks. The
+arithmetic is the same either way, so a product of the same values must have
+the same bits whatever the storage: leading dimensions of every residue, a
+base that is aligned to one element only, memory full of NaN between and
+around the columns, reversed columns.
+"""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from tests.conftest import say, unit_roundoff
+
+pytestmark = pytest.mark.gpu
+
+# Tile edges: below, at and above the 16/32/64/128 tiles and the 8 to 64 deep
+# k slabs, with remainders of every 16-byte vector.
+SHAPES = [(1, 3, 1), (31, 33, 15), (64, 65, 17), (129, 127, 66), (200, 131, 513), (515, 258, 33)]
+
+
+def _store(x, pad, off, reverse=False):
+    """x (rows x cols) column-major in a NaN-filled device buffer with `pad`
+    extra rows between columns, starting `off` elements in; reversed: the
+    columns run backwards. Returns (buffer, address of (0, 0), cs)."""
+    r, c = x.shape
+    ld = r + pad
+    buf = torch.full((off + ld * c + off,), float("nan"), dtype=x.dtype, device="cuda")
+    v = buf[off:off + ld * c].view(c, ld)
+    v[:, :r] = (x.flip(1) if reverse else x).T
+    start = buf.data_ptr() + (off + (ld * (c - 1) if reverse else 0)) * x.element_size()
+    return buf, start, -ld if reverse else ld
+
+
+def _run(blis, dt, ta, tb, m, n, k, a, b, c0, pad, off, reverse, tile):
+    ch, ct = ("d", C.c_double) if dt == torch.float64 else ("s", C.c_float)
+    ba, pa, la = _store(a.T if ta else a, pad, off, reverse)
+    bb, pb, lb = _store(b.T if tb else b, pad, off, reverse)
+    bc, pc, lc = _store(c0, pad, off)
+    if tile is not None:
+        blis.bli_amd_gemm_set_config(tile, 8, 1, 1)
+    try:
+        getattr(blis, f"bli_{ch}gemm")(8 if ta else 0, 8 if tb else 0, m, n, k,
+                                       C.byref(ct(1.25)), pa, 1, la, pb, 1, lb,
+                                       C.byref(ct(0.5)), pc, 1, lc)
+    finally:
+        if tile is not None:
+            blis.bli_amd_gemm_set_config(-1, 8, 1, 1)
+    v = bc[off:off + lc * n].view(n, lc)
+    assert torch.isnan(v[:, m:]).all() and torch.isnan(bc[:off]).all() and \
+        torch.isnan(bc[off + lc * n:]).all(), "wrote outside C"
+    return v[:, :m].T.cpu()
+
+
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+@pytest.mark.parametrize("ta", [0, 1])
+@pytest.mark.parametrize("tb", [0, 1])
+def test_same_bits_for_every_storage(blis, dt, ta, tb):
+    g = torch.Generator(device="cuda").manual_seed(ta + 2 * tb)
+    u = unit_roundoff(np.float64 if dt == torch.float64 else np.float32)
+    tiles = [None, 4, 6 if dt == torch.float64 else 12]
+    for m, n, k in SHAPES:
+        a, b, c0 = (torch.rand(r, c, generator=g, device="cuda", dtype=dt) * 2 - 1
+                    for r, c in ((m, k), (k, n), (m, n)))
+        ref = 1.25 * (a.double() @ b.double()) + 0.5 * c0.double()
+        scale = 1.25 * a.double().norm() * b.double().norm() + 0.5 * c0.double().norm()
+        base = None
+        for tile in tiles:
+            for pad, off, reverse in ((0, 0, False), (1, 1, False), (3, 3, False), (8, 2, False),
+                                      (2, 1, True)):
+                say(f"loads {dt} ta={ta} tb={tb} {m}x{n}x{k} tile={tile} pad={pad} off={off} "
+                    f"reverse={reverse}")
+                got = _run(blis, dt, ta, tb, m, n, k, a, b, c0, pad, off, reverse, tile)
+                if base is None:
+                    base = got
+                    err = (got.cuda().double() - ref).norm() / scale
+                    assert err <= 4 * (k + 2) * u
+                assert torch.equal(got, base)
+
+
+def test_leading_dimension_beyond_32_bit_offsets(blis):
+    """Columns 2^27 + 1 doubles apart: 32 lines of a slab span more than 4 GiB,
+    past what a descriptor's offsets reach, and every column start is odd."""
+    m, n, k, ld = 33, 40, 5, (1 << 27) + 1
+    say("loads: leading dimension beyond 32-bit offsets")
+    g = torch.Generator(device="cuda").manual_seed(7)
+    a = torch.rand(m, k, generator=g, device="cuda", dtype=torch.float64)
+    b = torch.rand(k, n, generator=g, device="cuda", dtype=torch.float64)
+    big = torch.empty(ld * (k - 1) + m, dtype=torch.float64, device="cuda")
+    for j in range(k):
+        big[j * ld:j * ld + m] = a[:, j]
+    tight = a.T.contiguous()
+    bt = b.T.contiguous()
+    out = []
+    for ptr, lda in ((tight.data_ptr(), m), (big.data_ptr(), ld)):
+        c = torch.zeros(n, m, dtype=torch.float64, device="cuda")
+        blis.bli_dgemm(0, 0, m, n, k, C.byref(C.c_double(1.0)), ptr, 1, lda, bt.data_ptr(), 1, k,
+                       C.byref(C.c_double(0.0)), c.data_ptr(), 1, m)
+        out.append(c)
+    assert torch.equal(out[0], out[1])
