@@ -67,19 +67,64 @@ __global__ __launch_bounds__(TL::NT) void gemm_strided_kernel(TileProblem<T> p, 
 
 // C := beta*C + sum_z parts_z, partitions added in ascending z (a fixed
 // order, so the result does not depend on scheduling). beta == 0 does not
-// read C.
+// read C. Only the stored region `cm` of C is written. A thread takes one
+// 16-byte vector of rows and keeps eight partitions' loads in flight: the sum
+// is one pass over s*m*n partials, bound by the latency of its loads while
+// the output is small.
 template <typename T>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const T* __restrict__ parts, int s,
                                                             int64_t m, int64_t n, T* c,
-                                                            int64_t c_si, int64_t c_sj, T beta) {
-    const int64_t total = m * n;
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total;
-         t += (int64_t)gridDim.x * blockDim.x) {
-        T acc = parts[t];
-        for (int z = 1; z < s; ++z) acc += parts[z * total + t];
-        const int64_t i = t % m, j = t / m;
+                                                            int64_t c_si, int64_t c_sj, T beta,
+                                                            CMask cm) {
+    using vec_t = typename Mma<T>::vec_t;
+    using uvec_t = typename Mma<T>::uvec_t;
+    constexpr int V = Mma<T>::V;
+    const uint32_t mv = (uint32_t)((m + V - 1) / V);
+    const int64_t total = (int64_t)mv * n, slice = m * n;
+    for (int64_t t = blockIdx.x * (int64_t)256 + threadIdx.x; t < total;
+         t += (int64_t)gridDim.x * 256) {
+        const int64_t j = total >> 32 ? t / mv : (uint32_t)t / mv;
+        const int64_t i = (t - j * mv) * V;
+        // Rows [lo, hi) of the vector are stored.
+        int64_t lo = i, hi = min(i + V, m);
+        if (cm.uplo == 1) lo = max(lo, j - cm.doff);
+        if (cm.uplo == 2) hi = min(hi, j - cm.doff + 1);
+        if (lo >= hi) continue;
+        const T* p = parts + i + j * m;
+        vec_t acc;
+        if (i + V <= m) {
+            acc = *reinterpret_cast<const uvec_t*>(p);
+            int z = 1;
+            for (; z + 8 <= s; z += 8) {
+                vec_t v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    v[u] = *reinterpret_cast<const uvec_t*>(p + (z + u) * slice);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) acc += v[u];
+            }
+            for (; z < s; ++z) acc += *reinterpret_cast<const uvec_t*>(p + z * slice);
+        } else {
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                acc[e] = T(0);
+                if (i + e < m) {
+                    T x = p[e];
+                    for (int z = 1; z < s; ++z) x += p[e + z * slice];
+                    acc[e] = x;
+                }
+            }
+        }
         T* dst = c + i * c_si + j * c_sj;
-        *dst = (beta == T(0)) ? acc : beta * *dst + acc;
+        if (c_si == 1 && lo == i && hi == i + V) {
+            if (beta != T(0)) acc = beta * *reinterpret_cast<const uvec_t*>(dst) + acc;
+            *reinterpret_cast<uvec_t*>(dst) = acc;
+        } else {
+#pragma unroll
+            for (int e = 0; e < V; ++e)
+                if (i + e >= lo && i + e < hi)
+                    dst[e * c_si] = (beta == T(0)) ? acc[e] : beta * dst[e * c_si] + acc[e];
+        }
     }
 }
 
@@ -169,13 +214,20 @@ void pack_run(Dt dt, const void* src, int64_t m, int64_t n, int64_t rs, int64_t 
 // Launch plumbing
 // ---------------------------------------------------------------------------
 
-// Split-k launch parameters: `parts` partitions of `kchunk` (the last one
-// shorter) into the workspace `ws`.
-struct SplitK {
-    int parts = 1;
-    int64_t kchunk = 0;
-    void* ws = nullptr;
-};
+void splitk_reduce_run(Dt dt, const SplitK& sk, const Plan& pl, double beta, const CMask& cm,
+                       hipStream_t st) {
+    const int64_t V = dt == Dt::F64 ? Mma<double>::V : Mma<float>::V;
+    const int g = grid_for((pl.m + V - 1) / V * pl.n);
+    if (dt == Dt::F64)
+        hipLaunchKernelGGL(splitk_reduce_kernel<double>, dim3(g), dim3(256), 0, st,
+                           (const double*)sk.ws, sk.parts, pl.m, pl.n, (double*)pl.c, pl.c_si,
+                           pl.c_sj, beta, cm);
+    else
+        hipLaunchKernelGGL(splitk_reduce_kernel<float>, dim3(g), dim3(256), 0, st,
+                           (const float*)sk.ws, sk.parts, pl.m, pl.n, (float*)pl.c, pl.c_si,
+                           pl.c_sj, (float)beta, cm);
+    HIP_CHECK(hipGetLastError());
+}
 
 template <typename T, class TL, bool BUF>
 static void launch_tl(const TileProblem<T>& p, bool a_k, bool b_k, GridInfo g, const SplitK& sk,
@@ -299,37 +351,96 @@ int gemm_default_tile(Dt dt, int64_t m, int64_t n, int64_t k) {
     return 4;
 }
 
-// Number of k partitions for a product whose output is small against its
-// depth (m, n <= k/4, k >= 2048): such products have too few output tiles to
-// fill 256 CUs and a long serial k loop in each. The count aims at about 512
-// workgroups of the tile gemm_split_tile gives (128x128 when m, n >= 1024,
-// else 64x64), keeps every partition at least 1024 deep and uses at most 64.
-// It depends on the shape only, so every tile gives the same partition.
-// Measured on MI355X (device time, default path, against the earlier rule of
-// about 2048 workgroups of 32x32 outputs on the selector's tile):
-//   FP64 1024x1024x8192 293 against 378-420 us (8 partitions of 128x128
-//   tiles against 2), 512x512x16384 185 against 202 us, 128x128x65536 75
-//   against 82 us;
-//   FP32 1024x1024x8192 160 against 189 us, 256x256x32768 64 against 72 us,
-//   128x128x65536 53 against 57 us.
-static int gemm_default_split(int64_t m, int64_t n, int64_t k) {
-    if (k < 2048 || 4 * std::max(m, n) > k) return 1;
-    const int64_t bt = (m >= 1024 && n >= 1024) ? 128 : 64;
-    int64_t s = std::max<int64_t>(1, 512 / (((m + bt - 1) / bt) * ((n + bt - 1) / bt)));
-    s = std::min<int64_t>(s, k / 1024);
-    return (int)std::min<int64_t>(s, 64);
+// Device time of a product on one tile with `parts` k partitions, in us: a
+// workgroup's launch, prologue and epilogue (fixed); its serial chain of k
+// slabs, each bound by its own latency (slab) while few workgroups share a
+// CU, or by the CU's matrix cores (slab_full per resident workgroup); and
+// for parts > 1 the reduction, one pass over the partitions. `resident` is
+// how many workgroups fit a CU. Fitted to the device times of 300 random
+// GEMM and 100 random SYRK shapes (m, n in [32, 8192], k in [128, 16384], SYRK
+// to 65536, both layouts of each operand) on these tiles with 1 to 64
+// partitions: rms error 20% (FP64) and 16% (FP32) over 10,800 timings.
+struct TileCost {
+    int tile, bm, bn, bk, resident;
+    double slab, slab_full, fixed;
+};
+static const TileCost COST_F64[] = {
+    { 3, 64, 64, 16, 4, 0.794, 0.561, 4.6 },
+    { 4, 32, 32, 16, 8, 0.662, 0.002, 1.7 },
+    { 10, 64, 128, 16, 3, 1.170, 0.988, 5.0 },
+};
+static const TileCost COST_F32[] = {
+    { 1, 128, 64, 32, 3, 1.326, 1.069, 6.0 },
+    { 3, 64, 64, 32, 4, 0.819, 0.609, 6.5 },
+    { 4, 32, 32, 32, 8, 0.457, 0.199, 4.7 },
+};
+
+static double tile_cost(Dt dt, const TileCost& t, int64_t m, int64_t n, int64_t k, int parts,
+                        bool masked) {
+    const int64_t gm = (m + t.bm - 1) / t.bm, gn = (n + t.bn - 1) / t.bn;
+    const int64_t tiles = masked ? (gm * gn + std::max(gm, gn)) / 2 : gm * gn;
+    const int64_t chunk = (k + 63) / 64 > parts ? ((k + 63) / 64 + parts - 1) / parts * 64 : 64;
+    const double slabs = (double)((std::min(chunk, k) + t.bk - 1) / t.bk);
+    const double wgs = (double)(tiles * parts);
+    const int64_t w = (tiles * parts + 255) / 256;
+    const bool fits = w <= t.resident;
+    const double lat = t.slab * (fits ? 1.0 : wgs / (256.0 * t.resident) + 0.3);
+    const double thr = t.slab_full * (fits ? (double)w : wgs / 256.0 + 0.5);
+    double us = t.fixed + slabs * std::max(lat, thr);
+    if (parts > 1) {
+        const double bytes = (2.0 * parts + 2.0) * (double)m * (double)n * (double)dt_size(dt);
+        us += 3.7 + (masked ? 0.6 : 1.0) * bytes / 5.35e6;
+    }
+    return us;
 }
 
-// Tile for a product that gemm_default_split splits: 128x128 tiles when
-// m, n >= 1024 (FP64 table tile 6, eight 64x32 waves; FP32 tile 0, four
-// 64x64 waves); 64x64 tiles when there are at least four of them (FP64 tile
-// 8, BK 32; FP32 tile 3); else 32x32 tiles (tile 4). A single 64x64 tile
-// leaves too few workgroups: FP64 64x64x262144 took 222 us on it against
-// 182 us on 32x32 tiles.
-static int gemm_split_tile(Dt dt, int64_t m, int64_t n) {
-    if (m >= 1024 && n >= 1024) return dt == Dt::F64 ? 6 : 0;
-    if (((m + 63) / 64) * ((n + 63) / 64) >= 4) return dt == Dt::F64 ? 8 : 3;
-    return 4;
+// k partitions of a product and the tile for it when there are several.
+// Products with few output tiles against the 256 CUs walk a long serial k
+// loop on a mostly idle chip; more partitions shorten the loop and cost a
+// pass over the partial outputs. The pair with the least modelled time is
+// taken. It depends on the type and the shape only, so every tile and every
+// operand layout gives the same bits. Over the fitted shapes it is within
+// 6.5% (FP64 GEMM), 4.6% (FP32 GEMM), 3.4% and 13% (SYRK) of the best
+// timing in geometric mean, where splitting only products with
+// m, n <= k/4 and k >= 2048 into 1024-deep partitions left 48%, 32% and,
+// for SYRK without partitions, 214% and 133%. Measured (us, before, now):
+// FP64 256x256x4096 51 / 23, 128x4096x4096 173 / 88, 64x3000x3000 126 / 38,
+// 700x500x1500 51 / 34.
+// One pass stays: up to k = 512 (single calls and batches of such products
+// agree bit for bit), where the partitions would take over 48 MiB, and from
+// 2048 tiles of 64 x 64, which fill the chip by themselves. An output of a
+// single 64 x 64 tile keeps partitions of 1024, up to 64 of them.
+SplitChoice gemm_choose_split(Dt dt, int64_t m, int64_t n, int64_t k, bool masked) {
+    SplitChoice c;
+    if (k <= 512) return c;
+    const int64_t t64 = ((m + 63) / 64) * ((n + 63) / 64);
+    if (t64 >= 2048) return c;
+    if (t64 == 1 && !masked) {
+        if (k >= 2048) c.split = (int)std::min<int64_t>(k / 1024, 64);
+        c.tile = 4;
+        return c;
+    }
+    static const int parts[] = { 1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 32, 40, 48, 64 };
+    const TileCost* tab = dt == Dt::F64 ? COST_F64 : COST_F32;
+    double best = 0.0;
+    for (int q = 0; q < 3; ++q)
+        for (int s : parts) {
+            if (s > 1 && (s * 64 > k || (double)s * m * n * dt_size(dt) > 48.0 * (1 << 20))) break;
+            const double us = tile_cost(dt, tab[q], m, n, k, s, masked);
+            if (best == 0.0 || us < best) { best = us; c.split = s; c.tile = tab[q].tile; }
+        }
+    return c;
+}
+
+// The same for a call on stream st. A captured product takes one pass unless
+// that is many times slower (m, n <= k/4 and k >= 2048): the graph would keep
+// the address of the partitions, which its replays share with other calls.
+SplitChoice split_on_stream(Dt dt, int64_t m, int64_t n, int64_t k, bool masked, hipStream_t st) {
+    const SplitChoice c = gemm_choose_split(dt, m, n, k, masked);
+    if (c.split <= 1 || (!masked && k >= 2048 && 4 * std::max(m, n) <= k)) return c;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIP_CHECK(hipStreamIsCapturing(st, &cap));
+    return cap == hipStreamCaptureStatusNone ? c : SplitChoice{};
 }
 
 // Process-wide override used when a caller passes no configuration
@@ -339,7 +450,7 @@ static GemmConfig g_override;
 // Split-k launch parameters for `split` requested partitions of whole
 // 64-deep k blocks (every tile's BK divides 64, so the partition, and with
 // it the rounding, is the same for every tile).
-static SplitK split_params(int64_t k, int split) {
+SplitK split_params(int64_t k, int split) {
     SplitK sk;
     if (split > 1) {
         const int64_t blocks = (k + 63) / 64;
@@ -365,24 +476,16 @@ static void launch_plan(Dt dt, Plan& pl, const GemmConfig& cfg, double alpha, do
     SplitK sk = split_params(pl.k, cfg.split_k);
     if (gemm_sup_deep_k(tile, sk.parts, pl.k) && gemm_sup_run(dt, pl, alpha, beta, st)) return;
     const size_t es = dt_size(dt);
-    if (sk.parts > 1) sk.ws = sc.take((size_t)sk.parts * pl.m * pl.n * es, 17);
+    if (sk.parts > 1) {
+        const size_t bytes = (size_t)sk.parts * pl.m * pl.n * es;
+        sk.ws = sc.base ? sc.take(bytes, 17) : stream_scratch(bytes, st);
+    }
     if (dt == Dt::F64) {
         launch_tile<double>(tile, make_problem<double>(pl, alpha, beta), pl.a_k, pl.b_k, g, sk, st);
     } else {
         launch_tile<float>(tile, make_problem<float>(pl, alpha, beta), pl.a_k, pl.b_k, g, sk, st);
     }
-    if (sk.parts > 1) {
-        const int gr = grid_for(pl.m * pl.n);
-        if (dt == Dt::F64)
-            hipLaunchKernelGGL(splitk_reduce_kernel<double>, dim3(gr), dim3(256), 0, st,
-                               (const double*)sk.ws, sk.parts, pl.m, pl.n, (double*)pl.c, pl.c_si,
-                               pl.c_sj, beta);
-        else
-            hipLaunchKernelGGL(splitk_reduce_kernel<float>, dim3(gr), dim3(256), 0, st,
-                               (const float*)sk.ws, sk.parts, pl.m, pl.n, (float*)pl.c, pl.c_si,
-                               pl.c_sj, (float)beta);
-        HIP_CHECK(hipGetLastError());
-    }
+    if (sk.parts > 1) splitk_reduce_run(dt, sk, pl, beta, CMask{}, st);
 }
 
 void gemm_run(const GemmDesc& d, const GemmConfig* cfg, hipStream_t st) {
@@ -409,12 +512,15 @@ void gemm_run(const GemmDesc& d, const GemmConfig* cfg, hipStream_t st) {
         const bool vb = vec_ok(pl.b, pl.b_packed, pl.ldb, d.dt);
         const bool vc = aligned16(pl.c) && pl.c_si == 1 && pl.c_sj % (d.dt == Dt::F64 ? 2 : 4) == 0;
         picked = config_of(selector_pick(d.dt, pl.m, pl.n, pl.k, pl.a_k, pl.b_k, va, vb, vc));
-        picked.split_k = g_override.split_k > 1 ? g_override.split_k
-                                                : gemm_default_split(pl.m, pl.n, pl.k);
-        // A product split by the shape rule takes the tile measured for it,
-        // unless the selector timed every configuration itself.
-        if (g_override.split_k <= 1 && picked.split_k > 1 && selector_mode() != SELECT_EXHAUSTIVE)
-            picked.tile = gemm_split_tile(d.dt, pl.m, pl.n);
+        if (g_override.split_k > 1) {
+            picked.split_k = g_override.split_k;
+        } else {
+            // A product split by the shape rule takes the rule's tile, unless
+            // the selector timed every configuration itself.
+            const SplitChoice sc = split_on_stream(d.dt, pl.m, pl.n, pl.k, false, st);
+            picked.split_k = sc.split;
+            if (sc.split > 1 && selector_mode() != SELECT_EXHAUSTIVE) picked.tile = sc.tile;
+        }
         cfg = &picked;
     }
     Scratch sc;
@@ -572,9 +678,9 @@ int bli_amd_gemm_noalloc(num_t dt, trans_t transa, trans_t transb, dim_t m, dim_
     }
     Plan pl = layout(g);
     GemmConfig cfg;
-    cfg.tile = gemm_default_tile(d, pl.m, pl.n, pl.k);
-    cfg.split_k = gemm_default_split(pl.m, pl.n, pl.k);
-    if (cfg.split_k > 1) cfg.tile = gemm_split_tile(d, pl.m, pl.n);
+    const SplitChoice choice = gemm_choose_split(d, pl.m, pl.n, pl.k, false);
+    cfg.split_k = choice.split;
+    cfg.tile = choice.split > 1 ? choice.tile : gemm_default_tile(d, pl.m, pl.n, pl.k);
     // Scratch this call needs, carved as Scratch::take does (256-byte
     // aligned pieces): packed general-stride operands and split-k slices.
     const size_t es = dt_size(d);
@@ -582,7 +688,16 @@ int bli_amd_gemm_noalloc(num_t dt, trans_t transa, trans_t transb, dim_t m, dim_
     if (pl.a_packed) need += align256((size_t)pl.m * pl.k * es);
     if (pl.b_packed) need += align256((size_t)pl.k * pl.n * es);
     const SplitK sk = split_params(pl.k, cfg.split_k);
-    if (sk.parts > 1) need += align256((size_t)sk.parts * pl.m * pl.n * es);
+    if (sk.parts > 1) {
+        const size_t slices = align256((size_t)sk.parts * pl.m * pl.n * es);
+        if (need + slices > NOALLOC_SCRATCH_BYTES) {
+            // No room for the partitions beside the packed operands: one pass.
+            cfg.split_k = 1;
+            cfg.tile = gemm_default_tile(d, pl.m, pl.n, pl.k);
+        } else {
+            need += slices;
+        }
+    }
     if (need > NOALLOC_SCRATCH_BYTES) return BLIS_INSUFFICIENT_STACK_BUF_SIZE;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return BLIS_FAILURE;

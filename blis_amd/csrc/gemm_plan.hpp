@@ -147,6 +147,26 @@ inline TileProblem<T> make_problem(const Plan& pl, double alpha, double beta) {
     return p;
 }
 
+// Split-k launch parameters (gemm.hip): `parts` partitions of `kchunk` (the
+// last one shorter), each an m x n column-major slice of the workspace `ws`.
+struct SplitK {
+    int parts = 1;
+    int64_t kchunk = 0;
+    void* ws = nullptr;
+};
+// The k partitions for a shape, and the tile when there are several (masked:
+// about half of the output tiles are stored).
+struct SplitChoice {
+    int split = 1;
+    int tile = -1;
+};
+SplitChoice gemm_choose_split(Dt dt, int64_t m, int64_t n, int64_t k, bool masked);
+SplitChoice split_on_stream(Dt dt, int64_t m, int64_t n, int64_t k, bool masked, hipStream_t st);
+SplitK split_params(int64_t k, int split);
+// C := beta*C + the sum of the partitions, on the stored region cm of C.
+void splitk_reduce_run(Dt dt, const SplitK& sk, const Plan& pl, double beta, const CMask& cm,
+                       hipStream_t st);
+
 // The single-call small-problem path (sup.hip): applies to m, n, k all at
 // most SMALL_GEMM_MAX_DIM with k > 64; the plan's operands must have a unit
 // stride. gemm_sup_deep_k: the 32 x 32 table tile over k > 64 in one

@@ -175,10 +175,10 @@ struct SlabLoader {
         }
     }
 
-    // Load the slab at k0; BUF loaders are called for consecutive slabs.
-    __device__ inline void load(int64_t k0, int tid) {
+    // Load slab s; BUF loaders are called for consecutive slabs.
+    __device__ inline void load(int s, int tid) {
         if constexpr (BUF) {
-            const uint32_t n = left > 0xFFFFFFFFll ? 0xFFFFFFFFu : (uint32_t)left;
+            const uint32_t n = (uint32_t)(left >> 32) != 0 ? 0xFFFFFFFFu : (uint32_t)left;
             auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)n, 0x00020000);
             const uint32_t step = (uint32_t)LINES * ((uint32_t)ld * (uint32_t)sizeof(T));
 #pragma unroll
@@ -190,6 +190,7 @@ struct SlabLoader {
             base += adv;
             left -= adv;
         } else {
+            const int64_t k0 = (int64_t)s * TL::BK;
             const bool whole = vec && row0 + ROWS <= rows && k0 + TL::BK <= K;   // uniform
 #pragma unroll
             for (int q = 0; q < NV; ++q) {
@@ -217,11 +218,11 @@ struct SlabLoader {
         }
     }
 
-    // Store the slab at k0 into an LDS stage, k-major.
-    __device__ inline void store(T* S, int64_t k0, int tid) {
+    // Store the loaded slab into an LDS stage, k-major; kleft: its k extent
+    // if it is a partial last slab, else 0.
+    __device__ inline void store(T* S, int kleft, int tid) {
         if constexpr (BUF && K_CONTIG) {
-            if (k0 + TL::BK > K) {
-                const int kleft = (int)(K - k0);
+            if (kleft != 0) {
 #pragma unroll
                 for (int q = 0; q < NV; ++q)
 #pragma unroll
@@ -526,7 +527,8 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
 #pragma unroll
         for (int j = 0; j < TL::TN; ++j) acc[i][j] = acc_t{};
 
-    const int64_t nk = (p.k + TL::BK - 1) / TL::BK;
+    const int nk = (int)((p.k + TL::BK - 1) / TL::BK);
+    const int ktail = (int)(p.k % TL::BK);   // extent of a partial last slab
     Loader_A al;
     Loader_B bl;
     al.init(p.a, p.m, p.k, p.lda, p.vec_a, m0, tid);
@@ -538,28 +540,29 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
         if (nk > 0) {
             al.load(0, tid);
             bl.load(0, tid);
-            al.store(smem, 0, tid);
-            bl.store(smem + TL::A_ELEMS, 0, tid);
+            al.store(smem, nk == 1 ? ktail : 0, tid);
+            bl.store(smem + TL::A_ELEMS, nk == 1 ? ktail : 0, tid);
         }
         __syncthreads();
         if constexpr (C_PF) {
             if (nk <= 1) prefetch_c<T, TL>(p, m0, n0, sink);
         }
-        for (int64_t s = 0; s < nk; ++s) {
+        for (int s = 0; s < nk; ++s) {
             T* cur = smem + (s & 1) * TL::STAGE;
             T* nxt = smem + ((s + 1) & 1) * TL::STAGE;
             const bool more = (s + 1) < nk;
             if (more) {
-                al.load((s + 1) * TL::BK, tid);
-                bl.load((s + 1) * TL::BK, tid);
+                al.load(s + 1, tid);
+                bl.load(s + 1, tid);
             }
             if constexpr (C_PF) {
                 if (s + 2 == nk) prefetch_c<T, TL>(p, m0, n0, sink);
             }
             mma_slab<T, TL>(cur, cur + TL::A_ELEMS, acc, wm0, wn0, lane);
             if (more) {
-                al.store(nxt, (s + 1) * TL::BK, tid);
-                bl.store(nxt + TL::A_ELEMS, (s + 1) * TL::BK, tid);
+                const int kleft = s + 2 == nk ? ktail : 0;
+                al.store(nxt, kleft, tid);
+                bl.store(nxt + TL::A_ELEMS, kleft, tid);
             }
             __syncthreads();
         }
@@ -579,40 +582,41 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
 #pragma unroll
             for (int q = 0; q < N; ++q) { auto t = l.r[q]; l.r[q] = other[q]; other[q] = t; }
         };
-        auto load = [&](auto buf, int64_t k0) {
-            if constexpr (decltype(buf)::value == 0) { al.load(k0, tid); bl.load(k0, tid); }
+        auto load = [&](auto buf, int s) {
+            if constexpr (decltype(buf)::value == 0) { al.load(s, tid); bl.load(s, tid); }
             else {
-                swap_in(al, ra, [&] { al.load(k0, tid); });
-                swap_in(bl, rb, [&] { bl.load(k0, tid); });
+                swap_in(al, ra, [&] { al.load(s, tid); });
+                swap_in(bl, rb, [&] { bl.load(s, tid); });
             }
         };
-        auto store = [&](auto buf, T* S, int64_t k0) {
+        auto store = [&](auto buf, T* S, int s) {
+            const int kleft = s + 1 == nk ? ktail : 0;
             if constexpr (decltype(buf)::value == 0) {
-                al.store(S, k0, tid);
-                bl.store(S + TL::A_ELEMS, k0, tid);
+                al.store(S, kleft, tid);
+                bl.store(S + TL::A_ELEMS, kleft, tid);
             } else {
-                swap_in(al, ra, [&] { al.store(S, k0, tid); });
-                swap_in(bl, rb, [&] { bl.store(S + TL::A_ELEMS, k0, tid); });
+                swap_in(al, ra, [&] { al.store(S, kleft, tid); });
+                swap_in(bl, rb, [&] { bl.store(S + TL::A_ELEMS, kleft, tid); });
             }
         };
         using Even = std::integral_constant<int, 0>;
         using Odd = std::integral_constant<int, 1>;
         if (nk > 0) {
             load(Even{}, 0);
-            if (nk > 1) load(Odd{}, TL::BK);
+            if (nk > 1) load(Odd{}, 1);
             store(Even{}, smem, 0);
         }
         __syncthreads();
-        auto step = [&](auto buf, int64_t s) {
+        auto step = [&](auto buf, int s) {
             constexpr int B = decltype(buf)::value;   // == s & 1
             T* cur = smem + B * TL::STAGE;
             T* nxt = smem + (1 - B) * TL::STAGE;
-            if (s + 2 < nk) load(buf, (s + 2) * TL::BK);
+            if (s + 2 < nk) load(buf, s + 2);
             mma_slab<T, TL>(cur, cur + TL::A_ELEMS, acc, wm0, wn0, lane);
-            if (s + 1 < nk) store(std::integral_constant<int, 1 - B>{}, nxt, (s + 1) * TL::BK);
+            if (s + 1 < nk) store(std::integral_constant<int, 1 - B>{}, nxt, s + 1);
             __syncthreads();
         };
-        for (int64_t s = 0; s < nk; s += 2) {
+        for (int s = 0; s < nk; s += 2) {
             step(Even{}, s);
             if (s + 1 < nk) step(Odd{}, s + 1);
         }

@@ -62,7 +62,7 @@ BLIS_AMD_HIDDEN void        sync_if_needed();
 // Grow-only device scratch, one buffer per slot: 0-1 GEMM operand packing
 // and transposes, 2-5 split-precision slices and statistics, 5-7 level-1/2
 // partials, 8-10 autotuner operands, 11-12 batch autotuner, 13-16 TRSM,
-// 17 GEMM split-k partitions, 18-19 TRSM 512-row inverses, 20-21 dense
+// 17 unused, 18-19 TRSM 512-row inverses, 20-21 dense
 // copies of structured operands (symm/trmm) and trmm's copy of B, 22-24
 // complex GEMM (A in 1e format, B in 1r format, a column-major copy of C),
 // 25-27 mixed-datatype GEMM (A and B in the computation type, the product).
@@ -70,6 +70,10 @@ BLIS_AMD_HIDDEN void        sync_if_needed();
 // products, constants).
 constexpr int WS_SLOTS = 32;
 BLIS_AMD_HIDDEN void*       workspace(size_t bytes, int slot);
+// Split-k partitions of products on stream st: a buffer of its own for each
+// of the last eight streams, so that products running side by side on
+// several streams do not share one. Valid for work enqueued on st now.
+BLIS_AMD_HIDDEN void*       stream_scratch(size_t bytes, hipStream_t st);
 BLIS_AMD_HIDDEN bool        synchronous();   // calls wait for their results
 BLIS_AMD_HIDDEN bool        is_device_pointer(const void* p);
 BLIS_AMD_HIDDEN void        check_hip(hipError_t e, const char* what, const char* file, int line);

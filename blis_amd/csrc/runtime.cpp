@@ -34,6 +34,15 @@ struct State {
     void* ws[WS_SLOTS] = {};
     size_t ws_bytes[WS_SLOTS] = {};
     std::mutex api;
+    // Split-k partitions: one buffer per stream that used them last.
+    struct StreamScratch {
+        hipStream_t st;
+        void* p;
+        size_t bytes;
+        unsigned long long used;
+    };
+    std::vector<StreamScratch> split;
+    unsigned long long split_clock = 0;
 };
 
 State& S() {
@@ -121,6 +130,45 @@ void* workspace(size_t bytes, int slot) {
         s.ws_bytes[slot] = want;
     }
     return s.ws[slot];
+}
+
+void* stream_scratch(size_t bytes, hipStream_t st) {
+    constexpr size_t MAX_STREAMS = 8;
+    State& s = S();
+    std::lock_guard<std::mutex> g(s.ws_mutex);
+    auto it = std::find_if(s.split.begin(), s.split.end(),
+                           [&](const State::StreamScratch& e) { return e.st == st; });
+    if (it == s.split.end()) {
+        if (s.split.size() >= MAX_STREAMS) {
+            // Give back the buffer of the stream that used its own longest
+            // ago. Its handle may be gone, so wait for the device.
+            auto old = std::min_element(s.split.begin(), s.split.end(),
+                                        [](const State::StreamScratch& a,
+                                           const State::StreamScratch& b) { return a.used < b.used; });
+            HIP_CHECK(hipDeviceSynchronize());
+            HIP_CHECK(hipFree(old->p));
+            s.split.erase(old);
+        }
+        s.split.push_back({ st, nullptr, 0, 0 });
+        it = s.split.end() - 1;
+    }
+    it->used = ++s.split_clock;
+    if (it->bytes < bytes) {
+        if (it->p) {
+            HIP_CHECK(hipStreamSynchronize(st));
+            HIP_CHECK(hipFree(it->p));
+            it->p = nullptr;
+            it->bytes = 0;
+        }
+        // Whole 16 MiB steps: a program's shapes settle after a few calls.
+        const size_t want = (bytes + ((size_t)16 << 20) - 1) >> 24 << 24;
+        if (hipMalloc(&it->p, want) != hipSuccess) {
+            (void)hipGetLastError();
+            abort_with(BLIS_MALLOC_RETURNED_NULL, "split-k scratch allocation");
+        }
+        it->bytes = want;
+    }
+    return it->p;
 }
 
 bool is_device_pointer(const void* p) {

@@ -67,8 +67,22 @@ StrucSpec transposed(const StrucSpec& s) {
 // the early return is taken by the whole workgroup before any barrier.
 template <typename T, class TL, bool A_K, bool B_K, bool BUF, bool MASK>
 __global__ __launch_bounds__(TL::NT) void gemm_struc_kernel(TileProblem<T> p, GridInfo g,
-                                                            StrucSpec s) {
+                                                            StrucSpec s, int64_t kchunk,
+                                                            T* parts) {
     __shared__ T smem[2 * TL::STAGE];
+    if (MASK && gridDim.y > 1) {
+        // One k partition per blockIdx.y into its slice of parts, as in
+        // gemm_kernel (masked products only: they have no per-tile k range).
+        const int64_t z = blockIdx.y, k0 = z * kchunk;
+        p.a += A_K ? k0 : k0 * p.lda;
+        p.b += B_K ? k0 : k0 * p.ldb;
+        p.k = min(kchunk, p.k - k0);
+        p.c = parts + z * p.m * p.n;
+        p.c_si = 1;
+        p.c_sj = p.m;
+        p.vec_c = 1;
+        p.beta = T(0);
+    }
     int tm, tn;
     const int bid = s.reverse ? (int)gridDim.x - 1 - (int)blockIdx.x : (int)blockIdx.x;
     tile_coords(bid, gridDim.x, g, tm, tn);
@@ -180,17 +194,18 @@ int grid_for(int64_t total) {
 
 template <typename T, class TL, bool BUF>
 void launch_struc_tl(const TileProblem<T>& p, bool a_k, bool b_k, GridInfo g,
-                     const StrucSpec& s, hipStream_t st) {
+                     const StrucSpec& s, const SplitK& sk, hipStream_t st) {
     g.grid_m = (int)((p.m + TL::BM - 1) / TL::BM);
     g.grid_n = (int)((p.n + TL::BN - 1) / TL::BN);
-    const dim3 grid(g.grid_m * g.grid_n), block(TL::NT);
+    const dim3 grid(g.grid_m * g.grid_n, sk.parts), block(TL::NT);
+    T* ws = (T*)sk.ws;
 #define BLIS_AMD_STRUC_LAUNCH(AK, BK)                                                        \
     if (s.cmask)                                                                             \
-        hipLaunchKernelGGL((gemm_struc_kernel<T, TL, AK, BK, BUF, true>), grid, block, 0, st, p,  \
-                           g, s);                                                            \
+        hipLaunchKernelGGL((gemm_struc_kernel<T, TL, AK, BK, BUF, true>), grid, block, 0, st,  \
+                           p, g, s, sk.kchunk, ws);                                          \
     else                                                                                     \
-        hipLaunchKernelGGL((gemm_struc_kernel<T, TL, AK, BK, BUF, false>), grid, block, 0, st, p, \
-                           g, s);
+        hipLaunchKernelGGL((gemm_struc_kernel<T, TL, AK, BK, BUF, false>), grid, block, 0, st, \
+                           p, g, s, sk.kchunk, ws);
     if (!a_k && !b_k) { BLIS_AMD_STRUC_LAUNCH(false, false) }
     else if (!a_k && b_k) { BLIS_AMD_STRUC_LAUNCH(false, true) }
     else if (a_k && !b_k) { BLIS_AMD_STRUC_LAUNCH(true, false) }
@@ -203,19 +218,19 @@ void launch_struc_tl(const TileProblem<T>& p, bool a_k, bool b_k, GridInfo g,
 // (gemm_default_tile): FP64 6, 10, 3, 4 and FP32 1, 12, 9, 10, 3, 4.
 template <typename T>
 void launch_struc(int tile, const TileProblem<T>& p, bool a_k, bool b_k, const GridInfo& g,
-                  const StrucSpec& s, hipStream_t st) {
+                  const StrucSpec& s, const SplitK& sk, hipStream_t st) {
     const TileShape& ts = tile_shape(dt_of<T>(), tile);
     if (!buf_problem(p, a_k, b_k, ts.bm, ts.bn, ts.bk)) {
         // Strides that buffer descriptors cannot take (gemm.hip).
         constexpr int BK = std::is_same<T, double>::value ? 16 : 32;
         if (ts.bm >= 64)
-            launch_struc_tl<T, TileCfg<T, 128, 64, BK, 32, 32>, false>(p, a_k, b_k, g, s, st);
+            launch_struc_tl<T, TileCfg<T, 128, 64, BK, 32, 32>, false>(p, a_k, b_k, g, s, sk, st);
         else
-            launch_struc_tl<T, TileCfg<T, 32, 32, BK, 16, 16>, false>(p, a_k, b_k, g, s, st);
+            launch_struc_tl<T, TileCfg<T, 32, 32, BK, 16, 16>, false>(p, a_k, b_k, g, s, sk, st);
         return;
     }
 #define BLIS_AMD_STRUC_CASE(idx, BM, BN, BK, WM, WN) \
-    case idx: launch_struc_tl<T, TileCfg<T, BM, BN, BK, WM, WN>, true>(p, a_k, b_k, g, s, st); return;
+    case idx: launch_struc_tl<T, TileCfg<T, BM, BN, BK, WM, WN>, true>(p, a_k, b_k, g, s, sk, st); return;
     if constexpr (std::is_same<T, double>::value) {
         switch (tile) {
         BLIS_AMD_STRUC_CASE(6, 128, 128, 16, 64, 32)
@@ -276,13 +291,25 @@ void gemm_struc_run(const GemmDesc& d, StrucSpec s, hipStream_t st) {
     g.group_m = 8;
     g.xcd_remap = 0;
     s.reverse = (s.kmode == K_ROW_END || s.kmode == K_COL_END) ? 1 : 0;
-    const int tile = gemm_default_tile(d.dt, pl.m, pl.n, pl.k);
+    int tile = gemm_default_tile(d.dt, pl.m, pl.n, pl.k);
+    SplitK sk;
+    if (s.cmask) {
+        // Few stored tiles over a long k: partitions of k, as for a plain
+        // product (500 x 500 from k = 30000, FP64: 1637 us in one pass).
+        const SplitChoice choice = split_on_stream(d.dt, pl.m, pl.n, pl.k, true, st);
+        sk = split_params(pl.k, choice.split);
+        if (sk.parts > 1) {
+            tile = choice.tile;
+            sk.ws = stream_scratch((size_t)sk.parts * pl.m * pl.n * dt_size(d.dt), st);
+        }
+    }
     if (d.dt == Dt::F64)
         launch_struc<double>(tile, make_problem<double>(pl, d.alpha, d.beta), pl.a_k, pl.b_k, g,
-                             s, st);
+                             s, sk, st);
     else
         launch_struc<float>(tile, make_problem<float>(pl, d.alpha, d.beta), pl.a_k, pl.b_k, g,
-                            s, st);
+                            s, sk, st);
+    if (sk.parts > 1) splitk_reduce_run(d.dt, sk, pl, d.beta, CMask{s.cmask, s.cdoff}, st);
 }
 
 // Dense copy of an n x n structured matrix into workspace slot `slot`

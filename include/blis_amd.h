@@ -31,8 +31,10 @@ void  bli_amd_synchronize( void );
    (split_k > 1: up to 64 partitions of whole 64-deep k blocks, each computed
    into library workspace, then added in partition order and combined with
    beta*C; 1 = one pass, or the built-in rule when tile is -1, which splits
-   only products with m, n <= k/4 and k >= 2048). Results depend on the k
-   partition only, never on the tile index or on how it was chosen. */
+   products of k > 512 whose output has few tiles, by the type and the shape
+   alone; under stream capture only those with m, n <= k/4 and k >= 2048).
+   Results depend on the k partition only, never on the tile index or on how
+   it was chosen. */
 void bli_amd_gemm_set_config( int tile, int group_m, int xcd_remap, int split_k );
 int  bli_amd_gemm_tile_count( int is_double );
 int  bli_amd_gemm_default_tile( int is_double, long long m, long long n, long long k );
@@ -42,9 +44,10 @@ int  bli_amd_gemm_default_tile( int is_double, long long m, long long n, long lo
    memory: code under HIP graph capture, serving loops, harnesses that
    forbid hipMalloc. C := beta*C + alpha*op(A)*op(B) for dt BLIS_FLOAT or
    BLIS_DOUBLE, with the same kernels and default configuration as
-   bli_?gemm (the results are the same bits). A, B and C must be device
-   memory; alpha and beta are host pointers. The call is asynchronous on
-   `stream` (a hipStream_t; NULL is the null stream) and allocates nothing:
+   bli_?gemm (the results are the same bits, except where the array has no
+   room for the k partitions beside packed operands and one pass is made).
+   A, B and C must be device memory; alpha and beta are host pointers. The
+   call is asynchronous on `stream` (a hipStream_t; NULL is the null stream) and allocates nothing:
    the scratch it needs (split-k partitions, packed copies of general-stride
    operands) comes from one fixed 64 MiB array per GPU that the library
    holds until the process ends. Every call on a GPU shares that array, so
