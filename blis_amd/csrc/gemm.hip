@@ -30,7 +30,8 @@ using namespace dev;
 // there first, into its own m x n column-major slice of `parts` (ld = m).
 // splitk_reduce_kernel then forms C.
 template <typename T, class TL, bool A_K, bool B_K, bool BUF>
-__global__ __launch_bounds__(TL::NT) void gemm_kernel(TileProblem<T> p, GridInfo g,
+__global__ __launch_bounds__(TL::NT)
+__attribute__((amdgpu_waves_per_eu(TL::waves_per_eu()))) void gemm_kernel(TileProblem<T> p, GridInfo g,
                                                       int64_t kchunk, T* parts) {
     __shared__ T smem[2 * TL::STAGE];
     if (gridDim.y > 1) {
@@ -53,7 +54,8 @@ __global__ __launch_bounds__(TL::NT) void gemm_kernel(TileProblem<T> p, GridInfo
 // C_z := beta*C_z + alpha*A_z*B_z with A_z = A + z*sa, B_z = B + z*sb,
 // C_z = C + z*sc.
 template <typename T, class TL, bool A_K, bool B_K, bool BUF>
-__global__ __launch_bounds__(TL::NT) void gemm_strided_kernel(TileProblem<T> p, GridInfo g,
+__global__ __launch_bounds__(TL::NT)
+__attribute__((amdgpu_waves_per_eu(TL::waves_per_eu()))) void gemm_strided_kernel(TileProblem<T> p, GridInfo g,
                                                               int64_t sa, int64_t sb, int64_t sc) {
     __shared__ T smem[2 * TL::STAGE];
     const int64_t z = blockIdx.y;

@@ -94,6 +94,20 @@ struct TileCfg {
     static constexpr int STAGE = A_ELEMS + B_ELEMS;
     static constexpr int NVA = (BM * BK / V) / NT;  // 16-byte vectors per thread
     static constexpr int NVB = (BN * BK / V) / NT;
+    // Waves per SIMD a kernel of this tile is compiled for: whole workgroups,
+    // as many as the LDS holds, while the registers of a wave (accumulators,
+    // staged vectors, two sets of fragments and about 20 more) fit. The
+    // unrolled k loop would take what it likes otherwise: 166 registers and
+    // one workgroup per CU for the 128 x 128 FP64 tile, 17.8 ms at 8192^3
+    // against 15.0 ms with two.
+    static constexpr int waves_per_eu() {
+        const int es = (int)sizeof(T) / 4, per = NW >= 4 ? NW / 4 : 1;
+        const int regs = TM * TN * 4 * es + (NVA + NVB) * 4 + 2 * (TM + TN) * es + 20;
+        int w = 163840 / (2 * STAGE * (int)sizeof(T)) * NW / 4;
+        if (w > 8) w = 8;
+        while (w > per && 512 / w / 8 * 8 < regs) w -= per;
+        return w < 1 ? 1 : w;
+    }
     static_assert(WM % 16 == 0 && WN % 16 == 0, "wave tile must be 16-aligned");
     static_assert(BK % 4 == 0 && BK % V == 0, "BK must cover MFMA k and vectors");
     static_assert((BM * BK / V) % NT == 0 && NVA >= 1, "A slab must split evenly");
@@ -218,16 +232,18 @@ struct SlabLoader {
         }
     }
 
-    // Store the loaded slab into an LDS stage, k-major; kleft: its k extent
-    // if it is a partial last slab, else 0.
-    __device__ inline void store(T* S, int kleft, int tid) {
+    // Store the loaded slab into an LDS stage, k-major; kext: its k extent
+    // (BK but for a partial last slab). The mask is applied to every slab: a
+    // branch around it would end the loop's basic block, and with it the
+    // compiler's freedom to move loads, LDS traffic and MFMAs past each other
+    // (8192^3 FP64 16.0 ms with the branch, 15.0 without).
+    __device__ inline void store(T* S, int kext, int tid) {
         if constexpr (BUF && K_CONTIG) {
-            if (kleft != 0) {
 #pragma unroll
-                for (int q = 0; q < NV; ++q)
+            for (int e = 0; e < V; ++e) {
+                const bool out = (tid % CV) * V + e >= kext;
 #pragma unroll
-                    for (int e = 0; e < V; ++e)
-                        if ((tid % CV) * V + e >= kleft) r[q][e] = T(0);
+                for (int q = 0; q < NV; ++q) r[q][e] = out ? T(0) : r[q][e];
             }
         }
 #pragma unroll
@@ -252,11 +268,9 @@ __device__ inline void mma_slab(const T* As, const T* Bs,
     using vec_t = typename Mma<T>::vec_t;
     constexpr int V = TL::V;
     const int lr = lane & 15, lk = lane >> 4;
-#pragma unroll
-    for (int ks = 0; ks < TL::BK; ks += 4) {
+    auto fragments = [&](int ks, T (&af)[TL::TM], T (&bf)[TL::TN]) {
         const T* ap = As + (ks + lk) * TL::LDA + wm0 + TL::TM * lr;
         const T* bp = Bs + (ks + lk) * TL::LDB + wn0 + TL::TN * lr;
-        T af[TL::TM], bf[TL::TN];
         if constexpr (TL::TM % V == 0) {
 #pragma unroll
             for (int q = 0; q < TL::TM / V; ++q) {
@@ -279,11 +293,33 @@ __device__ inline void mma_slab(const T* As, const T* Bs,
 #pragma unroll
             for (int j = 0; j < TL::TN; ++j) bf[j] = bp[j];
         }
+    };
+    auto multiply = [&](const T (&af)[TL::TM], const T (&bf)[TL::TN]) {
 #pragma unroll
         for (int i = 0; i < TL::TM; ++i)
 #pragma unroll
             for (int j = 0; j < TL::TN; ++j)
                 acc[i][j] = Mma<T>::mma(af[i], bf[j], acc[i][j]);
+    };
+    if constexpr (sizeof(T) == 8) {
+        // The next k step's fragments are read ahead of this one's MFMAs:
+        // 1% on the FP64 tiles (128 x 128 14.68 against 14.80 ms at 8192^3
+        // N/T, 64 x 128 249 against 257 us at 2000^3); the FP32 tiles gain
+        // nothing (256 x 128 at 8192^3 N/N 7.95 against 7.66 ms).
+        T af[2][TL::TM], bf[2][TL::TN];
+        fragments(0, af[0], bf[0]);
+#pragma unroll
+        for (int i = 0; i < TL::BK / 4; ++i) {
+            if (i + 1 < TL::BK / 4) fragments(4 * (i + 1), af[(i + 1) & 1], bf[(i + 1) & 1]);
+            multiply(af[i & 1], bf[i & 1]);
+        }
+    } else {
+#pragma unroll
+        for (int ks = 0; ks < TL::BK; ks += 4) {
+            T af[TL::TM], bf[TL::TN];
+            fragments(ks, af, bf);
+            multiply(af, bf);
+        }
     }
 }
 
@@ -528,7 +564,8 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
         for (int j = 0; j < TL::TN; ++j) acc[i][j] = acc_t{};
 
     const int nk = (int)((p.k + TL::BK - 1) / TL::BK);
-    const int ktail = (int)(p.k % TL::BK);   // extent of a partial last slab
+    const int klast = (int)(p.k - (int64_t)(nk - 1) * TL::BK);   // the last slab's extent
+    auto kext = [&](int s) { return s + 1 == nk ? klast : TL::BK; };
     Loader_A al;
     Loader_B bl;
     al.init(p.a, p.m, p.k, p.lda, p.vec_a, m0, tid);
@@ -537,40 +574,49 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
     // k == 0 (a batch problem with k == 0 or alpha == 0) touches neither A
     // nor B.
     if constexpr (PF == 1) {
+        // One slab in flight. The loop runs over pairs of slabs, one per LDS
+        // stage, each step one basic block: load the next slab, multiply this
+        // one, store the next, barrier. The last slab is multiplied after it.
+        auto step = [&](auto stage, int s) {
+            constexpr int B = decltype(stage)::value;
+            T* cur = smem + B * TL::STAGE;
+            T* nxt = smem + (1 - B) * TL::STAGE;
+            al.load(s + 1, tid);
+            bl.load(s + 1, tid);
+            mma_slab<T, TL>(cur, cur + TL::A_ELEMS, acc, wm0, wn0, lane);
+            al.store(nxt, kext(s + 1), tid);
+            bl.store(nxt + TL::A_ELEMS, kext(s + 1), tid);
+            __syncthreads();
+        };
+        using Even = std::integral_constant<int, 0>;
+        using Odd = std::integral_constant<int, 1>;
         if (nk > 0) {
             al.load(0, tid);
             bl.load(0, tid);
-            al.store(smem, nk == 1 ? ktail : 0, tid);
-            bl.store(smem + TL::A_ELEMS, nk == 1 ? ktail : 0, tid);
+            al.store(smem, kext(0), tid);
+            bl.store(smem + TL::A_ELEMS, kext(0), tid);
         }
         __syncthreads();
-        if constexpr (C_PF) {
-            if (nk <= 1) prefetch_c<T, TL>(p, m0, n0, sink);
+        int s = 0;
+        for (; s + 2 < nk; s += 2) {
+            step(Even{}, s);
+            step(Odd{}, s + 1);
         }
-        for (int s = 0; s < nk; ++s) {
-            T* cur = smem + (s & 1) * TL::STAGE;
-            T* nxt = smem + ((s + 1) & 1) * TL::STAGE;
-            const bool more = (s + 1) < nk;
-            if (more) {
-                al.load(s + 1, tid);
-                bl.load(s + 1, tid);
-            }
-            if constexpr (C_PF) {
-                if (s + 2 == nk) prefetch_c<T, TL>(p, m0, n0, sink);
-            }
+        if (s + 1 < nk) {
+            step(Even{}, s);
+            ++s;
+        }
+        if constexpr (C_PF) prefetch_c<T, TL>(p, m0, n0, sink);
+        if (nk > 0) {
+            const T* cur = smem + (s & 1) * TL::STAGE;
             mma_slab<T, TL>(cur, cur + TL::A_ELEMS, acc, wm0, wn0, lane);
-            if (more) {
-                const int kleft = s + 2 == nk ? ktail : 0;
-                al.store(nxt, kleft, tid);
-                bl.store(nxt + TL::A_ELEMS, kleft, tid);
-            }
-            __syncthreads();
         }
+        if constexpr (LDS_EPI) __syncthreads();   // the epilogue reuses the stages
     } else {
         // Two register buffers. At step s, buffer (s & 1) has already been
         // written to LDS and now receives slab s + 2; buffer ((s + 1) & 1)
         // holds slab s + 1 and is written to the other LDS stage after the
-        // multiply. The loop is unrolled by two so that each buffer is a
+        // multiply. The loop runs over pairs of slabs so that each buffer is a
         // fixed set of registers; one loader walks the slabs and its loaded
         // registers change places with the second buffer's.
         typename Mma<T>::vec_t ra[TL::NVA], rb[TL::NVB];   // odd slabs
@@ -590,13 +636,12 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
             }
         };
         auto store = [&](auto buf, T* S, int s) {
-            const int kleft = s + 1 == nk ? ktail : 0;
             if constexpr (decltype(buf)::value == 0) {
-                al.store(S, kleft, tid);
-                bl.store(S + TL::A_ELEMS, kleft, tid);
+                al.store(S, kext(s), tid);
+                bl.store(S + TL::A_ELEMS, kext(s), tid);
             } else {
-                swap_in(al, ra, [&] { al.store(S, kleft, tid); });
-                swap_in(bl, rb, [&] { bl.store(S + TL::A_ELEMS, kleft, tid); });
+                swap_in(al, ra, [&] { al.store(S, kext(s), tid); });
+                swap_in(bl, rb, [&] { bl.store(S + TL::A_ELEMS, kext(s), tid); });
             }
         };
         using Even = std::integral_constant<int, 0>;
@@ -607,19 +652,38 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
             store(Even{}, smem, 0);
         }
         __syncthreads();
-        auto step = [&](auto buf, int s) {
-            constexpr int B = decltype(buf)::value;   // == s & 1
-            T* cur = smem + B * TL::STAGE;
-            T* nxt = smem + (1 - B) * TL::STAGE;
-            if (s + 2 < nk) load(buf, s + 2);
+        auto multiply = [&](auto stage) {
+            const T* cur = smem + decltype(stage)::value * TL::STAGE;
             mma_slab<T, TL>(cur, cur + TL::A_ELEMS, acc, wm0, wn0, lane);
-            if (s + 1 < nk) store(std::integral_constant<int, 1 - B>{}, nxt, s + 1);
+        };
+        auto stage_next = [&](auto buf, int s) {   // slab s + 1 to the other stage
+            constexpr int B = decltype(buf)::value;
+            store(std::integral_constant<int, 1 - B>{}, smem + (1 - B) * TL::STAGE, s + 1);
             __syncthreads();
         };
-        for (int s = 0; s < nk; s += 2) {
+        auto step = [&](auto buf, int s) {         // slab s, with s + 2 < nk
+            load(buf, s + 2);
+            multiply(buf);
+            stage_next(buf, s);
+        };
+        int s = 0;
+        for (; s + 3 < nk; s += 2) {
             step(Even{}, s);
-            if (s + 1 < nk) step(Odd{}, s + 1);
+            step(Odd{}, s + 1);
         }
+        if (nk - s == 3) {
+            step(Even{}, s);
+            multiply(Odd{});
+            stage_next(Odd{}, s + 1);
+            multiply(Even{});
+        } else if (nk - s == 2) {
+            multiply(Even{});
+            stage_next(Even{}, s);
+            multiply(Odd{});
+        } else if (nk - s == 1) {
+            multiply(Even{});
+        }
+        if constexpr (LDS_EPI) __syncthreads();
     }
 
     if constexpr (MASK)

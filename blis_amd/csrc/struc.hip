@@ -66,7 +66,8 @@ StrucSpec transposed(const StrucSpec& s) {
 // One tile of a structured product. Workgroups are uniform in (tm, tn), so
 // the early return is taken by the whole workgroup before any barrier.
 template <typename T, class TL, bool A_K, bool B_K, bool BUF, bool MASK>
-__global__ __launch_bounds__(TL::NT) void gemm_struc_kernel(TileProblem<T> p, GridInfo g,
+__global__ __launch_bounds__(TL::NT)
+__attribute__((amdgpu_waves_per_eu(TL::waves_per_eu()))) void gemm_struc_kernel(TileProblem<T> p, GridInfo g,
                                                             StrucSpec s, int64_t kchunk,
                                                             T* parts) {
     __shared__ T smem[2 * TL::STAGE];
