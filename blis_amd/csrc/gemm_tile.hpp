@@ -73,6 +73,14 @@ template <> struct Mma<float> {
     __device__ static constexpr int acc_row(int r, int g) { return 4 * g + r; }
 };
 
+// Workgroup barrier that orders LDS accesses only. __syncthreads() also waits
+// for every global load in flight, which undoes prefetching across it.
+__device__ inline void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Workgroup tile BM x BN, k slab BK, wave tile WM x WN.
 template <typename T, int BM_, int BN_, int BK_, int WM_, int WN_>
 struct TileCfg {

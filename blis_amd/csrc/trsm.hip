@@ -16,25 +16,29 @@
 // L_eff * X = alpha * B' with L_eff lower or upper, by folding op(A) and the
 // side into strides. The solve recurses on halves: solve the leading half,
 // update the trailing half with one GEMM (the bulk of the m^2 n flops, on the
-// MFMA GEMM path), solve the trailing half. Leaves of at most NB = 256 rows
-// are solved by trsm_leaf_kernel in native precision: a wave owns CPW
-// columns of B with one row per lane per 64-row register block, and solves
-// by broadcast substitution against rows of the triangle held in registers,
-// multiplying by the reciprocal of each diagonal element.
+// MFMA GEMM path), solve the trailing half. Leaves of at most 512 rows are
+// solved by substitution in one launch (trsm_slab_kernel); when the triangle
+// is diagonally dominant and large, whole 512-row blocks are solved by a
+// product with their inverse instead.
 #include "internal.hpp"
+#include "gemm_tile.hpp"
 
 namespace blis_amd {
 
 namespace detail_trsm {
 
-constexpr int BR = 64;          // rows per register block (one per lane)
-constexpr int P = 4;            // register blocks per leaf
-constexpr int NB = BR * P;      // leaf rows
-constexpr int WPB = 4;          // waves per workgroup
-// Right-hand sides from which the inverted-diagonal path pays: inverting a
-// block costs about as much as solving NB right-hand sides by substitution.
+constexpr int64_t LB = 64;      // rows of the blocks inverted by substitution
+constexpr int WPB = 4;          // waves per workgroup of that kernel
+constexpr int NB = 256;         // rows of a block of the dominance check
+constexpr int64_t PB = 512;     // rows of a block solved by product
+constexpr int64_t SLAB = 512;   // most rows of a leaf solved by substitution
+// Right-hand sides and rows from which the inverted-diagonal path pays: it
+// spends about 75 us on checking and inverting, lost when a block fails the
+// check. FP64, n = 1024, by substitution and by product (us): 1024 rows 134
+// and 120, 2048 rows 313 and 233, 4096 rows 800 and 581.
 constexpr int64_t TRSM_INV_MIN_N = 512;
-// Columns per wave when inverting the diagonal blocks: each wave reads the
+constexpr int64_t TRSM_INV_MIN_ROWS = 3 * PB;
+// Columns per wave when inverting the 64-row blocks: each wave reads the
 // triangle's rows once for all of its columns.
 constexpr int INV_CPW = 2;
 
@@ -48,132 +52,227 @@ __device__ inline float lane_bcast(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// Solve a leaf of nrows <= NB rows for all n columns of B:
-// L * X = alpha * B with L(i,j) = a[i*ars + j*acs] (lower or upper, only the
-// stored triangle is read), B(i,j) = b[i*brs + j*bcs], X overwrites B.
-// Each wave owns CPW columns; its slab of B sits in LDS as P blocks of 64
-// rows (lane l holds row p*64 + l). Blocks are solved in order: the block in
-// work is loaded into registers, updated by the blocks solved before it
-// (x -= L_pq x_q, the gemm part of gemmtrsm, reading x_q as LDS broadcasts),
-// then solved by 64 broadcast steps: the solved row i, scaled by the
-// reciprocal of the diagonal, is read from lane i and every other lane
-// subtracts its L element times it.
-// Several independent leaves in one launch: leaf y = blockIdx.y starts at
-// a + y*a_step, b + y*b_step, and the last one has nrows_last rows.
-// INV: the right-hand side is alpha times the identity (b is written only),
-// so the leaf computes alpha inv(L). A wave's CPW columns lie in one 64-row
-// block p0, and the solution is zero in the blocks on the far side of p0
-// (above it for a lower triangle, below it for an upper one): those are
-// neither solved nor used in updates.
-template <typename T, bool LOWER, int CPW, bool INV = false>
-__global__ __launch_bounds__(64 * WPB) void trsm_leaf_kernel(const T* __restrict__ a, int64_t ars,
-                                                             int64_t acs, T* __restrict__ b,
-                                                             int64_t brs, int64_t bcs,
-                                                             int nrows, int64_t n, T alpha,
-                                                             int unit_diag, int64_t a_step,
-                                                             int64_t b_step, int nrows_last,
-                                                             int zgroup) {
-    __shared__ T xs[WPB][P][CPW][BR];
+// Inverses of 64-row diagonal blocks, one per blockIdx.y: block y is the
+// triangle at a + y*a_step (only the stored part is read), its inverse goes
+// to b + y*b_step with columns bcs apart. A wave owns CPW columns, row l of
+// them in lane l, and substitutes into columns of the identity: the solved
+// row i, scaled by the reciprocal of the diagonal, is read from lane i and
+// every other lane subtracts its L element times it. The block also zeroes
+// its columns of the 512-row block on the far side of the diagonal.
+template <typename T, bool LOWER, int CPW>
+__global__ __launch_bounds__(64 * WPB) void trsm_inverse_kernel(const T* __restrict__ a,
+                                                                int64_t ars, int64_t acs,
+                                                                T* __restrict__ b, int64_t bcs,
+                                                                int unit_diag, int64_t a_step,
+                                                                int64_t b_step) {
     a += (int64_t)blockIdx.y * a_step;
     b += (int64_t)blockIdx.y * b_step;
-    if (blockIdx.y == gridDim.y - 1) nrows = nrows_last;
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int64_t col0 = ((int64_t)blockIdx.x * WPB + wave) * CPW;
-    if (col0 >= n) return;      // whole wave leaves together (no block barriers below)
-    const int nblk = (nrows + BR - 1) / BR;
-
-    for (int p = 0; p < nblk; ++p)
+    const int col0 = (blockIdx.x * WPB + (threadIdx.x >> 6)) * CPW;
+    T x[CPW], l[LB];
+#pragma unroll
+    for (int c = 0; c < CPW; ++c) x[c] = lane == col0 + c ? T(1) : T(0);
+#pragma unroll
+    for (int i = 0; i < (int)LB; ++i) {
+        const bool stored = LOWER ? i < lane : i > lane;
+        l[i] = stored ? a[lane * ars + i * acs] : T(0);
+    }
+    const T inv = unit_diag ? T(1) : T(1) / a[lane * (ars + acs)];
+#pragma unroll
+    for (int s = 0; s < (int)LB; ++s) {
+        const int i = LOWER ? s : (int)LB - 1 - s;
+        const T inv_i = lane_bcast(inv, i);
 #pragma unroll
         for (int c = 0; c < CPW; ++c) {
-            const int r = p * BR + lane;
-            const int64_t col = col0 + c;
-            T v = T(0);
-            if (INV) v = (r < nrows && col < n && r == col) ? alpha : T(0);
-            else if (r < nrows && col < n) v = alpha * b[r * brs + col * bcs];
-            xs[wave][p][c][lane] = v;
+            const T xi = lane_bcast(x[c], i) * inv_i;
+            // Rows solved earlier are left as they are (an Inf in xi must
+            // not turn them into NaN through a zero of L).
+            if (lane == i) x[c] = xi;
+            else if (LOWER ? lane > i : lane < i) x[c] -= l[i] * xi;
         }
-    __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int c = 0; c < CPW; ++c) b[lane + (col0 + c) * bcs] = x[c];
+    constexpr int GROUP = (int)(PB / LB);
+    const int d = (int)(blockIdx.y % GROUP);
+    const int z0 = LOWER ? -d * (int)LB : (int)LB;
+    const int zn = LOWER ? d * (int)LB : (GROUP - 1 - d) * (int)LB;
+    for (int r = lane; r < zn; r += 64)
+#pragma unroll
+        for (int c = 0; c < CPW; ++c) b[(z0 + r) + (col0 + c) * bcs] = T(0);
+}
 
-    // First block in solve order that can be nonzero.
-    int t0 = 0;
-    if (INV) {
-        const int p0 = (int)(col0 / BR);
-        t0 = LOWER ? p0 : nblk - 1 - p0;
-        if (t0 < 0) t0 = 0;
-    }
-    T Lr[BR];
-#pragma unroll 1
-    for (int t = t0; t < nblk; ++t) {
-        const int pb = LOWER ? t : nblk - 1 - t;   // block being solved
-        const int row = pb * BR + lane;
-        T x[CPW];
-#pragma unroll
-        for (int c = 0; c < CPW; ++c) x[c] = xs[wave][pb][c][lane];
-        // Updates from the blocks solved earlier.
-#pragma unroll 1
-        for (int u = t0; u < t; ++u) {
-            const int q = LOWER ? u : nblk - 1 - u;
-#pragma unroll
-            for (int i = 0; i < BR; ++i) {
-                const int colA = q * BR + i;
-                Lr[i] = (row < nrows && colA < nrows) ? a[row * ars + colA * acs] : T(0);
-            }
-#pragma unroll
-            for (int i = 0; i < BR; ++i)
-#pragma unroll
-                for (int c = 0; c < CPW; ++c) x[c] -= Lr[i] * xs[wave][q][c][i];
-        }
-        // Diagonal block: stored triangle only, reciprocal of the diagonal.
-#pragma unroll
-        for (int i = 0; i < BR; ++i) {
-            const int colA = pb * BR + i;
-            const bool stored = LOWER ? (i < lane) : (i > lane);
-            Lr[i] = (stored && row < nrows && colA < nrows) ? a[row * ars + colA * acs] : T(0);
-        }
-        T inv = T(1);
-        if (!unit_diag && row < nrows) inv = T(1) / a[row * ars + row * acs];
-#pragma unroll
-        for (int s = 0; s < BR; ++s) {
-            const int i = LOWER ? s : BR - 1 - s;
-            const T inv_i = lane_bcast(inv, i);
-#pragma unroll
-            for (int c = 0; c < CPW; ++c) {
-                const T xi = lane_bcast(x[c], i) * inv_i;
-                // Rows solved earlier are left as they are (an Inf in xi
-                // must not turn them into NaN through a zero of L).
-                if (lane == i) x[c] = xi;
-                else if (LOWER ? lane > i : lane < i) x[c] -= Lr[i] * xi;
-            }
-        }
-#pragma unroll
-        for (int c = 0; c < CPW; ++c) xs[wave][pb][c][lane] = x[c];
-        // LDS is in order within a wave; this keeps the compiler from moving
-        // the reads of the next block above the writes.
-        __builtin_amdgcn_wave_barrier();
-    }
+// Solve L X = alpha B for m <= 128 * SLOTS rows and the 16 columns of B that a
+// workgroup of eight waves owns, by substitution. L(i, j) = a[i*ars + j*acs]
+// is lower triangular (an upper one comes with reversed rows and columns,
+// that is negative strides) and only its stored triangle is read;
+// B(i, j) = b[i*brs + j*bcs], X(i, j) = x[i*xrs + j*xcs], which may be B.
+//
+// The rows are tiles of 16; wave w keeps tiles w, w + 8, ... of its columns in
+// MFMA accumulators for the whole solve, row 4g + r of a tile in register r
+// of lane group g. (The FP64 accumulator holds D row 4r + g there, so its L
+// operand carries the tile's rows in the order 0, 4, 8, 12, 1, ...) A solved
+// tile's registers then are, as they stand, the four k steps of an MFMA's B
+// operand over columns 4g + r of L. Step q: every wave subtracts L(:, q-1)
+// X(q-1) from its tiles below, four MFMAs each, the owner of tile q first,
+// which then solves it while the others go on. The 16 x 16 diagonal block is
+// solved four rows at a time, which one lane holds for its column: plain
+// substitution inside the lane, each row scaled by the reciprocal of its
+// diagonal element, then four MFMAs subtract those rows from the ones below.
+// The chain of steps is the bound (1.6 us each in FP64, 1.2 in FP32, half of it
+// the diagonal block), so what a step needs is fetched ahead: L two steps, the
+// diagonal blocks before the first. 512 rows take 57 us (FP32 39) for up to 4096
+// columns, 256 rows 26 (19); a kernel that substitutes 64 rows at a time across
+// a wave took 83 us (68) for 256 rows. Also measured: one column of the tile
+// per lane with the block's elements as LDS broadcasts, 121 us for 512 rows;
+// rows broadcast across lane groups, 81 us; tiles for 1024 rows in one launch,
+// no faster than two leaves and an update.
+template <typename T, int SLOTS>
+__global__ __launch_bounds__(512) void trsm_slab_kernel(const T* __restrict__ a, int64_t ars,
+                                                        int64_t acs, const T* b, int64_t brs,
+                                                        int64_t bcs, T* xo, int64_t xrs,
+                                                        int64_t xcs, int m, int64_t n, T alpha,
+                                                        int unit_diag) {
+    using acc_t = typename dev::Mma<T>::acc_t;
+    __shared__ T xb[2][256];             // -X of the last two tiles, [register][lane]
+    __shared__ T diag[8 * SLOTS][256];   // diagonal blocks, [column][row], reciprocal diagonal
+    const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
+    const int lr = sizeof(T) == 8 ? 4 * (c & 3) + (c >> 2) : c;   // L operand row of this lane
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int P = (m + 15) / 16;
+    const int64_t col0 = (int64_t)blockIdx.x * 16;
+    const int64_t colc = (col0 + c < n ? col0 + c : n - 1) * bcs;
 
-    for (int p = 0; p < nblk; ++p)
+    // Rows and columns past the edge are clamped on load and not stored; in
+    // the last diagonal block they are rows of the identity.
+    acc_t acc[SLOTS];
+    const T* lp[SLOTS];
 #pragma unroll
-        for (int c = 0; c < CPW; ++c) {
-            const int r = p * BR + lane;
-            const int64_t col = col0 + c;
-            if (r < nrows && col < n) b[r * brs + col * bcs] = xs[wave][p][c][lane];
-        }
-    // Inverses of nrows-row leaves inside a block of zgroup leaves (INV
-    // only): zero the leaf's columns of that block on the far side of the
-    // diagonal, rows above the leaf (lower) or below it (upper).
-    if (INV && zgroup > 0) {
-        const int d = (int)(blockIdx.y % zgroup);
-        const int z0 = LOWER ? -d * nrows : nrows;
-        const int zn = LOWER ? d * nrows : (zgroup - 1 - d) * nrows;
-        for (int r = lane; r < zn; r += 64)
+    for (int j = 0; j < SLOTS; ++j) {
+        const int t = 8 * j + w;
+        acc[j] = acc_t{};
+        lp[j] = a + min(t * 16 + lr, m - 1) * ars + 4 * g * acs;
+        if (t < P) {
 #pragma unroll
-            for (int c = 0; c < CPW; ++c) {
-                const int64_t col = col0 + c;
-                if (col < n) b[(int64_t)(z0 + r) * brs + col * bcs] = T(0);
+            for (int r = 0; r < 4; ++r) {
+                const int row = min(t * 16 + 4 * g + r, m - 1);
+                acc[j][r] = alpha * b[row * brs + colc];
             }
+        }
     }
+    T l[2][SLOTS][4];
+    auto load_l = [&](auto buf, int p) {           // L(t, p) of the wave's tiles t > p
+        const int64_t off = (int64_t)p * 16 * acs;
+#pragma unroll
+        for (int j = 0; j < SLOTS; ++j)
+            if (8 * j + w > p && 8 * j + w < P)
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    l[decltype(buf)::value][j][k] = lp[j][off + k * acs];
+    };
+    // The diagonal blocks, one wave each at a time: row c, columns 4e + g.
+#pragma unroll 4
+    for (int q = w; q < P; q += 8) {
+        T v[4], own = T(1);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int dj = 4 * e + g, i = q * 16 + c;
+            v[e] = T(0);
+            if (i < m && (c > dj || (c == dj && !unit_diag)))
+                v[e] = a[i * ars + (int64_t)(q * 16 + dj) * acs];
+            own = c == dj && i < m && !unit_diag ? v[e] : own;
+        }
+        const T inv = T(1) / own;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            diag[q][(4 * e + g) * 16 + c] = c == 4 * e + g ? inv : v[e];
+    }
+    auto store_x = [&](int q) {                    // tile q of X, by one wave
+        const T* src = xb[q & 1];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            // Lanes along X's unit stride.
+            const int u = 4 * e + g, i = xcs == 1 ? u : c, j = xcs == 1 ? c : u;
+            if (q * 16 + i < m && col0 + j < n)
+                xo[(q * 16 + i) * xrs + (col0 + j) * xcs] = -src[(i & 3) * 64 + (i >> 2) * 16 + j];
+        }
+    };
+    using B0 = std::integral_constant<int, 0>;
+    using B1 = std::integral_constant<int, 1>;
+    load_l(B0{}, 0);
+    load_l(B1{}, 1);
+    __syncthreads();
+
+    auto step = [&](auto buf, int q) {
+        constexpr int B = decltype(buf)::value;    // == q & 1
+        T xf[4] = {};
+        auto subtract = [&](acc_t& d, const T (&lt)[4]) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) d = dev::Mma<T>::mma(lt[k], xf[k], d);
+        };
+        if (q > 0) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) xf[k] = xb[1 - B][k * 64 + lane];
+        }
+        if (w == (q & 7)) {
+            // The lane group's own 4 x 4 diagonal block, and the columns of
+            // L below it as an A operand.
+            const T* D = diag[q] + 4 * g * 17;
+            const T i0 = D[0], i1 = D[17], i2 = D[34], i3 = D[51];
+            const T l10 = D[1], l20 = D[2], l30 = D[3], l21 = D[18], l31 = D[19], l32 = D[35];
+            T low[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) low[k] = lr >= 4 * g + 4 ? diag[q][(4 * g + k) * 16 + lr] : T(0);
+            acc_t v = acc_t{};
+#pragma unroll
+            for (int j = 0; j < SLOTS; ++j)
+                if (8 * j + w == q) {
+                    if (q > 0) subtract(acc[j], l[1 - B][j]);
+                    v = acc[j];
+                }
+            T x[4] = {};                           // -X, rows 4g + r
+            auto rows = [&](auto sub) {            // rows 4s .. 4s + 3, held by lane group s
+                constexpr int s = decltype(sub)::value;
+                const T x0 = v[0] * i0;
+                const T x1 = (v[1] - l10 * x0) * i1;
+                const T x2 = (v[2] - l20 * x0 - l21 * x1) * i2;
+                const T x3 = (v[3] - l30 * x0 - l31 * x1 - l32 * x2) * i3;
+                // Zeros everywhere else, in both operands and in what is kept:
+                // an Inf of these rows or of L must not reach a row through a
+                // product that substitution does not form.
+                const bool own = g == s;
+                const T y[4] = { -x0, -x1, -x2, -x3 };
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    x[k] = own ? y[k] : x[k];
+                    if constexpr (s < 3)
+                        v = dev::Mma<T>::mma(own ? low[k] : T(0), own ? y[k] : T(0), v);
+                }
+            };
+            rows(std::integral_constant<int, 0>{});
+            rows(std::integral_constant<int, 1>{});
+            rows(std::integral_constant<int, 2>{});
+            rows(std::integral_constant<int, 3>{});
+#pragma unroll
+            for (int k = 0; k < 4; ++k) xb[B][k * 64 + lane] = x[k];
+        }
+        if (q > 0) {
+#pragma unroll
+            for (int j = 0; j < SLOTS; ++j)
+                if (8 * j + w > q && 8 * j + w < P) subtract(acc[j], l[1 - B][j]);
+            if (w == ((q + 4) & 7)) store_x(q - 1);
+        }
+        if (q + 1 < P) {
+            load_l(std::integral_constant<int, 1 - B>{}, q + 1);
+        }
+        dev::lds_barrier();
+    };
+#pragma unroll 1
+    for (int q = 0; q < P; q += 2) {
+        step(B0{}, q);
+        if (q + 1 < P) step(B1{}, q + 1);
+    }
+    if (w == 0) store_x(P - 1);
 }
 
 // Which diagonal blocks may be solved by multiplying with their inverse.
@@ -259,34 +358,23 @@ struct Solve {
     bool lower;
     bool unit;
     View a;          // L_eff(i,j) = a.ptr[i*a.rs + j*a.cs]
-    View b;          // B'(i,j)    = b.ptr[i*b.rs + j*b.cs]
     int64_t n;
     hipStream_t st;
-    // Inverted diagonal blocks (NB x NB each, column-major, ld NB) and the
-    // per-block flag that allows their use; null when not prepared.
-    const void* linv = nullptr;
-    const int* inv_ok = nullptr;
-    void* wtmp = nullptr;   // NB x n staging for a product leaf solved in place
     // Where the updates modify the right-hand side and where the solved rows
-    // live. Both are b for the in-place solve; when every block is solved by
-    // product they are separate buffers and B is written once at the end.
+    // live: B' for both, or separate buffers when blocks are solved by product
+    // (B is then written once at the end).
     View rhs;
     View x;
-    bool separate = false;
-    // Solves with every block inverted: inverses of the first npair aligned
-    // 512-row diagonal blocks (512 x 512 each, column-major, ld 512).
-    const void* linv2 = nullptr;
-    int64_t npair = 0;
-    // Band store of the inverses (when set, linv and linv2 only mark that
-    // the 256- and 512-row inverses exist): element (i, j) of the block
-    // diagonal inverse at band[(i - j + BAND_KL) + j * BAND_LD], so every
-    // diagonal block, and every block within BAND_KL of the diagonal, is a
-    // column-major matrix with leading dimension BAND_LD - 1, and the
-    // blocks along the diagonal are a constant stride apart.
+    // Band store of the inverses of the whole 512-row diagonal blocks, when
+    // those are solved by product: element (i, j) of the block diagonal
+    // inverse at band[(i - j + BAND_KL) + j * BAND_LD], so every diagonal
+    // block, and every block within BAND_KL of the diagonal, is a
+    // column-major matrix with leading dimension BAND_LD - 1, and the blocks
+    // along the diagonal are a constant stride apart.
     const void* band = nullptr;
 };
 
-constexpr int64_t BAND_KL = 2 * NB;
+constexpr int64_t BAND_KL = PB;
 constexpr int64_t BAND_LD = 2 * BAND_KL + 1;
 
 // Block (r, c) of the inverse in the band store (|r - c| + block size - 1 <= BAND_KL).
@@ -295,104 +383,47 @@ inline View band_view(const Solve& s, int64_t r, int64_t c) {
              1, BAND_LD - 1 };
 }
 
-// Diagonal quarters of the 512-row inverses from the 256-row ones (block
-// 2p at the top left, 2p+1 at the bottom right of pair p) and zeros in the
-// quarter outside the triangle; the other off-diagonal quarter is written by
-// GEMMs.
-template <typename T>
-__global__ __launch_bounds__(256) void trsm_assemble_kernel(const T* __restrict__ linv,
-                                                            T* __restrict__ linv2,
-                                                            int64_t npair, int upper) {
-    constexpr int64_t PB = 2 * NB;
-    const int64_t total = npair * PB * PB;
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total;
-         t += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t p = t / (PB * PB), e = t % (PB * PB), i = e % PB, j = e / PB;
-        if (upper ? (i < NB && j >= NB) : (i >= NB && j < NB)) continue;
-        T v = T(0);
-        if (i < NB && j < NB) v = linv[(2 * p) * NB * NB + i + j * NB];
-        else if (i >= NB && j >= NB) v = linv[(2 * p + 1) * NB * NB + (i - NB) + (j - NB) * NB];
-        linv2[t] = v;
-    }
-}
-
 inline void* offset(const View& v, int64_t i, int64_t j, size_t es) {
     return (char*)v.ptr + (i * v.rs + j * v.cs) * (int64_t)es;
 }
 
-// Launch `count` leaves of the same shape: leaf y solves the nb-row (the
-// last one nb_last-row) triangle at a + y*a_step for the n columns at
-// b + y*b_step with strides (brs, bcs).
-template <typename T, int CPW, bool INV = false>
-void leaf_launch(bool lower, bool unit, const void* a, int64_t ars, int64_t acs, void* b,
-                 int64_t brs, int64_t bcs, int64_t nb, int64_t n, double alpha, int count,
-                 int64_t a_step, int64_t b_step, int64_t nb_last, hipStream_t st,
-                 int zgroup = 0) {
-    static_assert(BR % CPW == 0, "a wave's columns must lie in one 64-row block");
-    const int64_t waves = (n + CPW - 1) / CPW;
-    const dim3 grid((unsigned)((waves + WPB - 1) / WPB), (unsigned)count), block(64 * WPB);
-    if (lower)
-        hipLaunchKernelGGL((trsm_leaf_kernel<T, true, CPW, INV>), grid, block, 0, st,
-                           (const T*)a, ars, acs, (T*)b, brs, bcs, (int)nb, n, (T)alpha,
-                           (int)unit, a_step, b_step, (int)nb_last, zgroup);
+// Inverses of `count` consecutive 64-row diagonal blocks into the band.
+template <typename T>
+void inverse_launch(const Solve& s, int count) {
+    const View b0 = band_view(s, 0, 0);
+    const dim3 grid((unsigned)(LB / INV_CPW / WPB), (unsigned)count), block(64 * WPB);
+    const int64_t a_step = LB * (s.a.rs + s.a.cs), b_step = LB * BAND_LD;
+    if (s.lower)
+        hipLaunchKernelGGL((trsm_inverse_kernel<T, true, INV_CPW>), grid, block, 0, s.st,
+                           (const T*)s.a.ptr, s.a.rs, s.a.cs, (T*)b0.ptr, b0.cs, (int)s.unit,
+                           a_step, b_step);
     else
-        hipLaunchKernelGGL((trsm_leaf_kernel<T, false, CPW, INV>), grid, block, 0, st,
-                           (const T*)a, ars, acs, (T*)b, brs, bcs, (int)nb, n, (T)alpha,
-                           (int)unit, a_step, b_step, (int)nb_last, zgroup);
+        hipLaunchKernelGGL((trsm_inverse_kernel<T, false, INV_CPW>), grid, block, 0, s.st,
+                           (const T*)s.a.ptr, s.a.rs, s.a.cs, (T*)b0.ptr, b0.cs, (int)s.unit,
+                           a_step, b_step);
     HIP_CHECK(hipGetLastError());
 }
 
-template <typename T, int CPW>
-void leaf_t(const Solve& s, const void* a, void* b, int64_t nb, double alpha) {
-    leaf_launch<T, CPW>(s.lower, s.unit, a, s.a.rs, s.a.cs, b, s.b.rs, s.b.cs, nb, s.n, alpha, 1,
-                        0, 0, nb, s.st);
-}
-
-// A leaf whose diagonal block passed the check: X_q = alpha * inv(L_qq) * R_q
-// as one GEMM, straight into x when it is a separate buffer, else into
-// staging and then copied over B_q.
-void leaf_by_product(const Solve& s, int64_t r0, int64_t nb, double alpha) {
-    const size_t es = dt_size(s.dt);
-    const int64_t q = r0 / NB;
-    GemmDesc d;
-    d.dt = s.dt;
-    d.m = nb; d.n = s.n; d.k = nb;
-    d.a = s.band ? band_view(s, r0, r0) : View{ (char*)s.linv + (size_t)q * NB * NB * es, 1, NB };
-    d.b = { offset(s.rhs, r0, 0, es), s.rhs.rs, s.rhs.cs };
-    d.alpha = alpha;
-    d.beta = 0.0;
-    if (s.separate) {
-        d.c = { offset(s.x, r0, 0, es), s.x.rs, s.x.cs };
-        gemm_run(d, nullptr, s.st);
-        return;
-    }
-    d.c = { s.wtmp, 1, nb };
-    gemm_run(d, nullptr, s.st);
-    const int64_t tiles = ((nb + 63) / 64) * ((s.n + 63) / 64);
-    const unsigned g = (unsigned)std::max<int64_t>(1, std::min<int64_t>(tiles, 8192));
-    if (s.dt == Dt::F64)
-        hipLaunchKernelGGL(trsm_copy_kernel<double>, dim3(g), dim3(256), 0, s.st,
-                           (const double*)s.wtmp, 1, nb, (double*)offset(s.b, r0, 0, es), s.b.rs,
-                           s.b.cs, nb, s.n);
+// X[r0 .. r0 + m - 1] = alpha * inv(L_rr) * R[r0 ..] by substitution, m <= SLAB.
+template <typename T>
+void slab(const Solve& s, int64_t r0, int64_t m, double alpha) {
+    const size_t es = sizeof(T);
+    // An upper triangle is a lower one with its rows and columns reversed.
+    const int64_t d = s.lower ? 1 : -1, f = s.lower ? r0 : r0 + m - 1;
+    const dim3 grid((unsigned)((s.n + 15) / 16)), block(512);
+    const T* a = (const T*)offset(s.a, f, f, es);
+    const T* b = (const T*)offset(s.rhs, f, 0, es);
+    T* x = (T*)offset(s.x, f, 0, es);
+    // Two or four 16-row tiles per wave (up to 256 or 512 rows).
+    if (m <= 256)
+        hipLaunchKernelGGL((trsm_slab_kernel<T, 2>), grid, block, 0, s.st, a, d * s.a.rs,
+                           d * s.a.cs, b, d * s.rhs.rs, s.rhs.cs, x, d * s.x.rs, s.x.cs, (int)m,
+                           s.n, (T)alpha, (int)s.unit);
     else
-        hipLaunchKernelGGL(trsm_copy_kernel<float>, dim3(g), dim3(256), 0, s.st,
-                           (const float*)s.wtmp, 1, nb, (float*)offset(s.b, r0, 0, es), s.b.rs,
-                           s.b.cs, nb, s.n);
+        hipLaunchKernelGGL((trsm_slab_kernel<T, 4>), grid, block, 0, s.st, a, d * s.a.rs,
+                           d * s.a.cs, b, d * s.rhs.rs, s.rhs.cs, x, d * s.x.rs, s.x.cs, (int)m,
+                           s.n, (T)alpha, (int)s.unit);
     HIP_CHECK(hipGetLastError());
-}
-
-void leaf(const Solve& s, int64_t r0, int64_t nb, double alpha) {
-    if (s.linv && r0 % NB == 0 && s.inv_ok[r0 / NB]) {
-        leaf_by_product(s, r0, nb, alpha);
-        return;
-    }
-    const size_t es = dt_size(s.dt);
-    void* a = offset(s.a, r0, r0, es);
-    void* b = offset(s.b, r0, 0, es);
-    // Two columns per wave: measured faster than one at n = 1024 on MI355X
-    // (each row of the triangle is read once for both columns).
-    if (s.dt == Dt::F64) leaf_t<double, 2>(s, a, b, nb, alpha);
-    else leaf_t<float, 2>(s, a, b, nb, alpha);
 }
 
 // R[dst rows] := beta * R[dst rows] - L_eff[dst rows, src rows] * X[src rows]
@@ -421,15 +452,13 @@ void update(const Solve& s, int64_t dst0, int64_t dstn, int64_t src0, int64_t sr
 }
 
 // X[r0 .. r0+511] = alpha * inv(L_pp) * R[r0 .. r0+511] for an aligned
-// 512-row block whose inverse was composed: one product in place of a
-// leaf, an update and a leaf.
-void leaf2_by_product(const Solve& s, int64_t r0, double alpha) {
+// 512-row block: one product with its inverse.
+void block_by_product(const Solve& s, int64_t r0, double alpha) {
     const size_t es = dt_size(s.dt);
     GemmDesc d;
     d.dt = s.dt;
-    d.m = 2 * NB; d.n = s.n; d.k = 2 * NB;
-    d.a = s.band ? band_view(s, r0, r0)
-                 : View{ (char*)s.linv2 + (size_t)(r0 / (2 * NB)) * 4 * NB * NB * es, 1, 2 * NB };
+    d.m = PB; d.n = s.n; d.k = PB;
+    d.a = band_view(s, r0, r0);
     d.b = { offset(s.rhs, r0, 0, es), s.rhs.rs, s.rhs.cs };
     d.c = { offset(s.x, r0, 0, es), s.x.rs, s.x.cs };
     d.alpha = alpha;
@@ -438,18 +467,16 @@ void leaf2_by_product(const Solve& s, int64_t r0, double alpha) {
 }
 
 void solve(const Solve& s, int64_t r0, int64_t m, double alpha) {
-    if (s.linv2 && m == 2 * NB && r0 % (2 * NB) == 0 && r0 / (2 * NB) < s.npair) {
-        leaf2_by_product(s, r0, alpha);
+    if (m <= SLAB) {
+        if (s.band && m == PB) block_by_product(s, r0, alpha);
+        else if (s.dt == Dt::F64) slab<double>(s, r0, m, alpha);
+        else slab<float>(s, r0, m, alpha);
         return;
     }
-    if (m <= NB) {
-        leaf(s, r0, m, alpha);
-        return;
-    }
-    // Split into halves rounded to whole leaves.
-    int64_t h = ((m / 2) + NB - 1) / NB * NB;
-    if (h >= m) h = m - NB;
-    const int64_t m1 = h, m2 = m - h;
+    // Halves of whole tiles; with inverted blocks, of whole blocks, the
+    // ragged rest at the end.
+    const int64_t unit = s.band ? PB : 16;
+    const int64_t m1 = (m / 2 + unit - 1) / unit * unit, m2 = m - m1;
     if (s.lower) {
         solve(s, r0, m1, alpha);
         update(s, r0 + m1, m2, r0, m1, alpha);
@@ -461,58 +488,15 @@ void solve(const Solve& s, int64_t r0, int64_t m, double alpha) {
     }
 }
 
-// Inverses of the aligned 512-row diagonal blocks from the 256-row inverses
-// at linv (ld NB): inv([[L11, 0], [L21, L22]]) =
+// Inverses of 2b rows from those of b rows in the band store (b = 64, 128,
+// 256), for every aligned pair: inv([[L11, 0], [L21, L22]]) =
 // [[inv(L11), 0], [-inv(L22) L21 inv(L11), inv(L22)]] for a lower triangle,
 // inv([[U11, U12], [0, U22]]) = [[inv(U11), -inv(U11) U12 inv(U22)],
-// [0, inv(U22)]] for an upper one. Two strided launches of 256^3 products
-// cover every pair. The blocks passed the dominance check, so the inverse
-// applied first has condition number at most 48 and the product form of
-// the 512-row leaf loses at most that factor against the leaf, update, leaf
-// sequence it replaces.
-void compose_pairs(Solve& s, const void* linv, int64_t rows) {
-    const size_t es = dt_size(s.dt);
-    const int64_t npair = rows / (2 * NB);
-    if (npair < 1) return;
-    void* linv2 = workspace((size_t)npair * 4 * NB * NB * es, 18);
-    void* t = workspace((size_t)npair * NB * NB * es, 19);
-    const int64_t total = npair * 4 * NB * NB;
-    const unsigned g = (unsigned)std::min<int64_t>((total + 255) / 256, 8192);
-    const int upper = s.lower ? 0 : 1;
-    if (s.dt == Dt::F64)
-        hipLaunchKernelGGL(trsm_assemble_kernel<double>, dim3(g), dim3(256), 0, s.st,
-                           (const double*)linv, (double*)linv2, npair, upper);
-    else
-        hipLaunchKernelGGL(trsm_assemble_kernel<float>, dim3(g), dim3(256), 0, s.st,
-                           (const float*)linv, (float*)linv2, npair, upper);
-    HIP_CHECK(hipGetLastError());
-    const size_t blk = (size_t)NB * NB * es;
-    // Lower: T_p = L21_p * inv(L11_p). Upper: T_p = U12_p * inv(U22_p).
-    GemmDesc d;
-    d.dt = s.dt;
-    d.m = NB; d.n = NB; d.k = NB;
-    d.a = upper ? View{ offset(s.a, 0, NB, es), s.a.rs, s.a.cs }
-                : View{ offset(s.a, NB, 0, es), s.a.rs, s.a.cs };
-    d.b = { (char*)const_cast<void*>(linv) + (upper ? blk : 0), 1, NB };
-    d.c = { t, 1, NB };
-    d.alpha = 1.0;
-    d.beta = 0.0;
-    gemm_strided_run(d, (int)npair, 2 * NB * (s.a.rs + s.a.cs), 2 * NB * NB, NB * NB, s.st);
-    // Lower: -inv(L22_p) * T_p into the bottom-left quarter of pair p.
-    // Upper: -inv(U11_p) * T_p into the top-right quarter.
-    d.a = { (char*)const_cast<void*>(linv) + (upper ? 0 : blk), 1, NB };
-    d.b = { t, 1, NB };
-    d.c = { (char*)linv2 + (upper ? (size_t)NB * 2 * NB * es : (size_t)NB * es), 1, 2 * NB };
-    d.alpha = -1.0;
-    gemm_strided_run(d, (int)npair, 2 * NB * NB, NB * NB, 4 * NB * NB, s.st);
-    s.linv2 = linv2;
-    s.npair = npair;
-}
-
-// The same composition in the band store, for every aligned pair of b-row
-// inverses: 2b-row inverses from b-row ones (b = 64, 128, 256). Both
-// products are one strided launch over the pairs: in the band the pairs are
-// 2b * BAND_LD elements apart, in the triangle 2b (rs + cs).
+// [0, inv(U22)]] for an upper one. Both products are one strided launch over
+// the pairs: in the band the pairs are 2b * BAND_LD elements apart, in the
+// triangle 2b (rs + cs). The blocks passed the dominance check, so the
+// inverse applied first has condition number at most 48 and the product form
+// loses at most that factor against the substitution it replaces.
 void compose_band(const Solve& s, int64_t rows, int64_t b) {
     const size_t es = dt_size(s.dt);
     const int64_t npair = rows / (2 * b);
@@ -560,40 +544,35 @@ void trsm_run(Dt dt, side_t side, uplo_t uplo, trans_t trans, diag_t diag, int64
     s.dt = dt;
     s.unit = (diag == BLIS_UNIT_DIAG);
     s.st = st;
+    View bv;          // B'(i,j) = bv.ptr[i*bv.rs + j*bv.cs]
     int64_t rows;
     if (side == BLIS_LEFT) {
         // L_eff = op(A).
         s.a = { a.ptr, t ? a.cs : a.rs, t ? a.rs : a.cs };
         s.lower = t ? !lower : lower;
-        s.b = b;
+        bv = b;
         s.n = n;
         rows = m;
     } else {
         // X op(A) = alpha B  <=>  op(A)^T X^T = alpha B^T.
         s.a = { a.ptr, t ? a.rs : a.cs, t ? a.cs : a.rs };
         s.lower = t ? lower : !lower;
-        s.b = { b.ptr, b.cs, b.rs };
+        bv = { b.ptr, b.cs, b.rs };
         s.n = m;
         rows = n;
     }
-    s.rhs = s.b;
-    s.x = s.b;
-    // Many leaves over many columns: check the diagonal blocks, invert them
-    // all in one launch, and solve the blocks that passed by GEMM products.
-    std::vector<int> ok;
-    if (rows > NB && s.n >= TRSM_INV_MIN_N) {
+    s.rhs = bv;
+    s.x = bv;
+    // A large triangle over many columns: check its whole 512-row diagonal
+    // blocks for dominance while they are inverted, and solve them by GEMM
+    // products when all pass. The composition multiplies blocks of the
+    // triangle in place, which needs a unit stride.
+    const int64_t whole = rows / PB * PB;
+    if (rows >= TRSM_INV_MIN_ROWS && s.n >= TRSM_INV_MIN_N && (s.a.rs == 1 || s.a.cs == 1)) {
         const size_t es = dt_size(dt);
-        const int nblk = (int)((rows + NB - 1) / NB);
-        const int64_t last = rows - (int64_t)(nblk - 1) * NB;
+        const int nblk = (int)(whole / NB);
         int* d_ok = (int*)workspace(sizeof(int) * nblk, 15);
-        // Whole 512-row blocks and a unit-stride triangle: the inverses are
-        // built in the band store from 64-row leaves; otherwise 256-row
-        // leaves are inverted directly (ragged last block).
-        const bool use_band = rows % (2 * NB) == 0 && (s.a.rs == 1 || s.a.cs == 1);
-        const int64_t total = (int64_t)nblk * NB * NB;
-        void* linv = use_band ? workspace((size_t)(rows + 1) * BAND_LD * es, 13)
-                              : workspace((size_t)total * es, 13);
-        const int64_t a_step = NB * (s.a.rs + s.a.cs);
+        void* band = workspace((size_t)(whole + 1) * BAND_LD * es, 13);
         // The check runs on a side stream, beside the inversion on the main
         // stream; only the host reads its flags (pinned memory, one wait).
         hipStream_t cs = check_stream();
@@ -605,78 +584,54 @@ void trsm_run(Dt dt, side_t side, uplo_t uplo, trans_t trans, diag_t diag, int64
         if (dt == Dt::F64) {
             if (s.lower)
                 hipLaunchKernelGGL((trsm_diag_check_kernel<double, true>), dim3(nblk), dim3(NB), 0,
-                                   cs, (const double*)s.a.ptr, s.a.rs, s.a.cs, rows, (int)s.unit,
+                                   cs, (const double*)s.a.ptr, s.a.rs, s.a.cs, whole, (int)s.unit,
                                    d_ok);
             else
                 hipLaunchKernelGGL((trsm_diag_check_kernel<double, false>), dim3(nblk), dim3(NB),
-                                   0, cs, (const double*)s.a.ptr, s.a.rs, s.a.cs, rows,
+                                   0, cs, (const double*)s.a.ptr, s.a.rs, s.a.cs, whole,
                                    (int)s.unit, d_ok);
         } else {
             if (s.lower)
                 hipLaunchKernelGGL((trsm_diag_check_kernel<float, true>), dim3(nblk), dim3(NB), 0,
-                                   cs, (const float*)s.a.ptr, s.a.rs, s.a.cs, rows, (int)s.unit,
+                                   cs, (const float*)s.a.ptr, s.a.rs, s.a.cs, whole, (int)s.unit,
                                    d_ok);
             else
                 hipLaunchKernelGGL((trsm_diag_check_kernel<float, false>), dim3(nblk), dim3(NB), 0,
-                                   cs, (const float*)s.a.ptr, s.a.rs, s.a.cs, rows, (int)s.unit,
+                                   cs, (const float*)s.a.ptr, s.a.rs, s.a.cs, whole, (int)s.unit,
                                    d_ok);
         }
         HIP_CHECK(hipGetLastError());
-        ok.assign(nblk, 0);
+        std::vector<int> ok(nblk, 0);
         static int* pinned = nullptr;
         constexpr int PINNED_FLAGS = 1 << 16;
         if (!pinned) HIP_CHECK(hipHostMalloc((void**)&pinned, sizeof(int) * PINNED_FLAGS));
         int* flags = nblk <= PINNED_FLAGS ? pinned : ok.data();
         HIP_CHECK(hipMemcpyAsync(flags, d_ok, sizeof(int) * nblk, hipMemcpyDeviceToHost, cs));
         HIP_CHECK(hipEventRecord(checked, cs));
-        // The inverses: leaves whose right-hand side is the identity, built
-        // in the kernel, skipping each column's zero blocks.
-        if (use_band) {
-            // 64-row leaves straight into the band (each also zeroes its
-            // columns of the 512-row block on the far side of the
-            // diagonal), then 128- and 256-row inverses by composition.
-            constexpr int64_t LB = 64;
-            s.band = linv;
-            const View b0 = band_view(s, 0, 0);
-            const int count = (int)(rows / LB);
-            const int zgroup = (int)(2 * NB / LB);
-            if (dt == Dt::F64)
-                leaf_launch<double, INV_CPW, true>(s.lower, s.unit, s.a.ptr, s.a.rs, s.a.cs,
-                                                   b0.ptr, 1, b0.cs, LB, LB, 1.0, count,
-                                                   LB * (s.a.rs + s.a.cs), LB * BAND_LD, LB, st,
-                                                   zgroup);
-            else
-                leaf_launch<float, INV_CPW, true>(s.lower, s.unit, s.a.ptr, s.a.rs, s.a.cs,
-                                                  b0.ptr, 1, b0.cs, LB, LB, 1.0, count,
-                                                  LB * (s.a.rs + s.a.cs), LB * BAND_LD, LB, st,
-                                                  zgroup);
-            compose_band(s, rows, LB);
-            compose_band(s, rows, 2 * LB);
-            // The 512-row inverses are used only when every block passes;
-            // they are composed before the wait for the check anyway, so
-            // that the GPU stays busy while the host reads the flags.
-            compose_band(s, rows, NB);
-        } else if (dt == Dt::F64) {
-            leaf_launch<double, INV_CPW, true>(s.lower, s.unit, s.a.ptr, s.a.rs, s.a.cs, linv, 1,
-                                               NB, NB, NB, 1.0, nblk, a_step, (int64_t)NB * NB,
-                                               last, st);
-        } else {
-            leaf_launch<float, INV_CPW, true>(s.lower, s.unit, s.a.ptr, s.a.rs, s.a.cs, linv, 1,
-                                              NB, NB, NB, 1.0, nblk, a_step, (int64_t)NB * NB,
-                                              last, st);
-        }
+        // 64-row inverses straight into the band, then 128-, 256- and 512-row
+        // ones by composition, all before the wait for the check, so that the
+        // GPU stays busy while the host reads the flags.
+        s.band = band;
+        if (dt == Dt::F64) inverse_launch<double>(s, (int)(whole / LB));
+        else inverse_launch<float>(s, (int)(whole / LB));
+        compose_band(s, whole, LB);
+        compose_band(s, whole, 2 * LB);
+        compose_band(s, whole, 4 * LB);
         HIP_CHECK(hipEventSynchronize(checked));
         HIP_CHECK(hipEventDestroy(checked));
         HIP_CHECK(hipEventDestroy(ready));
-        if (flags != ok.data()) std::copy(flags, flags + nblk, ok.begin());
-        s.linv = linv;
-        s.inv_ok = ok.data();
-        auto copy = [&](View src, View dst) {
-            if (src.rs == 1 && dst.rs == 1 && src.cs == rows && dst.cs == rows) {
-                // Both column-stored without padding: one contiguous span,
-                // which the runtime's copy moves at about 5.5 TB/s against
-                // 2.3 TB/s for the tiled kernel (32 MB: 12 against 28 us).
-                HIP_CHECK(hipMemcpyAsync(dst.ptr, src.ptr, (size_t)rows * s.n * es,
+        bool all = true;
+        for (int i = 0; i < nblk; ++i) all = all && flags[i];
+        if (all) {
+            // The right-hand side is updated in place and X is built in a
+            // separate column-major buffer, copied over B once at the end.
+            s.x = { workspace((size_t)rows * s.n * es, 16), 1, rows };
+            solve(s, 0, rows, alpha);
+            if (bv.rs == 1 && bv.cs == rows) {
+                // Column-stored without padding: one contiguous span, which
+                // the runtime's copy moves at about 5.5 TB/s against 2.3 TB/s
+                // for the tiled kernel (32 MB: 12 against 28 us).
+                HIP_CHECK(hipMemcpyAsync(bv.ptr, s.x.ptr, (size_t)rows * s.n * es,
                                          hipMemcpyDeviceToDevice, st));
                 return;
             }
@@ -684,39 +639,16 @@ void trsm_run(Dt dt, side_t side, uplo_t uplo, trans_t trans, diag_t diag, int64
             const unsigned gc = (unsigned)std::max<int64_t>(1, std::min<int64_t>(tiles, 8192));
             if (dt == Dt::F64)
                 hipLaunchKernelGGL(trsm_copy_kernel<double>, dim3(gc), dim3(256), 0, st,
-                                   (const double*)src.ptr, src.rs, src.cs, (double*)dst.ptr,
-                                   dst.rs, dst.cs, rows, s.n);
+                                   (const double*)s.x.ptr, s.x.rs, s.x.cs, (double*)bv.ptr, bv.rs,
+                                   bv.cs, rows, s.n);
             else
                 hipLaunchKernelGGL(trsm_copy_kernel<float>, dim3(gc), dim3(256), 0, st,
-                                   (const float*)src.ptr, src.rs, src.cs, (float*)dst.ptr,
-                                   dst.rs, dst.cs, rows, s.n);
+                                   (const float*)s.x.ptr, s.x.rs, s.x.cs, (float*)bv.ptr, bv.rs,
+                                   bv.cs, rows, s.n);
             HIP_CHECK(hipGetLastError());
-        };
-        bool all = true;
-        for (int v : ok) all = all && v;
-        if (all) {
-            // Every block by product: the right-hand side is updated in place
-            // and X is built in a separate column-major buffer, copied over B
-            // once at the end (no per-leaf staging copies).
-            s.x = { workspace((size_t)rows * s.n * es, 16), 1, rows };
-            s.separate = true;
-            // The composition multiplies off-diagonal blocks of the triangle
-            // in place, which needs a unit stride; a general-stride triangle
-            // keeps 256-row leaves with updates between them (the update
-            // GEMMs pack it).
-            if (use_band) {
-                s.linv2 = linv;
-                s.npair = rows / (2 * NB);
-            } else if (rows >= 2 * NB && (s.a.rs == 1 || s.a.cs == 1)) {
-                compose_pairs(s, linv, rows);
-            }
-            solve(s, 0, rows, alpha);
-            copy(s.x, s.b);
             return;
         }
-        // Some blocks by substitution: in place, product leaves through
-        // staging.
-        s.wtmp = workspace((size_t)NB * s.n * es, 14);
+        s.band = nullptr;
     }
     solve(s, 0, rows, alpha);
 }
