@@ -43,6 +43,13 @@ struct BatchDesc {
     int32_t     tiles_m32;   // tiles along m at 32 (wave-tile mode)
 };
 
+// A pointer out of a descriptor, told to be in global memory: as a generic
+// one it would be read and written with flat instructions, which also wait on
+// the LDS counter.
+template <typename T> __device__ inline T* global_ptr(void* p) {
+    return (T*)(__attribute__((address_space(1))) T*)(uintptr_t)p;
+}
+
 struct WorkItem {
     int32_t prob;
     int32_t tile;
@@ -60,10 +67,14 @@ template <> struct BatchTiles<float> {
     using Small = TileCfg<float, 32, 32, 32, 16, 16>;
 };
 
-// One persistent kernel per (tile shape, A layout, B layout) variant: each
-// instantiation holds only its own tile code, so its register count (and
-// with it the number of resident workgroups) is that of the plain GEMM
-// kernel with the same tile, and its code fits the instruction cache.
+// One persistent kernel per tile shape ("variant"): each instantiation holds
+// only its own tile code, so its register count (and with it the number of
+// resident workgroups) is that of the plain GEMM kernel with the same tile,
+// and its code fits the instruction cache. The operands' layouts are read from
+// the descriptor: with a kernel per layout too, eight kernels ran one after
+// another, each with a tail of its own. 10,000 FP64 problems (mode 8) take
+// the same 1.52 ms either way; 3,000 problems of dims up to 150 take 70 us in
+// place of 105, and 1,000 FP32 ones of dims up to 300 49 us in place of 110.
 // Work items of one variant, split into one list per XCD: list x is
 // items[off[x] .. off[x+1]). Workgroups are dispatched round-robin over the
 // 8 XCDs, so workgroup b (on XCD b % 8) walks list b % 8; every tile of a
@@ -89,9 +100,12 @@ struct XcdSegs {
 // Modes other than 4 can differ between the variants of one plan.
 constexpr int NMODE = 9;
 constexpr int WAVE_MODE = 4;
-// Mode used until the autotuner runs: the one measured fastest on uneven
-// batches of 10,000 problems (dims log-uniform in [8, 512]), for both types.
-constexpr int default_mode(Dt) { return 8; }
+// Mode a variant uses until the autotuner runs: the one measured fastest on
+// uneven batches of 10,000 problems (dims log-uniform in [8, 512]). Modes
+// 0 / 5 / 6 / 7 / 8, in us: FP64 64 x 64 tiles 1386 / 1190 / 1161 / 1125 /
+// 1128, 32 x 32 tiles 421 / 392 / 409 / 407 / 407; FP32 64 x 64 tiles 1058 /
+// 692 / 1014 / 633 / 592, 32 x 32 tiles 258 / 233 / 251 / 230 / 232.
+constexpr int default_mode(Dt dt, int v) { return dt == Dt::F64 && v == 1 ? 5 : 8; }
 // Modes whose kernels are the same as another's: run as, and timed with, it.
 constexpr int mode_kernel(int mode) { return mode == 1 ? 0 : mode == 2 ? 3 : mode; }
 constexpr int mode_pf(int mode) { return (mode == 2 || mode == 3) ? 2 : 1; }
@@ -102,7 +116,7 @@ template <typename T> constexpr bool mode_lds_epi(int mode) {
 }
 template <typename T> constexpr bool mode_c_pf(int mode) { return mode_lds_epi<T>(mode); }
 
-template <typename T, class TL, bool A_K, bool B_K, int MODE>
+template <typename T, class TL, int MODE>
 __global__ __launch_bounds__(TL::NT)
 __attribute__((amdgpu_waves_per_eu(mode_waves(MODE)))) void gemm_batch_kernel(const BatchDesc* __restrict__ descs,
                                                             const WorkItem* __restrict__ items,
@@ -129,14 +143,16 @@ __attribute__((amdgpu_waves_per_eu(mode_waves(MODE)))) void gemm_batch_kernel(co
             dn = descs[wn.prob];
         }
         TileProblem<T> p;
-        p.a = (const T*)d.a; p.b = (const T*)d.b; p.c = (T*)d.c;
+        p.a = (const T*)d.a; p.b = (const T*)d.b; p.c = global_ptr<T>(d.c);
         p.m = d.m; p.n = d.n; p.k = d.k;
         p.lda = d.lda; p.ldb = d.ldb; p.c_si = d.c_si; p.c_sj = d.c_sj;
         p.alpha = (T)d.alpha; p.beta = (T)d.beta;
         p.vec_a = p.vec_b = 0;      // loads go through buffer descriptors
         p.vec_c = d.c_si == 1;
+        p.a_k = d.flags & F_A_K;
+        p.b_k = d.flags & F_B_K;
         const int64_t tm = w.tile % d.tiles_m, tn = w.tile / d.tiles_m;
-        gemm_tile<T, TL, A_K, B_K, true, mode_pf(MODE), mode_lds_epi<T>(MODE),
+        gemm_tile<T, TL, false, false, Loads::RuntimeLayout, mode_pf(MODE), mode_lds_epi<T>(MODE),
                   mode_c_pf<T>(MODE)>(p, tm, tn, smem, sink);
         __syncthreads();
         if (!has_next) break;
@@ -146,10 +162,12 @@ __attribute__((amdgpu_waves_per_eu(mode_waves(MODE)))) void gemm_batch_kernel(co
     }
 }
 
-// Variant v = 4*small + 2*a_k + b_k.
-constexpr int NVARIANT = 8;
-__host__ __device__ inline int variant_of(int32_t flags) {
-    return ((flags & F_SMALL) ? 4 : 0) + ((flags & F_A_K) ? 2 : 0) + ((flags & F_B_K) ? 1 : 0);
+// Variant v: 0 for 64 x 64 tiles, 1 for 32 x 32. The wave mode has a kernel
+// per layout, 2*a_k + b_k.
+constexpr int NVARIANT = 2, NLAYOUT = 4;
+__host__ __device__ inline int variant_of(int32_t flags) { return (flags & F_SMALL) ? 1 : 0; }
+__host__ __device__ inline int layout_of(int32_t flags) {
+    return ((flags & F_A_K) ? 2 : 0) + ((flags & F_B_K) ? 1 : 0);
 }
 
 // The whole batch in one dispatch (every mode but the wave mode). Work
@@ -202,25 +220,21 @@ __attribute__((amdgpu_waves_per_eu(mode_waves(MODE)))) void gemm_batch_dyn_kerne
             dn = descs[wn.prob];
         }
         TileProblem<T> p;
-        p.a = (const T*)d.a; p.b = (const T*)d.b; p.c = (T*)d.c;
+        p.a = (const T*)d.a; p.b = (const T*)d.b; p.c = global_ptr<T>(d.c);
         p.m = d.m; p.n = d.n; p.k = d.k;
         p.lda = d.lda; p.ldb = d.ldb; p.c_si = d.c_si; p.c_sj = d.c_sj;
         p.alpha = (T)d.alpha; p.beta = (T)d.beta;
         p.vec_a = p.vec_b = 0;      // loads go through buffer descriptors
         p.vec_c = d.c_si == 1;
+        p.a_k = d.flags & F_A_K;
+        p.b_k = d.flags & F_B_K;
         const int64_t tm = w.tile % d.tiles_m, tn = w.tile / d.tiles_m;
         constexpr int PF = mode_pf(MODE);
         constexpr bool LE = mode_lds_epi<T>(MODE), CP = mode_c_pf<T>(MODE);
-        switch (variant_of(d.flags)) {
-        case 0: gemm_tile<T, Big, false, false, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
-        case 1: gemm_tile<T, Big, false, true, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
-        case 2: gemm_tile<T, Big, true, false, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
-        case 3: gemm_tile<T, Big, true, true, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
-        case 4: gemm_tile<T, Small, false, false, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
-        case 5: gemm_tile<T, Small, false, true, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
-        case 6: gemm_tile<T, Small, true, false, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
-        default: gemm_tile<T, Small, true, true, true, PF, LE, CP>(p, tm, tn, smem, sink); break;
-        }
+        if (d.flags & F_SMALL)
+            gemm_tile<T, Small, false, false, Loads::RuntimeLayout, PF, LE, CP>(p, tm, tn, smem, sink);
+        else
+            gemm_tile<T, Big, false, false, Loads::RuntimeLayout, PF, LE, CP>(p, tm, tn, smem, sink);
         if (threadIdx.x == 0) shared_idx[0] = nn;
         __syncthreads();   // smem free for the next tile; nn visible
         cur = nxt;
@@ -339,14 +353,8 @@ inline const void* variant_fn(int v) {
                                           typename BatchTiles<T>::Big>::type;
     using Small = typename BatchTiles<T>::Small;
     switch (v) {
-    case 0: return (const void*)&gemm_batch_kernel<T, Big, false, false, MODE>;
-    case 1: return (const void*)&gemm_batch_kernel<T, Big, false, true, MODE>;
-    case 2: return (const void*)&gemm_batch_kernel<T, Big, true, false, MODE>;
-    case 3: return (const void*)&gemm_batch_kernel<T, Big, true, true, MODE>;
-    case 4: return (const void*)&gemm_batch_kernel<T, Small, false, false, MODE>;
-    case 5: return (const void*)&gemm_batch_kernel<T, Small, false, true, MODE>;
-    case 6: return (const void*)&gemm_batch_kernel<T, Small, true, false, MODE>;
-    case 7: return (const void*)&gemm_batch_kernel<T, Small, true, true, MODE>;
+    case 0: return (const void*)&gemm_batch_kernel<T, Big, MODE>;
+    case 1: return (const void*)&gemm_batch_kernel<T, Small, MODE>;
     }
     abort_with(BLIS_INVALID_UKR_ID, "batch: variant");
     return nullptr;
@@ -354,9 +362,9 @@ inline const void* variant_fn(int v) {
 
 template <typename T>
 inline void variant_info(int mode, int v, const void*& fn, int& threads) {
-    threads = (v < 4) ? BatchTiles<T>::Big::NT : BatchTiles<T>::Small::NT;
+    threads = v == 0 ? BatchTiles<T>::Big::NT : BatchTiles<T>::Small::NT;
     if (mode == WAVE_MODE) {
-        // v = 2*a_k + b_k
+        // v is the layout
         threads = 256;
         switch (v) {
         case 0: fn = (const void*)&gemm_batch_wave_kernel<T, false, false>; return;
@@ -431,9 +439,9 @@ struct BatchPlan {
     WorkItem* d_items = nullptr;
     int nitems = 0;
     XcdSegs seg[NVARIANT] = {};       // per variant: absolute item offsets per XCD list
-    int grid[NMODE][NVARIANT] = {};   // persistent grid per kernel mode and variant
+    int grid[NMODE][NLAYOUT] = {};    // persistent grid per kernel mode and variant (layout)
     WorkItem* d_witems = nullptr;     // wave-tile mode: 32 x 32 tiles of every problem
-    XcdSegs wseg[4] = {};             // per layout variant (2*a_k + b_k)
+    XcdSegs wseg[NLAYOUT] = {};       // per layout
     int mode = 0;                     // kernel mode used by execute
     int vmode[NVARIANT] = {};         // per-variant kernel mode (mode != WAVE_MODE)
     // Single dispatch (gemm_batch_dyn_kernel): every variant's items in one
@@ -597,7 +605,7 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
         for (size_t pi = 0; pi < descs.size(); ++pi) {
             const BatchDesc& d = descs[pi];
             const int64_t t = (int64_t)d.tiles_m32 * ((d.n + 31) / 32);
-            const int lv = variant_of(d.flags) & 3;
+            const int lv = layout_of(d.flags);
             for (int64_t ti = 0; ti < t; ++ti) {
                 witems.push_back(WorkItem{(int32_t)pi, (int32_t)ti});
                 wk.push_back(d.k);
@@ -697,9 +705,8 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
     // kernels), a multiple of the XCD count, and no more per XCD than its
     // longest list.
     for (int mode = 0; mode < NMODE; ++mode)
-        for (int v = 0; v < NVARIANT; ++v) {
+        for (int v = 0; v < (mode == WAVE_MODE ? NLAYOUT : NVARIANT); ++v) {
             const bool wavem = mode == WAVE_MODE;
-            if (wavem && v >= 4) continue;
             const XcdSegs& sg = wavem ? plan->wseg[v] : plan->seg[v];
             int longest = 0;
             for (int x = 0; x < NXCD; ++x) longest = std::max(longest, sg.off[x + 1] - sg.off[x]);
@@ -715,8 +722,8 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
             const int slots = std::max(1, std::min(longest, cu_count() * per_cu / NXCD));
             plan->grid[mode][v] = slots * NXCD;
         }
-    plan->mode = default_mode(dt);
-    for (int v = 0; v < NVARIANT; ++v) plan->vmode[v] = plan->mode;
+    plan->mode = default_mode(dt, 0);
+    for (int v = 0; v < NVARIANT; ++v) plan->vmode[v] = default_mode(dt, v);
     plan->ndesc = (int)descs.size();
     plan->c_offs.resize(descs.size());
     for (size_t i = 0; i < descs.size(); ++i) {
@@ -757,7 +764,7 @@ static void plan_launch(const BatchPlan* plan, hipStream_t st, bool with_fallbac
     if (plan->dyn && plan->mode != WAVE_MODE)
         launch_dyn(plan, plan->mode, st);
     else
-        for (int v = 0; v < NVARIANT; ++v)
+        for (int v = 0; v < (plan->mode == WAVE_MODE ? NLAYOUT : NVARIANT); ++v)
             launch_variant(plan, plan->mode == WAVE_MODE ? WAVE_MODE : plan->vmode[v], v, st);
     if (!with_fallback) return;
     for (const BatchProblem& q : plan->fallback) {
@@ -1016,7 +1023,7 @@ static void plan_tune(BatchPlan* plan, int reps) {
     float vbest_ms[NVARIANT];
     float sum_ms = 0.f;
     for (int v = 0; v < NVARIANT; ++v) {
-        vbest[v] = default_mode(plan->dt);   // never the wave mode (it spans variants)
+        vbest[v] = default_mode(plan->dt, v);   // never the wave mode (it spans variants)
         vbest_ms[v] = 0.f;
         for (int mode = 0; mode < NMODE; ++mode) {
             if (mode == WAVE_MODE || mode != mode_kernel(mode) || plan->grid[mode][v] == 0) continue;
@@ -1026,10 +1033,10 @@ static void plan_tune(BatchPlan* plan, int reps) {
         sum_ms += vbest_ms[v];
     }
     const float wave_ms = time_ms([&] {
-        for (int v = 0; v < NVARIANT; ++v) launch_variant(plan, WAVE_MODE, v, st);
+        for (int v = 0; v < NLAYOUT; ++v) launch_variant(plan, WAVE_MODE, v, st);
     });
     // The single dispatch in every LDS-tile mode.
-    int dbest = default_mode(plan->dt);
+    int dbest = default_mode(plan->dt, 0);
     float dbest_ms = 0.f;
     for (int mode = 0; mode < NMODE; ++mode) {
         if (mode == WAVE_MODE || mode != mode_kernel(mode) || plan->dgrid[mode] == 0) continue;

@@ -139,6 +139,7 @@ struct TileProblem {
     T        alpha, beta;
     int      vec_a, vec_b;   // 16-byte alignment of A and B (loads without a descriptor)
     int      vec_c;          // c_si == 1: C is stored in vectors
+    int      a_k, b_k;       // layouts, where they are not template parameters
 };
 
 // One operand of a tile, read a k slab at a time. The operand is X_eff,
@@ -264,6 +265,65 @@ struct SlabLoader {
 #pragma unroll
                 for (int e = 0; e < V; ++e) S[(c * V + e) * LD + l] = r[q][e];
             }
+        }
+    }
+};
+
+// The same through a buffer descriptor with the layout decided at run time,
+// for kernels that walk problems of every layout (the batch): the layout only
+// enters a thread's offsets, the slab stride and the LDS store, so it costs a
+// uniform branch around the stores and no registers.
+template <typename T, class TL, int ROWS, int NV>
+struct SlabLoaderRt {
+    using vec_t = typename Mma<T>::vec_t;
+    static constexpr int V = TL::V;
+    static constexpr int LD = ROWS + TL::PAD;
+    static constexpr int CVK = TL::BK / V, CVR = ROWS / V;   // vectors along k, along rows
+    static_assert(TL::NT % CVK == 0 && TL::NT % CVR == 0, "whole lines apart");
+    vec_t r[NV];
+    bool k_contig;
+    const char* base;
+    int64_t left, adv;
+    uint32_t off0, step;
+
+    __device__ inline void init(const T* x, int64_t rows, int64_t K, int64_t ld, int k_contig_,
+                                int64_t row0, int tid) {
+        constexpr int ES = (int)sizeof(T);
+        k_contig = k_contig_ != 0;
+        const uint32_t line = (uint32_t)ld * ES;
+        const int c = k_contig ? tid % CVK : tid % CVR, l = k_contig ? tid / CVK : tid / CVR;
+        off0 = (uint32_t)l * line + (uint32_t)(c * 16);
+        step = (uint32_t)(k_contig ? TL::NT / CVK : TL::NT / CVR) * line;
+        adv = (k_contig ? (int64_t)TL::BK : TL::BK * ld) * ES;
+        base = (const char*)(x + (k_contig ? row0 * ld : row0));
+        left = (k_contig ? (rows - 1 - row0) * ld + K : (K - 1) * ld + (rows - row0)) * ES;
+    }
+
+    __device__ inline void load(int, int) {
+        const uint32_t n = (uint32_t)(left >> 32) != 0 ? 0xFFFFFFFFu : (uint32_t)left;
+        auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)n, 0x00020000);
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+            auto t = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(off0 + q * step), 0, 0);
+            r[q] = __builtin_bit_cast(vec_t, t);
+        }
+        base += adv;
+        left -= adv;
+    }
+
+    __device__ inline void store(T* S, int kext, int tid) {
+        if (k_contig) {
+            const int c = tid % CVK, l = tid / CVK;
+#pragma unroll
+            for (int q = 0; q < NV; ++q)
+#pragma unroll
+                for (int e = 0; e < V; ++e)
+                    S[(c * V + e) * LD + l + q * (TL::NT / CVK)] = c * V + e < kext ? r[q][e] : T(0);
+        } else {
+            const int c = tid % CVR, l = tid / CVR;
+#pragma unroll
+            for (int q = 0; q < NV; ++q)
+                *reinterpret_cast<vec_t*>(S + (l + q * (TL::NT / CVR)) * LD + c * V) = r[q];
         }
     }
 };
@@ -528,7 +588,7 @@ __device__ inline void store_tile_lds(const TileProblem<T>& p,
 
 // Compute one BM x BN tile (tile coordinates tm, tn) of one problem. smem
 // must hold 2*TL::STAGE elements. The caller synchronises before reusing smem.
-// BUF: the operands are read through buffer descriptors (SlabLoader).
+// LOADS: how the operands are read.
 // PF: k slabs whose global loads are in flight while a slab is multiplied
 // (1: one register buffer; 2: two, for tiles that stream their operands
 // from HBM, such as the small problems of a batch).
@@ -552,14 +612,21 @@ __device__ inline void prefetch_c(const TileProblem<T>& p, int64_t m0, int64_t n
     __builtin_amdgcn_global_load_lds((const void*)(p.c + r + c * p.c_sj), (lds_ptr_t)dst, 4, 0, 0);
 }
 
-template <typename T, class TL, bool A_K, bool B_K, bool BUF, int PF, bool LDS_EPI,
+// How a tile routine reads its operands: Guarded and Buffer are SlabLoader,
+// RuntimeLayout is SlabLoaderRt (A_K and B_K are not used then).
+enum class Loads { Guarded, Buffer, RuntimeLayout };
+
+template <typename T, class TL, bool A_K, bool B_K, Loads LOADS, int PF, bool LDS_EPI,
           bool C_PF = false, bool MASK = false>
 __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64_t n0, T* smem,
                                       int* sink = nullptr, CMask cm = CMask{}) {
     static_assert(PF == 1 || PF == 2, "prefetch depth");
     using acc_t = typename Mma<T>::acc_t;
-    using Loader_A = SlabLoader<T, TL, TL::BM, A_K, TL::NVA, BUF>;
-    using Loader_B = SlabLoader<T, TL, TL::BN, B_K, TL::NVB, BUF>;
+    constexpr bool RT = LOADS == Loads::RuntimeLayout, BUF = LOADS == Loads::Buffer;
+    using Loader_A = typename std::conditional<RT, SlabLoaderRt<T, TL, TL::BM, TL::NVA>,
+                                               SlabLoader<T, TL, TL::BM, A_K, TL::NVA, BUF>>::type;
+    using Loader_B = typename std::conditional<RT, SlabLoaderRt<T, TL, TL::BN, TL::NVB>,
+                                               SlabLoader<T, TL, TL::BN, B_K, TL::NVB, BUF>>::type;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int wm = wave % TL::WGM, wn = wave / TL::WGM;
@@ -576,8 +643,8 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
     auto kext = [&](int s) { return s + 1 == nk ? klast : TL::BK; };
     Loader_A al;
     Loader_B bl;
-    al.init(p.a, p.m, p.k, p.lda, p.vec_a, m0, tid);
-    bl.init(p.b, p.n, p.k, p.ldb, p.vec_b, n0, tid);
+    al.init(p.a, p.m, p.k, p.lda, RT ? p.a_k : p.vec_a, m0, tid);
+    bl.init(p.b, p.n, p.k, p.ldb, RT ? p.b_k : p.vec_b, n0, tid);
 
     // k == 0 (a batch problem with k == 0 or alpha == 0) touches neither A
     // nor B.
@@ -709,14 +776,14 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
 // slab before the epilogue (one-slab prefetch depth only), through `sink`
 // (NT ints of LDS nobody reads). MASK: write only the stored region `cm` of
 // a structured C (store_tile_masked).
-template <typename T, class TL, bool A_K, bool B_K, bool BUF, int PF = 1, bool LDS_EPI = false,
+template <typename T, class TL, bool A_K, bool B_K, Loads LOADS, int PF = 1, bool LDS_EPI = false,
           bool C_PF = false, bool MASK = false>
 __device__ inline void gemm_tile(const TileProblem<T>& p, int64_t tm, int64_t tn, T* smem,
                                  int* sink = nullptr, CMask cm = CMask{}) {
     static_assert(!C_PF || PF == 1, "C prefetch is placed for one slab in flight");
     static_assert(!MASK || !LDS_EPI, "masked stores go straight from the accumulators");
     const int64_t m0 = tm * TL::BM, n0 = tn * TL::BN;
-    gemm_tile_impl<T, TL, A_K, B_K, BUF, PF, LDS_EPI, C_PF, MASK>(p, m0, n0, smem, sink, cm);
+    gemm_tile_impl<T, TL, A_K, B_K, LOADS, PF, LDS_EPI, C_PF, MASK>(p, m0, n0, smem, sink, cm);
 }
 
 } // namespace dev

@@ -110,8 +110,8 @@ __attribute__((amdgpu_waves_per_eu(TL::waves_per_eu()))) void gemm_struc_kernel(
     p.a += A_K ? kb : kb * p.lda;
     p.b += B_K ? kb : kb * p.ldb;
     p.k = ke - kb;
-    gemm_tile<T, TL, A_K, B_K, BUF, 1, false, false, MASK>(p, tm, tn, smem, nullptr,
-                                                           CMask{s.cmask, s.cdoff});
+    gemm_tile<T, TL, A_K, B_K, BUF ? Loads::Buffer : Loads::Guarded, 1, false, false, MASK>(
+        p, tm, tn, smem, nullptr, CMask{s.cmask, s.cdoff});
 }
 
 // Dense column-major copy (ld = ldd) of an n x n structured matrix stored

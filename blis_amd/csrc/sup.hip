@@ -32,7 +32,7 @@ __global__ __launch_bounds__(SUP_THREADS) void gemm_sup_kernel(TileProblem<T> p,
     static_assert(TL::NT == SUP_THREADS, "sup tile shape");
     __shared__ T smem[2 * TL::STAGE];
     const int tm = blockIdx.x % grid_m, tn = blockIdx.x / grid_m;
-    gemm_tile<T, TL, A_K, B_K, true, 2>(p, tm, tn, smem);
+    gemm_tile<T, TL, A_K, B_K, Loads::Buffer, 2>(p, tm, tn, smem);
 }
 
 namespace {
