@@ -34,8 +34,8 @@ constexpr int64_t PB = 512;     // rows of a block solved by product
 constexpr int64_t SLAB = 512;   // most rows of a leaf solved by substitution
 // Right-hand sides and rows from which the inverted-diagonal path pays: it
 // spends about 75 us on checking and inverting, lost when a block fails the
-// check. FP64, n = 1024, by substitution and by product (us): 1024 rows 134
-// and 120, 2048 rows 313 and 233, 4096 rows 800 and 581.
+// check. FP64, n = 1024, by substitution and by product (us): 1024 rows 149
+// and 120, 2048 rows 330 and 222, 4096 rows 834 and 559.
 constexpr int64_t TRSM_INV_MIN_N = 512;
 constexpr int64_t TRSM_INV_MIN_ROWS = 3 * PB;
 // Columns per wave when inverting the 64-row blocks: each wave reads the
@@ -108,21 +108,26 @@ __global__ __launch_bounds__(64 * WPB) void trsm_inverse_kernel(const T* __restr
 // that is negative strides) and only its stored triangle is read;
 // B(i, j) = b[i*brs + j*bcs], X(i, j) = x[i*xrs + j*xcs], which may be B.
 //
-// The rows are tiles of 16; wave w keeps tiles w, w + 8, ... of its columns in
-// MFMA accumulators for the whole solve, row 4g + r of a tile in register r
-// of lane group g. (The FP64 accumulator holds D row 4r + g there, so its L
-// operand carries the tile's rows in the order 0, 4, 8, 12, 1, ...) A solved
-// tile's registers then are, as they stand, the four k steps of an MFMA's B
-// operand over columns 4g + r of L. Step q: every wave subtracts L(:, q-1)
+// The rows are tiles of 16; wave w keeps the sums -L X of tiles w, w + 8, ... of
+// its columns in MFMA accumulators for the whole solve, row 4g + r of a tile in
+// register r of lane group g. (The FP64 accumulator holds D row 4r + g there,
+// so its L operand carries the tile's rows in the order 0, 4, 8, 12, 1, ...)
+// The sums start from zero and B joins a row's when the row is solved: it is
+// often much larger than the products, and would set the size of every
+// rounding (FP32 error of X against FP64 at 512 rows, dominant triangle:
+// 3.6e-7 from B, 2.6e-7 from B in two leaves, 3.7e-8 so; 450 rows of a factor
+// that is not dominant: 3.7e-7, 2.8e-7, 1.0e-7). A solved tile's registers then
+// are, as they stand, the four k steps of an MFMA's B operand over columns
+// 4g + r of L. Step q: every wave subtracts L(:, q-1)
 // X(q-1) from its tiles below, four MFMAs each, the owner of tile q first,
 // which then solves it while the others go on. The 16 x 16 diagonal block is
 // solved four rows at a time, which one lane holds for its column: plain
 // substitution inside the lane, each row scaled by the reciprocal of its
 // diagonal element, then four MFMAs subtract those rows from the ones below.
-// The chain of steps is the bound (1.6 us each in FP64, 1.2 in FP32, half of it
+// The chain of steps is the bound (1.8 us each in FP64, 1.3 in FP32, half of it
 // the diagonal block), so what a step needs is fetched ahead: L two steps, the
-// diagonal blocks before the first. 512 rows take 57 us (FP32 39) for up to 4096
-// columns, 256 rows 26 (19); a kernel that substitutes 64 rows at a time across
+// diagonal blocks before the first. 512 rows take 60 us (FP32 42) for 1024
+// columns and 68 (45) for 4096, 256 rows 26 to 28 (18 to 19); a kernel that substitutes 64 rows at a time across
 // a wave took 83 us (68) for 256 rows. Also measured: one column of the tile
 // per lane with the block's elements as LDS broadcasts, 121 us for 512 rows;
 // rows broadcast across lane groups, 81 us; tiles for 1024 rows in one launch,
@@ -152,14 +157,13 @@ __global__ __launch_bounds__(512) void trsm_slab_kernel(const T* __restrict__ a,
         const int t = 8 * j + w;
         acc[j] = acc_t{};
         lp[j] = a + min(t * 16 + lr, m - 1) * ars + 4 * g * acs;
-        if (t < P) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = min(t * 16 + 4 * g + r, m - 1);
-                acc[j][r] = alpha * b[row * brs + colc];
-            }
-        }
     }
+    T bt[4];                                       // B of the wave's next tile to solve
+    auto load_b = [&](int t) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bt[r] = b[min(t * 16 + 4 * g + r, m - 1) * brs + colc];
+    };
+    load_b(w);
     T l[2][SLOTS][4];
     auto load_l = [&](auto buf, int p) {           // L(t, p) of the wave's tiles t > p
         const int64_t off = (int64_t)p * 16 * acs;
@@ -233,10 +237,10 @@ __global__ __launch_bounds__(512) void trsm_slab_kernel(const T* __restrict__ a,
             T x[4] = {};                           // -X, rows 4g + r
             auto rows = [&](auto sub) {            // rows 4s .. 4s + 3, held by lane group s
                 constexpr int s = decltype(sub)::value;
-                const T x0 = v[0] * i0;
-                const T x1 = (v[1] - l10 * x0) * i1;
-                const T x2 = (v[2] - l20 * x0 - l21 * x1) * i2;
-                const T x3 = (v[3] - l30 * x0 - l31 * x1 - l32 * x2) * i3;
+                const T x0 = fma(alpha, bt[0], v[0]) * i0;
+                const T x1 = fma(alpha, bt[1], v[1] - l10 * x0) * i1;
+                const T x2 = fma(alpha, bt[2], v[2] - l20 * x0 - l21 * x1) * i2;
+                const T x3 = fma(alpha, bt[3], v[3] - l30 * x0 - l31 * x1 - l32 * x2) * i3;
                 // Zeros everywhere else, in both operands and in what is kept:
                 // an Inf of these rows or of L must not reach a row through a
                 // product that substitution does not form.
@@ -255,6 +259,7 @@ __global__ __launch_bounds__(512) void trsm_slab_kernel(const T* __restrict__ a,
             rows(std::integral_constant<int, 3>{});
 #pragma unroll
             for (int k = 0; k < 4; ++k) xb[B][k * 64 + lane] = x[k];
+            if (q + 8 < P) load_b(q + 8);
         }
         if (q > 0) {
 #pragma unroll
