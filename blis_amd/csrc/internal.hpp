@@ -72,7 +72,9 @@ constexpr int WS_SLOTS = 32;
 BLIS_AMD_HIDDEN void*       workspace(size_t bytes, int slot);
 // Split-k partitions of products on stream st: a buffer of its own for each
 // of the last eight streams, so that products running side by side on
-// several streams do not share one. Valid for work enqueued on st now.
+// several streams do not share one. Valid for work enqueued on st now; a
+// buffer handed out while st is captured is never freed, since the graph may
+// be replayed at any time.
 BLIS_AMD_HIDDEN void*       stream_scratch(size_t bytes, hipStream_t st);
 BLIS_AMD_HIDDEN bool        synchronous();   // calls wait for their results
 BLIS_AMD_HIDDEN bool        is_device_pointer(const void* p);

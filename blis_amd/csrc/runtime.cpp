@@ -40,6 +40,7 @@ struct State {
         void* p;
         size_t bytes;
         unsigned long long used;
+        bool captured;      // a graph holds its address: kept until the process ends
     };
     std::vector<StreamScratch> split;
     unsigned long long split_clock = 0;
@@ -136,25 +137,37 @@ void* stream_scratch(size_t bytes, hipStream_t st) {
     constexpr size_t MAX_STREAMS = 8;
     State& s = S();
     std::lock_guard<std::mutex> g(s.ws_mutex);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIP_CHECK(hipStreamIsCapturing(st, &cap));
     auto it = std::find_if(s.split.begin(), s.split.end(),
                            [&](const State::StreamScratch& e) { return e.st == st; });
+    if (it != s.split.end() && it->captured && it->bytes < bytes) {
+        s.split.erase(it);      // stays with the graphs that hold it
+        it = s.split.end();
+    }
     if (it == s.split.end()) {
-        if (s.split.size() >= MAX_STREAMS) {
+        const auto held = std::count_if(s.split.begin(), s.split.end(),
+                                        [](const State::StreamScratch& e) { return e.captured; });
+        if (s.split.size() - (size_t)held >= MAX_STREAMS) {
             // Give back the buffer of the stream that used its own longest
             // ago. Its handle may be gone, so wait for the device.
             auto old = std::min_element(s.split.begin(), s.split.end(),
                                         [](const State::StreamScratch& a,
-                                           const State::StreamScratch& b) { return a.used < b.used; });
+                                           const State::StreamScratch& b) {
+                                            if (a.captured != b.captured) return b.captured;
+                                            return a.used < b.used;
+                                        });
             HIP_CHECK(hipDeviceSynchronize());
             HIP_CHECK(hipFree(old->p));
             s.split.erase(old);
         }
-        s.split.push_back({ st, nullptr, 0, 0 });
+        s.split.push_back({ st, nullptr, 0, 0, false });
         it = s.split.end() - 1;
     }
     it->used = ++s.split_clock;
+    it->captured = it->captured || cap != hipStreamCaptureStatusNone;
     if (it->bytes < bytes) {
-        if (it->p) {
+        if (it->p) {            // no graph holds it
             HIP_CHECK(hipStreamSynchronize(st));
             HIP_CHECK(hipFree(it->p));
             it->p = nullptr;
