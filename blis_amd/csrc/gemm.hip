@@ -47,7 +47,8 @@ __attribute__((amdgpu_waves_per_eu(TL::waves_per_eu()))) void gemm_kernel(TilePr
     }
     int tm, tn;
     tile_coords(blockIdx.x, gridDim.x, g, tm, tn);
-    gemm_tile<T, TL, A_K, B_K, BUF ? Loads::Buffer : Loads::Guarded>(p, tm, tn, smem);
+    gemm_tile<T, TL, A_K, B_K, BUF ? Loads::Buffer : Loads::Guarded, 1, lds_epilogue<TL>()>(
+        p, tm, tn, smem);
 }
 
 // count products at fixed element strides, one per blockIdx.y:
@@ -64,7 +65,8 @@ __attribute__((amdgpu_waves_per_eu(TL::waves_per_eu()))) void gemm_strided_kerne
     p.c += z * sc;
     int tm, tn;
     tile_coords(blockIdx.x, gridDim.x, g, tm, tn);
-    gemm_tile<T, TL, A_K, B_K, BUF ? Loads::Buffer : Loads::Guarded>(p, tm, tn, smem);
+    gemm_tile<T, TL, A_K, B_K, BUF ? Loads::Buffer : Loads::Guarded, 1, lds_epilogue<TL>()>(
+        p, tm, tn, smem);
 }
 
 // C := beta*C + sum_z parts_z, partitions added in ascending z (a fixed

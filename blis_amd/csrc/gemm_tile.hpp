@@ -771,10 +771,22 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
         store_tile<T, TL, false>(p, acc, m0 + wm0, n0 + wn0, lane);
 }
 
-// LDS_EPI: write C through store_tile_lds (the batch kernels) instead of
-// straight from the accumulators. C_PF: prefetch the C tile into L2 one
-// slab before the epilogue (one-slab prefetch depth only), through `sink`
-// (NT ints of LDS nobody reads). MASK: write only the stored region `cm` of
+// Whether a tile of the plain kernels writes C through LDS: when a lane's TM
+// rows are not whole 16-byte vectors (FP32 waves of 32 rows), so that writing
+// from the accumulators would go element by element, and the C tile fits the
+// stages. FP32 8192 x 8192 x 256 on the 64 x 64 tile takes 298 us in place of
+// 376, on 128 x 64 with eight waves 294 in place of 391; 3001 x 2999 x 333 on
+// 64 x 64 64 in place of 81. Vectors from the accumulators are as fast as
+// through LDS (128 x 64 with four waves: 308 and 311 us), and so are the
+// one-row waves of the 32 x 32 tile (389 and 390 us), which keep the shorter
+// path.
+template <class TL> constexpr bool lds_epilogue() {
+    return TL::TM > 1 && TL::TM % TL::V != 0 && TL::BN * (TL::BM + TL::V) <= 2 * TL::STAGE;
+}
+
+// LDS_EPI: write C through store_tile_lds instead of straight from the
+// accumulators. C_PF: prefetch the C tile into L2 one slab before the epilogue
+// (one-slab prefetch depth only), through `sink` (NT ints of LDS nobody reads). MASK: write only the stored region `cm` of
 // a structured C (store_tile_masked).
 template <typename T, class TL, bool A_K, bool B_K, Loads LOADS, int PF = 1, bool LDS_EPI = false,
           bool C_PF = false, bool MASK = false>
