@@ -1,10 +1,10 @@
-// batch.hip — uneven batched GEMM in one persistent launch.
+// batch.hip — uneven batched GEMM in persistent launches.
 //
 // The reference's ?gemm_batch_ (frame/compat/extra/bla_gemm_batch.c:172-241)
 // loops over groups and problems and calls bli_gemm_ex once per problem, so
 // each problem pays the full front-end and thread-fork cost and small
 // problems take the sup path (frame/3/bli_l3_sup.c:37-130). Here the whole
-// batch is one kernel:
+// batch is one kernel per tile size:
 //   * the host turns every problem into a descriptor (operand layout folded
 //     into flags, as the single-GEMM planner does) and every output tile into
 //     a work item (problem index, tile index);
@@ -446,11 +446,9 @@ struct BatchPlan {
     int vmode[NVARIANT] = {};         // per-variant kernel mode (mode != WAVE_MODE)
     // Single dispatch (gemm_batch_dyn_kernel): every variant's items in one
     // list per XCD, the workgroup count per mode, the per-XCD counters. Off
-    // until the autotuner picks it: on the 10,000-problem batch (dims
-    // log-uniform in [8, 512]) the kernel holding all eight tile paths
-    // needs more registers (FP64 mode 8: 320 bytes per lane of spills
-    // against 20-64 for the per-variant kernels) and measured slower
-    // (d 1.83 ms at best against 1.74 ms, s 1.24 against 1.03 ms).
+    // until the autotuner picks it: it measured slower (10,000 problems, dims
+    // log-uniform in [8, 512]: d 1.51 ms at best, in mode 5, against 1.50, s
+    // 1.12 against 0.83; 3,000 problems of dims up to 150: d 152 us against 68).
     bool dyn = false;
     WorkItem* d_ditems = nullptr;
     XcdSegs dseg = {};

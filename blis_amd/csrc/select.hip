@@ -275,10 +275,10 @@ int selector_pick(Dt dt, int64_t m, int64_t n, int64_t k, bool a_k, bool b_k, bo
         // FP64 products of at least 1024 output tiles of 128 x 128 whose
         // operands all allow 16-byte access keep the heuristic's large
         // tile: the band its rule was tuned on by exhaustive search, where
-        // it measured within 1-2% of the best configuration on shapes with
-        // dimensions divisible by 64 (and 88% of the FP64 peak at 8192^3),
-        // while a network's pick there cost 5% at 8192^3. (The FP32 rule
-        // is no better than the network in that band.)
+        // it measures within 2% of the best configuration in total over the
+        // 354 shapes of the tuning databases there (and 94% of the FP64 peak
+        // at 8192^3), while an earlier network's pick cost 5% at 8192^3. (The
+        // FP32 rule, 21% off there, is no better than the network.)
         const int64_t t128 = ((m + 127) / 128) * ((n + 127) / 128);
         if (dt == Dt::F64 && t128 >= 1024 && va && vb && vc) {
             cfg = heuristic_cfg(dt, m, n, k);

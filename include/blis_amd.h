@@ -96,8 +96,8 @@ int   bli_amd_gemm_batch_plan_autotune( void* plan, int reps );
 void  bli_amd_gemm_batch_plan_set_mode( void* plan, int mode );
 int   bli_amd_gemm_batch_plan_get_mode( void* plan );
 /* on != 0: one dispatch for all tile variants; 0 (the default): one
-   persistent kernel per variant (tile size x operand layouts), one after
-   another. The autotuner chooses between the two. */
+   persistent kernel per variant (tile size), one after another. The
+   autotuner chooses between the two. */
 void  bli_amd_gemm_batch_plan_set_single_dispatch( void* plan, int on );
 int   bli_amd_gemm_batch_plan_get_single_dispatch( void* plan );
 
