@@ -171,3 +171,50 @@ def test_captured_product_takes_one_pass(blis):
     finally:
         blis.bli_amd_gemm_set_config(-1, 8, 1, 1)
         blis.bli_amd_set_stream(None, 1)
+
+
+def test_partitions_in_a_graph_outlive_other_streams(blis):
+    """A graph holds the address of its stream's partitions: the first products
+    of more streams than the library keeps buffers for, and a larger product on
+    the same stream, leave them alone."""
+    say("split rule: partitions held by a graph")
+    g = torch.Generator(device="cuda").manual_seed(7)
+    m, n, k = 128, 96, 8192          # split under capture too
+    a, b = _rand(g, torch.float64, k, m), _rand(g, torch.float64, n, k)
+    out, other = (torch.empty(n, m, dtype=torch.float64, device="cuda") for _ in range(2))
+    big_a, big_b = _rand(g, torch.float64, 4096, 700), _rand(g, torch.float64, 700, 4096)
+    big = torch.empty(700, 700, dtype=torch.float64, device="cuda")
+    one, zero = C.byref(C.c_double(1.0)), C.byref(C.c_double(0.0))
+
+    def call(dst):
+        blis.bli_dgemm(0, 0, m, n, k, one, a.data_ptr(), 1, m, b.data_ptr(), 1, k, zero,
+                       dst.data_ptr(), 1, m)
+
+    st = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    try:
+        blis.bli_amd_set_stream(st.cuda_stream, 0)
+        call(out)
+        torch.cuda.synchronize()
+        want = out.clone()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=st):
+            call(out)
+        for _ in range(3):
+            for s in [torch.cuda.Stream() for _ in range(9)]:
+                blis.bli_amd_set_stream(s.cuda_stream, 0)
+                other.fill_(7.0)
+                torch.cuda.synchronize()
+                call(other)
+                torch.cuda.synchronize()
+                assert torch.equal(other, want)
+            blis.bli_amd_set_stream(st.cuda_stream, 0)
+            blis.bli_dgemm(0, 0, 700, 700, 4096, one, big_a.data_ptr(), 1, 700, big_b.data_ptr(),
+                           1, 4096, zero, big.data_ptr(), 1, 700)
+            out.fill_(7.0)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want)
+    finally:
+        blis.bli_amd_set_stream(None, 1)
