@@ -438,7 +438,7 @@ SplitChoice gemm_choose_split(Dt dt, int64_t m, int64_t n, int64_t k, bool maske
 
 // The same for a call on stream st. A captured product takes one pass unless
 // that is many times slower (m, n <= k/4 and k >= 2048): the graph would keep
-// the address of the partitions, which its replays share with other calls.
+// its partitions for as long as the process lives.
 SplitChoice split_on_stream(Dt dt, int64_t m, int64_t n, int64_t k, bool masked, hipStream_t st) {
     const SplitChoice c = gemm_choose_split(dt, m, n, k, masked);
     if (c.split <= 1 || (!masked && k >= 2048 && 4 * std::max(m, n) <= k)) return c;
@@ -472,18 +472,21 @@ static void launch_plan(Dt dt, Plan& pl, const GemmConfig& cfg, double alpha, do
     GridInfo g{};
     g.group_m = cfg.group_m;
     g.xcd_remap = cfg.xcd_remap;
-    const int tile = cfg.tile >= 0 ? cfg.tile : gemm_default_tile(dt, pl.m, pl.n, pl.k);
+    int tile = cfg.tile >= 0 ? cfg.tile : gemm_default_tile(dt, pl.m, pl.n, pl.k);
     if (tile < 0 || tile >= tile_count(dt)) abort_with(BLIS_INVALID_UKR_ID, "gemm: bad tile");
-    if (dt == Dt::F64 && tile == 13) transpose_k_operands(pl, dt, sc, st);
     // Split-k: each partition a full product into its own m x n slice of
     // scratch, then one reduction into C.
     SplitK sk = split_params(pl.k, cfg.split_k);
-    if (gemm_sup_deep_k(tile, sk.parts, pl.k) && gemm_sup_run(dt, pl, alpha, beta, st)) return;
-    const size_t es = dt_size(dt);
     if (sk.parts > 1) {
-        const size_t bytes = (size_t)sk.parts * pl.m * pl.n * es;
+        const size_t bytes = (size_t)sk.parts * pl.m * pl.n * dt_size(dt);
         sk.ws = sc.base ? sc.take(bytes, 17) : stream_scratch(bytes, st);
+        if (sk.ws == nullptr) {     // no memory for the slices
+            sk = SplitK{};
+            tile = gemm_default_tile(dt, pl.m, pl.n, pl.k);
+        }
     }
+    if (dt == Dt::F64 && tile == 13) transpose_k_operands(pl, dt, sc, st);
+    if (gemm_sup_deep_k(tile, sk.parts, pl.k) && gemm_sup_run(dt, pl, alpha, beta, st)) return;
     if (dt == Dt::F64) {
         launch_tile<double>(tile, make_problem<double>(pl, alpha, beta), pl.a_k, pl.b_k, g, sk, st);
     } else {

@@ -71,10 +71,11 @@ BLIS_AMD_HIDDEN void        sync_if_needed();
 constexpr int WS_SLOTS = 32;
 BLIS_AMD_HIDDEN void*       workspace(size_t bytes, int slot);
 // Split-k partitions of products on stream st: a buffer of its own for each
-// of the last eight streams, so that products running side by side on
-// several streams do not share one. Valid for work enqueued on st now; a
-// buffer handed out while st is captured is never freed, since the graph may
-// be replayed at any time.
+// of the last eight streams and for each stream of a capture, so that products
+// on several streams and in graphs replayed beside them do not share one.
+// Valid for work enqueued on st now, and in a graph for as long as it lives.
+// nullptr when there is no memory, or graphs hold 1 GiB of partitions: the
+// product is then made in one pass.
 BLIS_AMD_HIDDEN void*       stream_scratch(size_t bytes, hipStream_t st);
 BLIS_AMD_HIDDEN bool        synchronous();   // calls wait for their results
 BLIS_AMD_HIDDEN bool        is_device_pointer(const void* p);

@@ -34,16 +34,17 @@ struct State {
     void* ws[WS_SLOTS] = {};
     size_t ws_bytes[WS_SLOTS] = {};
     std::mutex api;
-    // Split-k partitions: one buffer per stream that used them last.
+    // Split-k partitions: one buffer per stream that used them last, and one
+    // per captured stream, which its graph holds (capture: the capture's id).
     struct StreamScratch {
         hipStream_t st;
         void* p;
         size_t bytes;
-        unsigned long long used;
-        bool captured;      // a graph holds its address: kept until the process ends
+        unsigned long long used, capture;
     };
-    std::vector<StreamScratch> split;
+    std::vector<StreamScratch> split, split_graph;
     unsigned long long split_clock = 0;
+    size_t split_graph_bytes = 0;
 };
 
 State& S() {
@@ -133,52 +134,72 @@ void* workspace(size_t bytes, int slot) {
     return s.ws[slot];
 }
 
+// hipMalloc and hipFree are refused while a stream is captured in a mode other
+// than relaxed. The buffers here never become part of a graph's work, so the
+// calling thread may use both: the capture is left alone.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode)); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+static void* try_malloc(size_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
+// Partitions of a product that is being captured. The graph holds the address
+// and may be replayed at any time on any stream, beside eager products and
+// other graphs, so the buffer belongs to this capture of this stream (whose
+// own products run one after another) and is never freed: HIP does not tell
+// when the last executable copy of a graph is gone. What all graphs hold is
+// bounded; past it, products are captured in one pass.
+static void* capture_scratch(State& s, size_t bytes, hipStream_t st, unsigned long long id) {
+    constexpr size_t MAX_BYTES = (size_t)1 << 30, MAX_OPEN = 64;
+    for (const State::StreamScratch& e : s.split_graph)
+        if (e.capture == id && e.st == st && e.bytes >= bytes) return e.p;
+    const size_t want = (bytes + ((size_t)2 << 20) - 1) >> 21 << 21;
+    if (want > MAX_BYTES - s.split_graph_bytes) return nullptr;
+    void* p = try_malloc(want);
+    if (p == nullptr) return nullptr;
+    s.split_graph_bytes += want;
+    // Only captures still open are looked up: the oldest entry goes.
+    if (s.split_graph.size() >= MAX_OPEN) s.split_graph.erase(s.split_graph.begin());
+    s.split_graph.push_back({ st, p, want, 0, id });
+    return p;
+}
+
 void* stream_scratch(size_t bytes, hipStream_t st) {
     constexpr size_t MAX_STREAMS = 8;
     State& s = S();
     std::lock_guard<std::mutex> g(s.ws_mutex);
+    RelaxedCapture relaxed;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    HIP_CHECK(hipStreamIsCapturing(st, &cap));
+    unsigned long long id = 0;
+    HIP_CHECK(hipStreamGetCaptureInfo(st, &cap, &id));
+    if (cap != hipStreamCaptureStatusNone) return capture_scratch(s, bytes, st, id);
     auto it = std::find_if(s.split.begin(), s.split.end(),
                            [&](const State::StreamScratch& e) { return e.st == st; });
-    if (it != s.split.end() && it->captured && it->bytes < bytes) {
-        s.split.erase(it);      // stays with the graphs that hold it
-        it = s.split.end();
+    if (it == s.split.end() && s.split.size() >= MAX_STREAMS) {
+        // Take the buffer of the stream that used its own longest ago.
+        it = std::min_element(s.split.begin(), s.split.end(),
+                              [](const State::StreamScratch& a, const State::StreamScratch& b) {
+                                  return a.used < b.used;
+                              });
+        it->bytes = 0;          // free it below: its last user may still run
+        it->st = st;
     }
-    if (it == s.split.end()) {
-        const auto held = std::count_if(s.split.begin(), s.split.end(),
-                                        [](const State::StreamScratch& e) { return e.captured; });
-        if (s.split.size() - (size_t)held >= MAX_STREAMS) {
-            // Give back the buffer of the stream that used its own longest
-            // ago. Its handle may be gone, so wait for the device.
-            auto old = std::min_element(s.split.begin(), s.split.end(),
-                                        [](const State::StreamScratch& a,
-                                           const State::StreamScratch& b) {
-                                            if (a.captured != b.captured) return b.captured;
-                                            return a.used < b.used;
-                                        });
-            HIP_CHECK(hipDeviceSynchronize());
-            HIP_CHECK(hipFree(old->p));
-            s.split.erase(old);
-        }
-        s.split.push_back({ st, nullptr, 0, 0, false });
-        it = s.split.end() - 1;
-    }
+    if (it == s.split.end()) it = s.split.insert(it, { st, nullptr, 0, 0, 0 });
     it->used = ++s.split_clock;
-    it->captured = it->captured || cap != hipStreamCaptureStatusNone;
     if (it->bytes < bytes) {
-        if (it->p) {            // no graph holds it
-            HIP_CHECK(hipStreamSynchronize(st));
-            HIP_CHECK(hipFree(it->p));
-            it->p = nullptr;
-            it->bytes = 0;
-        }
+        // hipFree waits for the device, and so for every product that uses it.
+        if (it->p) HIP_CHECK(hipFree(it->p));
         // Whole 16 MiB steps: a program's shapes settle after a few calls.
         const size_t want = (bytes + ((size_t)16 << 20) - 1) >> 24 << 24;
-        if (hipMalloc(&it->p, want) != hipSuccess) {
-            (void)hipGetLastError();
-            abort_with(BLIS_MALLOC_RETURNED_NULL, "split-k scratch allocation");
-        }
+        it->p = try_malloc(want);
+        if (it->p == nullptr) abort_with(BLIS_MALLOC_RETURNED_NULL, "split-k scratch allocation");
         it->bytes = want;
     }
     return it->p;

@@ -299,10 +299,10 @@ void gemm_struc_run(const GemmDesc& d, StrucSpec s, hipStream_t st) {
         // product (500 x 500 from k = 30000, FP64: 1637 us in one pass).
         const SplitChoice choice = split_on_stream(d.dt, pl.m, pl.n, pl.k, true, st);
         sk = split_params(pl.k, choice.split);
-        if (sk.parts > 1) {
-            tile = choice.tile;
+        if (sk.parts > 1)
             sk.ws = stream_scratch((size_t)sk.parts * pl.m * pl.n * dt_size(d.dt), st);
-        }
+        if (sk.ws) tile = choice.tile;
+        else sk = SplitK{};
     }
     if (d.dt == Dt::F64)
         launch_struc<double>(tile, make_problem<double>(pl, d.alpha, d.beta), pl.a_k, pl.b_k, g,

@@ -33,6 +33,9 @@ void  bli_amd_synchronize( void );
    beta*C; 1 = one pass, or the built-in rule when tile is -1, which splits
    products of k > 512 whose output has few tiles, by the type and the shape
    alone; under stream capture only those with m, n <= k/4 and k >= 2048).
+   A product that is captured gets partitions that its graph alone uses and
+   that stay allocated until the process ends; once graphs hold 1 GiB of them,
+   or where there is no memory, products are made in one pass.
    Results depend on the k partition only, never on the tile index or on how
    it was chosen. */
 void bli_amd_gemm_set_config( int tile, int group_m, int xcd_remap, int split_k );
