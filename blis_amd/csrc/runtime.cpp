@@ -199,8 +199,7 @@ void* stream_scratch(size_t bytes, hipStream_t st) {
         // Whole 16 MiB steps: a program's shapes settle after a few calls.
         const size_t want = (bytes + ((size_t)16 << 20) - 1) >> 24 << 24;
         it->p = try_malloc(want);
-        if (it->p == nullptr) abort_with(BLIS_MALLOC_RETURNED_NULL, "split-k scratch allocation");
-        it->bytes = want;
+        it->bytes = it->p ? want : 0;
     }
     return it->p;
 }

@@ -128,12 +128,14 @@ int main() {
     if (take(4, 30) == nullptr) fail("a capture after many streams");
     if (take(4, 31) == nullptr) fail("a new stream beside a capture");
     end(30);
-    // No memory: the caller makes one pass.
+    // No memory: the caller makes one pass; later calls ask again.
     memory_left = false;
+    if (take(4, 40) != nullptr) fail("a buffer without memory");
     begin(41, 11);
     if (take(4, 41) != nullptr) fail("a captured buffer without memory");
     end(41);
     memory_left = true;
+    if (take(4, 40) == nullptr) fail("memory is back");
     // What graphs hold is bounded, and so are the streams' buffers.
     bool refused_one = false;
     for (unsigned long long id = 100; id < 200; ++id) {
