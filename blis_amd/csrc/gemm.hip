@@ -355,96 +355,15 @@ int gemm_default_tile(Dt dt, int64_t m, int64_t n, int64_t k) {
     return 4;
 }
 
-// Device time of a product on one tile with `parts` k partitions, in us: a
-// workgroup's launch, prologue and epilogue (fixed); its serial chain of k
-// slabs, each bound by its own latency (slab) while few workgroups share a
-// CU, or by the CU's matrix cores (slab_full per resident workgroup); and
-// for parts > 1 the reduction, one pass over the partitions. `resident` is
-// how many workgroups fit a CU. Fitted to the device times of 300 random
-// GEMM and 100 random SYRK shapes (m, n in [32, 8192], k in [128, 16384], SYRK
-// to 65536, both layouts of each operand) on these tiles with 1 to 64
-// partitions: rms error 20% (FP64) and 16% (FP32) over 10,800 timings.
-struct TileCost {
-    int tile, bm, bn, bk, resident;
-    double slab, slab_full, fixed;
-};
-static const TileCost COST_F64[] = {
-    { 3, 64, 64, 16, 4, 0.794, 0.561, 4.6 },
-    { 4, 32, 32, 16, 8, 0.662, 0.002, 1.7 },
-    { 10, 64, 128, 16, 3, 1.170, 0.988, 5.0 },
-};
-static const TileCost COST_F32[] = {
-    { 1, 128, 64, 32, 3, 1.326, 1.069, 6.0 },
-    { 3, 64, 64, 32, 4, 0.819, 0.609, 6.5 },
-    { 4, 32, 32, 32, 8, 0.457, 0.199, 4.7 },
-};
-
-static double tile_cost(Dt dt, const TileCost& t, int64_t m, int64_t n, int64_t k, int parts,
-                        bool masked) {
-    const int64_t gm = (m + t.bm - 1) / t.bm, gn = (n + t.bn - 1) / t.bn;
-    const int64_t tiles = masked ? (gm * gn + std::max(gm, gn)) / 2 : gm * gn;
-    const int64_t chunk = (k + 63) / 64 > parts ? ((k + 63) / 64 + parts - 1) / parts * 64 : 64;
-    const double slabs = (double)((std::min(chunk, k) + t.bk - 1) / t.bk);
-    const double wgs = (double)(tiles * parts);
-    const int64_t w = (tiles * parts + 255) / 256;
-    const bool fits = w <= t.resident;
-    const double lat = t.slab * (fits ? 1.0 : wgs / (256.0 * t.resident) + 0.3);
-    const double thr = t.slab_full * (fits ? (double)w : wgs / 256.0 + 0.5);
-    double us = t.fixed + slabs * std::max(lat, thr);
-    if (parts > 1) {
-        const double bytes = (2.0 * parts + 2.0) * (double)m * (double)n * (double)dt_size(dt);
-        us += 3.7 + (masked ? 0.6 : 1.0) * bytes / 5.35e6;
-    }
-    return us;
-}
-
-// k partitions of a product and the tile for it when there are several.
-// Products with few output tiles against the 256 CUs walk a long serial k
-// loop on a mostly idle chip; more partitions shorten the loop and cost a
-// pass over the partial outputs. The pair with the least modelled time is
-// taken. It depends on the type and the shape only, so every tile and every
-// operand layout gives the same bits. Over the fitted shapes it is within
-// 6.5% (FP64 GEMM), 4.6% (FP32 GEMM), 3.4% and 13% (SYRK) of the best
-// timing in geometric mean, where splitting only products with
-// m, n <= k/4 and k >= 2048 into 1024-deep partitions left 48%, 32% and,
-// for SYRK without partitions, 214% and 133%. Measured (us, before, now):
-// FP64 256x256x4096 51 / 23, 128x4096x4096 173 / 88, 64x3000x3000 126 / 38,
-// 700x500x1500 51 / 34.
-// One pass stays: up to k = 512 (single calls and batches of such products
-// agree bit for bit), where the partitions would take over 48 MiB, and from
-// 2048 tiles of 64 x 64, which fill the chip by themselves. An output of a
-// single 64 x 64 tile keeps partitions of 1024, up to 64 of them.
-SplitChoice gemm_choose_split(Dt dt, int64_t m, int64_t n, int64_t k, bool masked) {
-    SplitChoice c;
-    if (k <= 512) return c;
-    const int64_t t64 = ((m + 63) / 64) * ((n + 63) / 64);
-    if (t64 >= 2048) return c;
-    if (t64 == 1 && !masked) {
-        if (k >= 2048) c.split = (int)std::min<int64_t>(k / 1024, 64);
-        c.tile = 4;
-        return c;
-    }
-    static const int parts[] = { 1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 32, 40, 48, 64 };
-    const TileCost* tab = dt == Dt::F64 ? COST_F64 : COST_F32;
-    double best = 0.0;
-    for (int q = 0; q < 3; ++q)
-        for (int s : parts) {
-            if (s > 1 && (s * 64 > k || (double)s * m * n * dt_size(dt) > 48.0 * (1 << 20))) break;
-            const double us = tile_cost(dt, tab[q], m, n, k, s, masked);
-            if (best == 0.0 || us < best) { best = us; c.split = s; c.tile = tab[q].tile; }
-        }
-    return c;
-}
-
-// The same for a call on stream st. A captured product takes one pass unless
-// that is many times slower (m, n <= k/4 and k >= 2048): the graph would keep
-// its partitions for as long as the process lives.
+// gemm_choose_split for a call on stream st. A captured product takes one pass
+// unless that is many times slower (m, n <= k/4 and k >= 2048): the graph would
+// keep its partitions for as long as the process lives.
 SplitChoice split_on_stream(Dt dt, int64_t m, int64_t n, int64_t k, bool masked, hipStream_t st) {
     const SplitChoice c = gemm_choose_split(dt, m, n, k, masked);
     if (c.split <= 1 || (!masked && k >= 2048 && 4 * std::max(m, n) <= k)) return c;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     HIP_CHECK(hipStreamIsCapturing(st, &cap));
-    return cap == hipStreamCaptureStatusNone ? c : SplitChoice{};
+    return cap == hipStreamCaptureStatusNone ? c : gemm_choose_split(dt, m, n, k, masked, 1);
 }
 
 // Process-wide override used when a caller passes no configuration

@@ -9,6 +9,7 @@
 #include "internal.hpp"
 #include "gemm_tile.hpp"
 #include "gemm_tiles.hpp"
+#include "gemm_split.hpp"
 
 namespace blis_amd {
 
@@ -154,13 +155,6 @@ struct SplitK {
     int64_t kchunk = 0;
     void* ws = nullptr;
 };
-// The k partitions for a shape, and the tile when there are several (masked:
-// about half of the output tiles are stored).
-struct SplitChoice {
-    int split = 1;
-    int tile = -1;
-};
-SplitChoice gemm_choose_split(Dt dt, int64_t m, int64_t n, int64_t k, bool masked);
 SplitChoice split_on_stream(Dt dt, int64_t m, int64_t n, int64_t k, bool masked, hipStream_t st);
 SplitK split_params(int64_t k, int split);
 // C := beta*C + the sum of the partitions, on the stored region cm of C.

@@ -296,13 +296,20 @@ void gemm_struc_run(const GemmDesc& d, StrucSpec s, hipStream_t st) {
     SplitK sk;
     if (s.cmask) {
         // Few stored tiles over a long k: partitions of k, as for a plain
-        // product (500 x 500 from k = 30000, FP64: 1637 us in one pass).
-        const SplitChoice choice = split_on_stream(d.dt, pl.m, pl.n, pl.k, true, st);
+        // product (500 x 500 from k = 30000, FP64: 1637 us in one pass). The
+        // model's tile also serves one pass: the size heuristic's counts the
+        // tiles that are not stored (FP64 n = 2061, k = 920: 166 us on its 64 x
+        // 128 tiles, 94 on 32 x 32).
+        SplitChoice choice = split_on_stream(d.dt, pl.m, pl.n, pl.k, true, st);
         sk = split_params(pl.k, choice.split);
-        if (sk.parts > 1)
+        if (sk.parts > 1) {
             sk.ws = stream_scratch((size_t)sk.parts * pl.m * pl.n * dt_size(d.dt), st);
-        if (sk.ws) tile = choice.tile;
-        else sk = SplitK{};
+            if (sk.ws == nullptr) {
+                sk = SplitK{};
+                choice = gemm_choose_split(d.dt, pl.m, pl.n, pl.k, true, 1);
+            }
+        }
+        if (choice.tile >= 0) tile = choice.tile;
     }
     if (d.dt == Dt::F64)
         launch_struc<double>(tile, make_problem<double>(pl, d.alpha, d.beta), pl.a_k, pl.b_k, g,

@@ -1,4 +1,5 @@
-"""The buffers of split-k partitions, on the CPU against a model of HIP
+"""Host code of split-k products, compiled and run on the CPU: the rule for the
+partitions (native/split_rule_check.cpp), and their buffers against a model of HIP
 (native/split_scratch_check.cpp): nothing that HIP refuses is called while a
 stream is captured, a graph's buffer is its own and is never freed, the pool is
 bounded, and without memory the product is told to make one pass."""
@@ -12,14 +13,15 @@ import pytest
 from tests.conftest import ROOT
 
 
-def test_partition_buffers_and_capture(tmp_path):
+@pytest.mark.parametrize("check", ["split_scratch_check", "split_rule_check"])
+def test_native(tmp_path, check):
     cxx = shutil.which("g++")
     if cxx is None:
         pytest.skip("no C++ compiler")
     exe = tmp_path / "check"
     subprocess.run([cxx, "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__",
                     "-DBLIS_IS_BUILDING_LIBRARY", "-I/opt/rocm/include", f"-I{ROOT / 'include'}",
-                    str(ROOT / "tests" / "native" / "split_scratch_check.cpp"), "-o", str(exe),
+                    str(ROOT / "tests" / "native" / f"{check}.cpp"), "-o", str(exe),
                     "-lpthread"], check=True)
     p = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
     assert p.returncode == 0 and p.stdout.strip() == "ok", p.stdout + p.stderr
