@@ -94,8 +94,9 @@ inline double split_cost(Dt dt, const SplitModel& sm, const TileCost& t, int64_t
 }
 
 // The pair of partitions (at most `most`) and tile with the least modelled
-// time. The partitions depend on the type and the shape only, so every tile and
-// every operand layout gives the same bits.
+// time. The partitions depend on the type, k and the pair of m and n in either
+// order, so every tile and every operand layout gives the same bits: a product
+// whose C is stored by rows is computed transposed (layout(), gemm_plan.hpp).
 // One pass stays: up to k = 512 (single calls and batches of such products
 // agree bit for bit), where the partitions would take over 48 MiB, and from
 // 2048 stored tiles of 64 x 64, which fill the chip by themselves. An output of
@@ -117,14 +118,21 @@ inline SplitChoice gemm_choose_split(Dt dt, int64_t m, int64_t n, int64_t k, boo
     static const int parts[] = { 1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64 };
     const SplitModel& sm = split_model(dt, masked);
     double best = 0.0;
+    const int64_t hi = std::max(m, n), lo = std::min(m, n);
     for (int s : parts) {
         if (s > 1 && (k <= 512 || s > most || s * 64 > k ||
                       (double)s * m * n * dt_size(dt) > 48.0 * (1 << 20)))
             break;
         for (int q = 0; q < sm.tiles; ++q) {
-            const double us = split_cost(dt, sm, sm.t[q], m, n, k, s, masked);
-            if (best == 0.0 || us < best) { best = us; c.split = s; c.tile = sm.t[q].tile; }
+            const double us = split_cost(dt, sm, sm.t[q], hi, lo, k, s, masked);
+            if (best == 0.0 || us < best) { best = us; c.split = s; }
         }
+    }
+    // The tile for these partitions, from m and n as they are.
+    best = 0.0;
+    for (int q = 0; q < sm.tiles; ++q) {
+        const double us = split_cost(dt, sm, sm.t[q], m, n, k, c.split, masked);
+        if (best == 0.0 || us < best) { best = us; c.tile = sm.t[q].tile; }
     }
     return c;
 }

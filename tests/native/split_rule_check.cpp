@@ -1,7 +1,7 @@
 // split_rule_check.cpp — the rule for k partitions (gemm_split.hpp) over random
-// shapes, on the CPU: no modelled time lies below the card's peak, every tile of
-// a model is the fastest somewhere, and the partitions stay within their
-// limits. Prints "ok", or what went wrong.
+// shapes, on the CPU: no modelled time lies below the card's peak, more than one
+// tile is chosen, the partitions stay within their limits and are the same when
+// m and n change places (C stored by rows or by columns). Prints "ok", or what went wrong.
 #include "../../blis_amd/csrc/gemm_split.hpp"
 
 #include <cmath>
@@ -43,6 +43,8 @@ int main() {
                 if (c.split > 1 && m > 64 &&
                     (double)c.split * m * n * dt_size(dt) > 48.0 * (1 << 20))
                     fail("partitions over 48 MiB", dt, m, n, k, masked);
+                if (gemm_choose_split(dt, n, m, k, masked).split != c.split)
+                    fail("other partitions with m and n exchanged", dt, m, n, k, masked);
                 if (gemm_choose_split(dt, m, n, k, masked, 1).split != 1)
                     fail("one pass asked for", dt, m, n, k, masked);
                 if (c.split > 1) split_tiles.insert(c.tile);

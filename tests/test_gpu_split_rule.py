@@ -72,6 +72,24 @@ def test_gemm_partitions_against_fp64(blis, dt, beta):
 
 
 @pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+def test_same_bits_for_c_by_rows_and_by_columns(blis, dt):
+    """Shapes far from square, whose best tiles differ in the two orders."""
+    g = torch.Generator(device="cuda").manual_seed(8)
+    for m, n, k in [(793, 975, 1670), (165, 1931, 6413), (1931, 165, 6413), (4000, 300, 900),
+                    (130, 700, 577)]:
+        say(f"split rule storage of C {dt} {m}x{n}x{k}")
+        a, b = _rand(g, dt, k, m), _rand(g, dt, n, k)
+        out = []
+        for rows in (False, True):
+            c = torch.empty((m, n) if rows else (n, m), dtype=dt, device="cuda")
+            getattr(blis, f"bli_{_ch(dt)}gemm")(
+                0, 0, m, n, k, C.byref(_ct(dt)(1.0)), a.data_ptr(), 1, m, b.data_ptr(), 1, k,
+                C.byref(_ct(dt)(0.0)), c.data_ptr(), n if rows else 1, 1 if rows else m)
+            out.append(c if rows else c.T)
+        assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
 @pytest.mark.parametrize("uplo", [LOWER, UPPER])
 @pytest.mark.parametrize("trans", [0, 8])
 def test_syrk_partitions_against_fp64(blis, dt, uplo, trans):
