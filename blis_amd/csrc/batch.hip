@@ -503,9 +503,13 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
             else general = true;
             // The kernels read through buffer descriptors; strides that do
             // not allow it run as plain GEMMs.
-            if (!general)
-                general = !buf_ok(d.lda, (flags & F_A_K) ? q.k : q.m, 64, dt) ||
-                          !buf_ok(d.ldb, (flags & F_B_K) ? q.k : q.n, 64, dt);
+            if (!general) {
+                const bool ak = flags & F_A_K, bk = flags & F_B_K;
+                d.lda = ak ? line_ld(d.lda, q.k, q.m) : line_ld(d.lda, q.m, q.k);
+                d.ldb = bk ? line_ld(d.ldb, q.k, q.n) : line_ld(d.ldb, q.n, q.k);
+                general = !buf_ok(d.lda, ak ? q.k : q.m, ak, 64, dt) ||
+                          !buf_ok(d.ldb, bk ? q.k : q.n, bk, 64, dt);
+            }
         } else {
             d.lda = 1; d.ldb = 1;
         }

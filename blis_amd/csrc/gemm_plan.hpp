@@ -68,6 +68,10 @@ struct Scratch {
     }
 };
 
+// The distance between the lines of an operand that has only one (a vector) is
+// never used: the line's own length stands for whatever the caller passed.
+inline int64_t line_ld(int64_t ld, int64_t run, int64_t lines) { return lines == 1 ? run : ld; }
+
 // Storage normalisation without side effects: row-stored C is recast as
 // C^T = B^T A^T, each operand is classified as rows- or k-contiguous, and an
 // operand with neither unit stride is marked for packing into a contiguous
@@ -95,6 +99,8 @@ inline Plan layout(const GemmDesc& d0) {
     if (d.b.rs == 1) { p.b = d.b.ptr; p.ldb = d.b.cs; p.b_k = true; }
     else if (d.b.cs == 1) { p.b = d.b.ptr; p.ldb = d.b.rs; p.b_k = false; }
     else { p.b = nullptr; p.b_src = d.b; p.ldb = d.k; p.b_k = true; p.b_packed = true; }
+    p.lda = p.a_k ? line_ld(p.lda, p.k, p.m) : line_ld(p.lda, p.m, p.k);
+    p.ldb = p.b_k ? line_ld(p.ldb, p.k, p.n) : line_ld(p.ldb, p.n, p.k);
     return p;
 }
 
@@ -118,19 +124,23 @@ inline bool vec_ok(const void* ptr, bool packed, int64_t ld, Dt dt) {
     return (packed || aligned16(ptr)) && ld % V == 0;
 }
 
-// Whether a tile kernel may read an operand (contiguous extent `run`, `ld`
-// between lines, `lines` of them in a slab) through a buffer descriptor:
-// lines that do not overlap or run backwards, so that everything past the
-// last element is past the descriptor's end, and 32-bit byte offsets.
-inline bool buf_ok(int64_t ld, int64_t run, int lines, Dt dt) {
-    return ld >= run && ld <= (((int64_t)1 << 32) - 65536) / (lines * (int64_t)dt_size(dt));
+// Whether a tile kernel may read an operand (`ld` between lines, each `run`
+// elements long, contiguous along k or along its rows, at most `lines` of
+// them in a slab) through a buffer descriptor: everything past k must read as
+// zero or be masked, and byte offsets have 32 bits. Lines along k are past the
+// descriptor's end after the last one, unless they overlap or run backwards; an
+// operand contiguous along k is masked past k, so its lines may overlap
+// (frames of a signal, one hop apart).
+inline bool buf_ok(int64_t ld, int64_t run, bool k_contig, int lines, Dt dt) {
+    return ld >= (k_contig ? 0 : run) &&
+           ld <= (((int64_t)1 << 32) - 65536) / (lines * (int64_t)dt_size(dt));
 }
 
-// The same for both operands of a problem on a bm x bn x bk tile.
+// buf_ok for both operands of a problem on a bm x bn x bk tile.
 template <typename T>
 inline bool buf_problem(const TileProblem<T>& p, bool a_k, bool b_k, int bm, int bn, int bk) {
-    return buf_ok(p.lda, a_k ? p.k : p.m, a_k ? bm : bk, dt_of<T>()) &&
-           buf_ok(p.ldb, b_k ? p.k : p.n, b_k ? bn : bk, dt_of<T>());
+    return buf_ok(p.lda, a_k ? p.k : p.m, a_k, a_k ? bm : bk, dt_of<T>()) &&
+           buf_ok(p.ldb, b_k ? p.k : p.n, b_k, b_k ? bn : bk, dt_of<T>());
 }
 
 template <typename T>

@@ -157,15 +157,15 @@ struct TileProblem {
 // that are never stored; the k positions past K of a K_CONTIG operand, which
 // every output sums over, are zeroed on the way to LDS. Buffer loads need
 // 4-byte alignment only, so odd leading dimensions take the same path. It
-// needs ld >= the contiguous extent and slab offsets below 2^32 bytes
-// (buf_ok in gemm_plan.hpp). Against 64-bit addresses with element loads on
-// edge and unaligned tiles (device time): 1999 x 1501 x 1003 T/N on odd
+// needs lines along k that neither overlap nor run backwards (those along the
+// rows may overlap) and slab offsets below 2^32 bytes (buf_ok in
+// gemm_plan.hpp). Against 64-bit addresses with element loads on edge and
+// unaligned tiles (device time): 1999 x 1501 x 1003 T/N on odd
 // leading dimensions 150 against 170 us, 512^3 12.2 against 13.5 us, the
 // 10,000-problem FP64 batch 1546 against 1739 us (its 64 x 64 kernels no
 // longer spill); 8192^3, all interior, is unchanged.
-// Not BUF (negative, overlapping or very large strides): 16-byte loads for
-// slabs wholly inside an aligned operand, element loads behind bounds checks
-// otherwise.
+// Not BUF (the other strides): 16-byte loads for slabs wholly inside an
+// aligned operand, element loads behind bounds checks otherwise.
 template <typename T, class TL, int ROWS, bool K_CONTIG, int NV, bool BUF>
 struct SlabLoader {
     using vec_t = typename Mma<T>::vec_t;

@@ -105,3 +105,103 @@ def test_leading_dimension_beyond_32_bit_offsets(blis):
                        C.byref(C.c_double(0.0)), c.data_ptr(), 1, m)
         out.append(c)
     assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+def test_vectors_with_any_stride_between_lines(blis, dt):
+    """An operand of one line (k = 1, m = 1 or n = 1) has no second line: the
+    bits do not depend on the stride given for it."""
+    g = torch.Generator(device="cuda").manual_seed(21)
+    ch, ct = ("d", C.c_double) if dt == torch.float64 else ("s", C.c_float)
+    for m, n, k in [(130, 70, 1), (1, 70, 300), (130, 1, 300), (1, 1, 700), (33, 1, 513)]:
+        a, b, c0 = (torch.rand(r, c, generator=g, device="cuda", dtype=dt) * 2 - 1
+                    for r, c in ((m, k), (k, n), (m, n)))
+        base = None
+        for ta, tb in ((0, 0), (1, 0), (0, 1), (1, 1)):
+            for ld in (None, 1, 0, -3, 1 << 33):
+                st, args = [], []
+                for x, t, in ((a, ta), (b, tb)):
+                    x = (x.T if t else x)
+                    buf = x.T.contiguous()               # column-major
+                    st.append(buf)
+                    args.append(ld if ld is not None and x.shape[1] == 1 else x.shape[0])
+                c = c0.T.contiguous()
+                say(f"loads one line {dt} {m}x{n}x{k} ta={ta} tb={tb} ld={ld} {args}")
+                getattr(blis, f"bli_{ch}gemm")(8 * ta, 8 * tb, m, n, k, C.byref(ct(1.25)),
+                                               st[0].data_ptr(), 1, args[0], st[1].data_ptr(), 1,
+                                               args[1], C.byref(ct(0.5)), c.data_ptr(), 1, m)
+                base = c if base is None else base
+                assert torch.equal(c, base)
+
+
+def _frames(x, hop, rows, length):
+    return torch.stack([x[i * hop:i * hop + length] for i in range(rows)])
+
+
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+def test_overlapping_frames(blis, dt):
+    """Rows of A (or columns of B) that are windows of one signal, a hop apart:
+    the bits of the same values stored without overlap."""
+    g = torch.Generator(device="cuda").manual_seed(22)
+    ch, ct = ("d", C.c_double) if dt == torch.float64 else ("s", C.c_float)
+    for rows, cols, k, hop in [(200, 33, 131, 7), (65, 129, 600, 1), (40, 40, 17, 16),
+                               (300, 150, 1000, 0), (129, 64, 515, 257)]:
+        sig = torch.full((hop * (rows - 1) + k + 64,), float("nan"), dtype=dt, device="cuda")
+        sig[:hop * (rows - 1) + k] = torch.rand(hop * (rows - 1) + k, generator=g, device="cuda",
+                                                dtype=dt) * 2 - 1
+        y = torch.rand(cols, k, generator=g, device="cuda", dtype=dt) * 2 - 1
+        tight = _frames(sig, hop, rows, k).contiguous()
+        for side in "ab":
+            out = []
+            for ptr, ld in ((tight.data_ptr(), k), (sig.data_ptr(), hop)):
+                say(f"loads frames {dt} {side} {rows}x{cols}x{k} hop={hop} ld={ld}")
+                m, n = (rows, cols) if side == "a" else (cols, rows)
+                c = torch.zeros(n, m, dtype=dt, device="cuda")
+                fa, fb = (ptr, y.data_ptr()) if side == "a" else (y.data_ptr(), ptr)
+                la, lb = (ld, k) if side == "a" else (k, ld)
+                getattr(blis, f"bli_{ch}gemm")(8, 0, m, n, k, C.byref(ct(1.0)), fa, 1, la, fb, 1,
+                                               lb, C.byref(ct(0.0)), c.data_ptr(), 1, m)
+                out.append(c)
+            assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+def test_batch_plan_takes_vectors_and_frames(blis, dt):
+    """A plan runs them in its own kernels (they have work items), with the bits
+    of single calls."""
+    ch, ct = ("d", C.c_double) if dt == torch.float64 else ("s", C.c_float)
+    g = torch.Generator(device="cuda").manual_seed(23)
+    # (m, n, k, ta, tb, lda, ldb)
+    probs = [(100, 80, 1, 0, 0, 1, 1), (90, 1, 60, 0, 0, 90, 1), (1, 75, 64, 1, 0, 3, 64),
+             (70, 40, 100, 1, 0, 5, 100), (50, 66, 130, 0, 0, 50, 2), (130, 20, 33, 1, 0, 0, 33)]
+    buf = torch.rand(1 << 16, generator=g, device="cuda", dtype=dt) * 2 - 1
+    one, half = ct(1.0), ct(0.5)
+    outs, wants = [], []
+    for m, n, k, ta, tb, lda, ldb in probs:
+        c = torch.rand(n, m, generator=g, device="cuda", dtype=dt)
+        w = c.clone()
+        getattr(blis, f"bli_{ch}gemm")(8 * ta, 8 * tb, m, n, k, C.byref(one), buf.data_ptr(), 1,
+                                       lda, buf[1000:].data_ptr(), 1, ldb, C.byref(half),
+                                       w.data_ptr(), 1, m)
+        outs.append(c)
+        wants.append(w)
+    real = np.float64 if dt == torch.float64 else np.float32
+    col = lambda i, t=np.int64: np.array([p[i] for p in probs], t)
+    ones, cnt = np.ones(len(probs), np.int64), len(probs)
+    arrs = [col(3, np.int32) * 8, col(4, np.int32) * 8, col(0), col(1), col(2),
+            np.full(cnt, 1.0, real), np.full(cnt, buf.data_ptr(), np.int64), ones, col(5),
+            np.full(cnt, buf[1000:].data_ptr(), np.int64), ones, col(6), np.full(cnt, 0.5, real),
+            np.array([c.data_ptr() for c in outs], np.int64), ones, col(0)]
+    arrs = [np.ascontiguousarray(x, x.dtype) for x in arrs]
+    torch.cuda.synchronize()
+    say(f"loads batch plan {dt}")
+    plan = getattr(blis, f"bli_amd_{ch}gemm_batch_plan_create")(
+        *[x.ctypes.data for x in arrs], cnt, ones.ctypes.data)
+    try:
+        assert blis.bli_amd_gemm_batch_plan_work_items(plan) >= cnt
+        blis.bli_amd_gemm_batch_plan_execute(plan, 1)
+        torch.cuda.synchronize()
+        for c, w in zip(outs, wants):
+            assert torch.equal(c, w)
+    finally:
+        blis.bli_amd_gemm_batch_plan_destroy(plan)
