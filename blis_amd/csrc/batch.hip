@@ -28,7 +28,7 @@ using namespace dev;
 namespace detail_batch {
 
 enum : int32_t {
-    F_A_K = 1, F_B_K = 2, F_SMALL = 4
+    F_A_K = 1, F_B_K = 2, F_SMALL = 4, F_GUARDED = 8
 };
 
 struct BatchDesc {
@@ -116,7 +116,8 @@ template <typename T> constexpr bool mode_lds_epi(int mode) {
 }
 template <typename T> constexpr bool mode_c_pf(int mode) { return mode_lds_epi<T>(mode); }
 
-template <typename T, class TL, int MODE>
+// GUARDED: the problems whose strides a buffer descriptor does not take.
+template <typename T, class TL, int MODE, bool GUARDED = false>
 __global__ __launch_bounds__(TL::NT)
 __attribute__((amdgpu_waves_per_eu(mode_waves(MODE)))) void gemm_batch_kernel(const BatchDesc* __restrict__ descs,
                                                             const WorkItem* __restrict__ items,
@@ -152,8 +153,8 @@ __attribute__((amdgpu_waves_per_eu(mode_waves(MODE)))) void gemm_batch_kernel(co
         p.a_k = d.flags & F_A_K;
         p.b_k = d.flags & F_B_K;
         const int64_t tm = w.tile % d.tiles_m, tn = w.tile / d.tiles_m;
-        gemm_tile<T, TL, false, false, Loads::RuntimeLayout, mode_pf(MODE), mode_lds_epi<T>(MODE),
-                  mode_c_pf<T>(MODE)>(p, tm, tn, smem, sink);
+        gemm_tile<T, TL, false, false, GUARDED ? Loads::RuntimeGuarded : Loads::RuntimeLayout,
+                  mode_pf(MODE), mode_lds_epi<T>(MODE), mode_c_pf<T>(MODE)>(p, tm, tn, smem, sink);
         __syncthreads();
         if (!has_next) break;
         it = nit;
@@ -360,6 +361,15 @@ inline const void* variant_fn(int v) {
     return nullptr;
 }
 
+// Problems with strides that descriptors do not take (backwards, overlapping
+// along k, lines far apart): 32 x 32 tiles behind bounds checks, in a launch of
+// its own in every mode. 100 problems of dims up to 128 whose A runs backwards:
+// FP64 10 us, one plain product after another 574.
+template <typename T>
+inline const void* guarded_fn() {
+    return (const void*)&gemm_batch_kernel<T, typename BatchTiles<T>::Small, 0, true>;
+}
+
 template <typename T>
 inline void variant_info(int mode, int v, const void*& fn, int& threads) {
     threads = v == 0 ? BatchTiles<T>::Big::NT : BatchTiles<T>::Small::NT;
@@ -442,6 +452,9 @@ struct BatchPlan {
     int grid[NMODE][NLAYOUT] = {};    // persistent grid per kernel mode and variant (layout)
     WorkItem* d_witems = nullptr;     // wave-tile mode: 32 x 32 tiles of every problem
     XcdSegs wseg[NLAYOUT] = {};       // per layout
+    WorkItem* d_gitems = nullptr;     // problems for guarded_fn, in no other list
+    XcdSegs gseg = {};
+    int ggrid = 0;
     int mode = 0;                     // kernel mode used by execute
     int vmode[NVARIANT] = {};         // per-variant kernel mode (mode != WAVE_MODE)
     // Single dispatch (gemm_batch_dyn_kernel): every variant's items in one
@@ -467,6 +480,7 @@ struct BatchPlan {
         if (d_descs) (void)hipFree(d_descs);
         if (d_items) (void)hipFree(d_items);
         if (d_witems) (void)hipFree(d_witems);
+        if (d_gitems) (void)hipFree(d_gitems);
         if (d_ditems) (void)hipFree(d_ditems);
         if (d_ctr) (void)hipFree(d_ctr);
     }
@@ -477,7 +491,7 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
     plan->dt = dt;
     std::vector<BatchDesc> descs;
     descs.reserve(probs.size());
-    std::vector<WorkItem> items;
+    std::vector<WorkItem> items, gitems;
     std::vector<int32_t> item_k;
     for (const BatchProblem& q0 : probs) {
         BatchProblem q = q0;
@@ -501,14 +515,15 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
             if (q.b.rs == 1) { d.ldb = q.b.cs; flags |= F_B_K; }
             else if (q.b.cs == 1) { d.ldb = q.b.rs; }
             else general = true;
-            // The kernels read through buffer descriptors; strides that do
-            // not allow it run as plain GEMMs.
+            // The kernels read through buffer descriptors, but for the one
+            // that takes the other strides.
             if (!general) {
                 const bool ak = flags & F_A_K, bk = flags & F_B_K;
                 d.lda = ak ? line_ld(d.lda, q.k, q.m) : line_ld(d.lda, q.m, q.k);
                 d.ldb = bk ? line_ld(d.ldb, q.k, q.n) : line_ld(d.ldb, q.n, q.k);
-                general = !buf_ok(d.lda, ak ? q.k : q.m, ak, 64, dt) ||
-                          !buf_ok(d.ldb, bk ? q.k : q.n, bk, 64, dt);
+                if (!buf_ok(d.lda, ak ? q.k : q.m, ak, 64, dt) ||
+                    !buf_ok(d.ldb, bk ? q.k : q.n, bk, 64, dt))
+                    flags |= F_GUARDED;
             }
         } else {
             d.lda = 1; d.ldb = 1;
@@ -527,8 +542,8 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
         // padded area by more than that.
         const bool small = (double)((q.m + 31) / 32) * (double)((q.n + 31) / 32) * 0.4 <
                            (double)((q.m + 63) / 64) * (double)((q.n + 63) / 64);
-        if (small) flags |= F_SMALL;
-        const int tb = small ? 32 : 64;
+        if (small || (flags & F_GUARDED)) flags |= F_SMALL;
+        const int tb = (flags & F_SMALL) ? 32 : 64;
         d.flags = flags;
         d.tiles_m = (int32_t)((q.m + tb - 1) / tb);
         d.tiles_m32 = (int32_t)((q.m + 31) / 32);
@@ -536,8 +551,12 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
         const int32_t pi = (int32_t)descs.size();
         descs.push_back(d);
         for (int64_t t = 0; t < (int64_t)d.tiles_m * tiles_n; ++t) {
-            items.push_back(WorkItem{ pi, (int32_t)t });
-            item_k.push_back(d.k);
+            if (flags & F_GUARDED) {
+                gitems.push_back(WorkItem{ pi, (int32_t)t });
+            } else {
+                items.push_back(WorkItem{ pi, (int32_t)t });
+                item_k.push_back(d.k);
+            }
         }
     }
     // Items are grouped by kernel variant, then by XCD list, then
@@ -587,7 +606,7 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
         }
     std::vector<WorkItem> sorted(ni);
     for (size_t i = 0; i < ni; ++i) sorted[i] = items[order[i]];
-    plan->nitems = (int)sorted.size();
+    plan->nitems = (int)(sorted.size() + gitems.size());
     if (!descs.empty()) {
         HIP_CHECK(hipMalloc(&plan->d_descs, descs.size() * sizeof(BatchDesc)));
         HIP_CHECK(hipMemcpyAsync(plan->d_descs, descs.data(), descs.size() * sizeof(BatchDesc),
@@ -606,6 +625,7 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
         std::vector<int32_t> wk, wv, wx;
         for (size_t pi = 0; pi < descs.size(); ++pi) {
             const BatchDesc& d = descs[pi];
+            if (d.flags & F_GUARDED) continue;
             const int64_t t = (int64_t)d.tiles_m32 * ((d.n + 31) / 32);
             const int lv = layout_of(d.flags);
             for (int64_t ti = 0; ti < t; ++ti) {
@@ -687,6 +707,26 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
         HIP_CHECK(hipMalloc(&plan->d_ctr, sizeof(zeros)));
         HIP_CHECK(hipMemcpyAsync(plan->d_ctr, zeros, sizeof(zeros), hipMemcpyHostToDevice, st));
     }
+    // Guarded problems: dealt over the XCD lists, longest first in each.
+    if (!gitems.empty()) {
+        std::stable_sort(gitems.begin(), gitems.end(), [&](const WorkItem& x, const WorkItem& y) {
+            if (x.prob % NXCD != y.prob % NXCD) return x.prob % NXCD < y.prob % NXCD;
+            return descs[x.prob].k > descs[y.prob].k;
+        });
+        for (const WorkItem& w : gitems) plan->gseg.off[w.prob % NXCD + 1]++;
+        int longest = 0;
+        for (int x = 0; x < NXCD; ++x) {
+            longest = std::max(longest, plan->gseg.off[x + 1]);
+            plan->gseg.off[x + 1] += plan->gseg.off[x];
+        }
+        int per_cu = 0;
+        HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &per_cu, dt == Dt::F64 ? guarded_fn<double>() : guarded_fn<float>(), 256, 0));
+        plan->ggrid = std::min(longest, cu_count() * std::max(1, per_cu) / NXCD) * NXCD;
+        HIP_CHECK(hipMalloc(&plan->d_gitems, gitems.size() * sizeof(WorkItem)));
+        HIP_CHECK(hipMemcpyAsync(plan->d_gitems, gitems.data(), gitems.size() * sizeof(WorkItem),
+                                 hipMemcpyHostToDevice, st));
+    }
     HIP_CHECK(hipStreamSynchronize(st));
     // Single dispatch: one resident wave of workgroups, a multiple of the
     // XCD count, and no more per XCD than its longest list.
@@ -762,7 +802,18 @@ static void launch_dyn(const BatchPlan* plan, int mode, hipStream_t st) {
     HIP_CHECK(hipLaunchKernel(fn, dim3(plan->dgrid[mode]), dim3(256), args, 0, st));
 }
 
+static void launch_guarded(const BatchPlan* plan, hipStream_t st) {
+    if (plan->ggrid == 0) return;
+    const void* fn = plan->dt == Dt::F64 ? guarded_fn<double>() : guarded_fn<float>();
+    const BatchDesc* descs = plan->d_descs;
+    const WorkItem* items = plan->d_gitems;
+    XcdSegs seg = plan->gseg;
+    void* args[] = {(void*)&descs, (void*)&items, (void*)&seg};
+    HIP_CHECK(hipLaunchKernel(fn, dim3(plan->ggrid), dim3(256), args, 0, st));
+}
+
 static void plan_launch(const BatchPlan* plan, hipStream_t st, bool with_fallback = true) {
+    launch_guarded(plan, st);
     if (plan->dyn && plan->mode != WAVE_MODE)
         launch_dyn(plan, plan->mode, st);
     else

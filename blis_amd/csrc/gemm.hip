@@ -31,7 +31,7 @@ using namespace dev;
 // splitk_reduce_kernel then forms C.
 template <typename T, class TL, bool A_K, bool B_K, bool BUF>
 __global__ __launch_bounds__(TL::NT)
-__attribute__((amdgpu_waves_per_eu(TL::waves_per_eu()))) void gemm_kernel(TileProblem<T> p, GridInfo g,
+__attribute__((amdgpu_waves_per_eu(TL::waves_per_eu(BUF)))) void gemm_kernel(TileProblem<T> p, GridInfo g,
                                                       int64_t kchunk, T* parts) {
     __shared__ T smem[2 * TL::STAGE];
     if (gridDim.y > 1) {
@@ -56,7 +56,7 @@ __attribute__((amdgpu_waves_per_eu(TL::waves_per_eu()))) void gemm_kernel(TilePr
 // C_z = C + z*sc.
 template <typename T, class TL, bool A_K, bool B_K, bool BUF>
 __global__ __launch_bounds__(TL::NT)
-__attribute__((amdgpu_waves_per_eu(TL::waves_per_eu()))) void gemm_strided_kernel(TileProblem<T> p, GridInfo g,
+__attribute__((amdgpu_waves_per_eu(TL::waves_per_eu(BUF)))) void gemm_strided_kernel(TileProblem<T> p, GridInfo g,
                                                               int64_t sa, int64_t sb, int64_t sc) {
     __shared__ T smem[2 * TL::STAGE];
     const int64_t z = blockIdx.y;
@@ -257,16 +257,18 @@ static void launch_tl(const TileProblem<T>& p, bool a_k, bool b_k, GridInfo g, c
 }
 
 // Every tile of the table reads its operands through buffer descriptors. A
-// problem whose strides do not allow that runs on one of two tiles built
-// without them, a large and a small one: the tile never changes the result.
+// problem whose strides do not allow that runs on one of three tiles built
+// without them, the one nearest in size: the tile never changes the result.
 template <typename T>
 static void launch_tile(int tile, const TileProblem<T>& p, bool a_k, bool b_k,
                         const GridInfo& g, const SplitK& sk, hipStream_t st) {
     const TileShape& ts = tile_shape(dt_of<T>(), tile);
     if (!buf_problem(p, a_k, b_k, ts.bm, ts.bn, ts.bk)) {
         constexpr int BK = std::is_same<T, double>::value ? 16 : 32;
-        if (ts.bm >= 64)
+        if (ts.bm * ts.bn > 64 * 64)
             launch_tl<T, TileCfg<T, 128, 64, BK, 32, 32>, false>(p, a_k, b_k, g, sk, st);
+        else if (ts.bm == 64)
+            launch_tl<T, TileCfg<T, 64, 64, BK, 32, 32>, false>(p, a_k, b_k, g, sk, st);
         else
             launch_tl<T, TileCfg<T, 32, 32, BK, 16, 16>, false>(p, a_k, b_k, g, sk, st);
         return;

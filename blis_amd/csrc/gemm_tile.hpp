@@ -107,13 +107,16 @@ struct TileCfg {
     // staged vectors, two sets of fragments and about 20 more) fit. The
     // unrolled k loop would take what it likes otherwise: 166 registers and
     // one workgroup per CU for the 128 x 128 FP64 tile, 17.8 ms at 8192^3
-    // against 15.0 ms with two.
-    static constexpr int waves_per_eu() {
+    // against 15.0 ms with two. Loads without a descriptor keep 64-bit addresses
+    // and bounds besides, so their kernels give up a workgroup for registers (the
+    // 128 x 64 FP64 tile spilled up to 15).
+    static constexpr int waves_per_eu(bool buf) {
         const int es = (int)sizeof(T) / 4, per = NW >= 4 ? NW / 4 : 1;
         const int regs = TM * TN * 4 * es + (NVA + NVB) * 4 + 2 * (TM + TN) * es + 20;
         int w = 163840 / (2 * STAGE * (int)sizeof(T)) * NW / 4;
         if (w > 8) w = 8;
         while (w > per && 512 / w / 8 * 8 < regs) w -= per;
+        if (!buf && w > per) w -= per;
         return w < 1 ? 1 : w;
     }
     static_assert(WM % 16 == 0 && WN % 16 == 0, "wave tile must be 16-aligned");
@@ -269,11 +272,12 @@ struct SlabLoader {
     }
 };
 
-// The same through a buffer descriptor with the layout decided at run time,
-// for kernels that walk problems of every layout (the batch): the layout only
-// enters a thread's offsets, the slab stride and the LDS store, so it costs a
-// uniform branch around the stores and no registers.
-template <typename T, class TL, int ROWS, int NV>
+// The same with the layout decided at run time, for kernels that walk problems
+// of every layout (the batch): the layout only enters a thread's offsets, the
+// slab stride and the LDS store, so it costs a uniform branch around the stores
+// and no registers. Not BUF: element loads behind bounds checks, for strides
+// that a descriptor does not take.
+template <typename T, class TL, int ROWS, int NV, bool BUF>
 struct SlabLoaderRt {
     using vec_t = typename Mma<T>::vec_t;
     static constexpr int V = TL::V;
@@ -283,32 +287,59 @@ struct SlabLoaderRt {
     vec_t r[NV];
     bool k_contig;
     const char* base;
-    int64_t left, adv;
+    int64_t left, adv;      // BUF: as SlabLoader's; else lines and length of a line left
     uint32_t off0, step;
+    int64_t ld;             // not BUF
 
-    __device__ inline void init(const T* x, int64_t rows, int64_t K, int64_t ld, int k_contig_,
+    __device__ inline void init(const T* x, int64_t rows, int64_t K, int64_t ld_, int k_contig_,
                                 int64_t row0, int tid) {
         constexpr int ES = (int)sizeof(T);
         k_contig = k_contig_ != 0;
-        const uint32_t line = (uint32_t)ld * ES;
         const int c = k_contig ? tid % CVK : tid % CVR, l = k_contig ? tid / CVK : tid / CVR;
-        off0 = (uint32_t)l * line + (uint32_t)(c * 16);
-        step = (uint32_t)(k_contig ? TL::NT / CVK : TL::NT / CVR) * line;
-        adv = (k_contig ? (int64_t)TL::BK : TL::BK * ld) * ES;
-        base = (const char*)(x + (k_contig ? row0 * ld : row0));
-        left = (k_contig ? (rows - 1 - row0) * ld + K : (K - 1) * ld + (rows - row0)) * ES;
+        if constexpr (BUF) {
+            const uint32_t line = (uint32_t)ld_ * ES;
+            off0 = (uint32_t)l * line + (uint32_t)(c * 16);
+            step = (uint32_t)(k_contig ? TL::NT / CVK : TL::NT / CVR) * line;
+            adv = (k_contig ? (int64_t)TL::BK : TL::BK * ld_) * ES;
+            base = (const char*)(x + (k_contig ? row0 * ld_ : row0));
+            left = (k_contig ? (rows - 1 - row0) * ld_ + K : (K - 1) * ld_ + (rows - row0)) * ES;
+        } else {
+            ld = ld_;
+            // This thread's first element, and what is left of lines and of a line
+            // from there; a slab moves along the line or to later lines.
+            base = (const char*)(x + (k_contig ? (row0 + l) * ld : row0 + l * ld) + c * V);
+            left = (k_contig ? rows - row0 : K) - l;
+            adv = (k_contig ? K : rows - row0) - c * V;
+        }
     }
 
     __device__ inline void load(int, int) {
-        const uint32_t n = (uint32_t)(left >> 32) != 0 ? 0xFFFFFFFFu : (uint32_t)left;
-        auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)n, 0x00020000);
+        if constexpr (BUF) {
+            const uint32_t n = (uint32_t)(left >> 32) != 0 ? 0xFFFFFFFFu : (uint32_t)left;
+            auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)n, 0x00020000);
 #pragma unroll
-        for (int q = 0; q < NV; ++q) {
-            auto t = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(off0 + q * step), 0, 0);
-            r[q] = __builtin_bit_cast(vec_t, t);
+            for (int q = 0; q < NV; ++q) {
+                auto t = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(off0 + q * step), 0, 0);
+                r[q] = __builtin_bit_cast(vec_t, t);
+            }
+            base += adv;
+            left -= adv;
+        } else {
+            const int lines = k_contig ? TL::NT / CVK : TL::NT / CVR;
+#pragma unroll
+            for (int q = 0; q < NV; ++q) {
+                const T* src = (const T*)base + q * lines * ld;
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    T val = T(0);
+                    if (q * lines < left && e < adv) val = src[e];
+                    r[q][e] = val;
+                }
+            }
+            base += (k_contig ? (int64_t)TL::BK : TL::BK * ld) * (int64_t)sizeof(T);
+            if (k_contig) adv -= TL::BK;
+            else left -= TL::BK;
         }
-        base += adv;
-        left -= adv;
     }
 
     __device__ inline void store(T* S, int kext, int tid) {
@@ -613,8 +644,8 @@ __device__ inline void prefetch_c(const TileProblem<T>& p, int64_t m0, int64_t n
 }
 
 // How a tile routine reads its operands: Guarded and Buffer are SlabLoader,
-// RuntimeLayout is SlabLoaderRt (A_K and B_K are not used then).
-enum class Loads { Guarded, Buffer, RuntimeLayout };
+// RuntimeLayout and RuntimeGuarded SlabLoaderRt (A_K and B_K are not used then).
+enum class Loads { Guarded, Buffer, RuntimeLayout, RuntimeGuarded };
 
 template <typename T, class TL, bool A_K, bool B_K, Loads LOADS, int PF, bool LDS_EPI,
           bool C_PF = false, bool MASK = false>
@@ -622,10 +653,11 @@ __device__ inline void gemm_tile_impl(const TileProblem<T>& p, int64_t m0, int64
                                       int* sink = nullptr, CMask cm = CMask{}) {
     static_assert(PF == 1 || PF == 2, "prefetch depth");
     using acc_t = typename Mma<T>::acc_t;
-    constexpr bool RT = LOADS == Loads::RuntimeLayout, BUF = LOADS == Loads::Buffer;
-    using Loader_A = typename std::conditional<RT, SlabLoaderRt<T, TL, TL::BM, TL::NVA>,
+    constexpr bool RT = LOADS == Loads::RuntimeLayout || LOADS == Loads::RuntimeGuarded;
+    constexpr bool BUF = LOADS == Loads::Buffer || LOADS == Loads::RuntimeLayout;
+    using Loader_A = typename std::conditional<RT, SlabLoaderRt<T, TL, TL::BM, TL::NVA, BUF>,
                                                SlabLoader<T, TL, TL::BM, A_K, TL::NVA, BUF>>::type;
-    using Loader_B = typename std::conditional<RT, SlabLoaderRt<T, TL, TL::BN, TL::NVB>,
+    using Loader_B = typename std::conditional<RT, SlabLoaderRt<T, TL, TL::BN, TL::NVB, BUF>,
                                                SlabLoader<T, TL, TL::BN, B_K, TL::NVB, BUF>>::type;
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;

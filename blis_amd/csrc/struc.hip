@@ -67,7 +67,7 @@ StrucSpec transposed(const StrucSpec& s) {
 // the early return is taken by the whole workgroup before any barrier.
 template <typename T, class TL, bool A_K, bool B_K, bool BUF, bool MASK>
 __global__ __launch_bounds__(TL::NT)
-__attribute__((amdgpu_waves_per_eu(TL::waves_per_eu()))) void gemm_struc_kernel(TileProblem<T> p, GridInfo g,
+__attribute__((amdgpu_waves_per_eu(TL::waves_per_eu(BUF)))) void gemm_struc_kernel(TileProblem<T> p, GridInfo g,
                                                             StrucSpec s, int64_t kchunk,
                                                             T* parts) {
     __shared__ T smem[2 * TL::STAGE];

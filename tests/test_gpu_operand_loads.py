@@ -169,28 +169,47 @@ def test_overlapping_frames(blis, dt):
 def test_batch_plan_takes_vectors_and_frames(blis, dt):
     """A plan runs them in its own kernels (they have work items), with the bits
     of single calls."""
+    # (m, n, k, ta, tb, lda, ldb)
+    _plan_against_calls(blis, dt, [
+        (100, 80, 1, 0, 0, 1, 1), (90, 1, 60, 0, 0, 90, 1), (1, 75, 64, 1, 0, 3, 64),
+        (70, 40, 100, 1, 0, 5, 100), (50, 66, 130, 0, 0, 50, 2), (130, 20, 33, 1, 0, 0, 33)])
+
+
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+def test_batch_plan_takes_backward_and_overlapping_lines(blis, dt):
+    """Strides that descriptors do not take, in either operand and layout, beside
+    problems that have none, in every mode of the plan and replayed from its
+    graph."""
+    _plan_against_calls(blis, dt, [
+        (100, 80, 70, 0, 0, -100, 70), (31, 33, 129, 1, 0, -129, 129), (65, 64, 1, 0, 1, 65, -64),
+        (64, 1, 300, 1, 0, -300, 300), (33, 97, 40, 0, 0, 33, -41), (17, 15, 16, 0, 0, 5, 16),
+        (128, 40, 65, 1, 1, -65, -40), (50, 50, 50, 0, 0, 50, 50), (200, 90, 33, 1, 0, 33, 33)],
+        modes=(0, 3, 4, 5, 7, 8))
+
+
+def _plan_against_calls(blis, dt, probs, modes=(None,)):
     ch, ct = ("d", C.c_double) if dt == torch.float64 else ("s", C.c_float)
     g = torch.Generator(device="cuda").manual_seed(23)
-    # (m, n, k, ta, tb, lda, ldb)
-    probs = [(100, 80, 1, 0, 0, 1, 1), (90, 1, 60, 0, 0, 90, 1), (1, 75, 64, 1, 0, 3, 64),
-             (70, 40, 100, 1, 0, 5, 100), (50, 66, 130, 0, 0, 50, 2), (130, 20, 33, 1, 0, 0, 33)]
-    buf = torch.rand(1 << 16, generator=g, device="cuda", dtype=dt) * 2 - 1
+    # (0, 0) of both operands lies in the middle of the buffer: lines may run
+    # backwards from there.
+    buf = torch.rand(1 << 17, generator=g, device="cuda", dtype=dt) * 2 - 1
+    pa, pb = buf[1 << 16:].data_ptr(), buf[(1 << 16) + 1000:].data_ptr()
     one, half = ct(1.0), ct(0.5)
-    outs, wants = [], []
+    outs, wants, starts = [], [], []
     for m, n, k, ta, tb, lda, ldb in probs:
         c = torch.rand(n, m, generator=g, device="cuda", dtype=dt)
         w = c.clone()
-        getattr(blis, f"bli_{ch}gemm")(8 * ta, 8 * tb, m, n, k, C.byref(one), buf.data_ptr(), 1,
-                                       lda, buf[1000:].data_ptr(), 1, ldb, C.byref(half),
-                                       w.data_ptr(), 1, m)
+        getattr(blis, f"bli_{ch}gemm")(8 * ta, 8 * tb, m, n, k, C.byref(one), pa, 1, lda, pb, 1,
+                                       ldb, C.byref(half), w.data_ptr(), 1, m)
         outs.append(c)
+        starts.append(c.clone())
         wants.append(w)
     real = np.float64 if dt == torch.float64 else np.float32
     col = lambda i, t=np.int64: np.array([p[i] for p in probs], t)
     ones, cnt = np.ones(len(probs), np.int64), len(probs)
     arrs = [col(3, np.int32) * 8, col(4, np.int32) * 8, col(0), col(1), col(2),
-            np.full(cnt, 1.0, real), np.full(cnt, buf.data_ptr(), np.int64), ones, col(5),
-            np.full(cnt, buf[1000:].data_ptr(), np.int64), ones, col(6), np.full(cnt, 0.5, real),
+            np.full(cnt, 1.0, real), np.full(cnt, pa, np.int64), ones, col(5),
+            np.full(cnt, pb, np.int64), ones, col(6), np.full(cnt, 0.5, real),
             np.array([c.data_ptr() for c in outs], np.int64), ones, col(0)]
     arrs = [np.ascontiguousarray(x, x.dtype) for x in arrs]
     torch.cuda.synchronize()
@@ -199,9 +218,17 @@ def test_batch_plan_takes_vectors_and_frames(blis, dt):
         *[x.ctypes.data for x in arrs], cnt, ones.ctypes.data)
     try:
         assert blis.bli_amd_gemm_batch_plan_work_items(plan) >= cnt
-        blis.bli_amd_gemm_batch_plan_execute(plan, 1)
-        torch.cuda.synchronize()
-        for c, w in zip(outs, wants):
-            assert torch.equal(c, w)
+        for mode in modes:
+            if mode is not None:
+                blis.bli_amd_gemm_batch_plan_set_mode(plan, mode)
+            for graph in (0, 1, 1):
+                say(f"loads batch plan {dt} mode={mode} graph={graph}")
+                for c, c0 in zip(outs, starts):
+                    c.copy_(c0)
+                torch.cuda.synchronize()
+                blis.bli_amd_gemm_batch_plan_execute(plan, graph)
+                torch.cuda.synchronize()
+                for c, w in zip(outs, wants):
+                    assert torch.equal(c, w)
     finally:
         blis.bli_amd_gemm_batch_plan_destroy(plan)
