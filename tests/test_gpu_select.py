@@ -305,3 +305,17 @@ def test_learned_selector_is_default_and_host_inference_matches(L):
                                                    int(sub["ldc"][i]))
                     for i in range(len(rows))])
     assert np.array_equal(got, want), np.where(got != want)[0][:10]
+
+
+def test_small_k_is_picked_as_sixteen(L):
+    """Below the k that the network was trained on, the pick is that of k = 16."""
+    L.bli_amd_gemm_selected_config.argtypes = [C.c_int] * 3 + [C.c_int64] * 6
+    assert L.bli_amd_gemm_get_selector() == 1        # the learned selector, the default
+    for dbl in (0, 1):
+        for m, n in [(711, 22), (2798, 208), (519, 1250), (6929, 7926), (3, 4000)]:
+            for k in (1, 4, 12, 15):
+                # N/T: the leading dimensions do not depend on k.
+                say(f"selector small k dbl={dbl} {m}x{n}x{k}")
+                pick = [L.bli_amd_gemm_selected_config(dbl, 0, 8, m, n, kk, m, n, m)
+                        for kk in (k, 16)]
+                assert pick[0] == pick[1]
