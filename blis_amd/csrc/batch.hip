@@ -486,6 +486,25 @@ struct BatchPlan {
     }
 };
 
+// The XCD list of every problem with work: greedily, largest first, to the
+// least loaded list of the problem's group (ties keep submission order).
+template <typename Group>
+static std::vector<int32_t> place_problems(const std::vector<double>& work, int groups,
+                                           Group group) {
+    std::vector<int32_t> order(work.size()), place(work.size(), 0);
+    std::iota(order.begin(), order.end(), 0);
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int32_t x, int32_t y) { return work[x] > work[y]; });
+    std::vector<double> load((size_t)groups * NXCD, 0.0);
+    for (int32_t pi : order) {
+        if (work[pi] == 0.0) continue;
+        double* l = load.data() + group(pi) * NXCD;
+        place[pi] = (int32_t)(std::min_element(l, l + NXCD) - l);
+        l[place[pi]] += work[pi];
+    }
+    return place;
+}
+
 static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipStream_t st) {
     auto* plan = new BatchPlan();
     plan->dt = dt;
@@ -564,7 +583,7 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
     // to XCD lists greedily, largest first, to the least-loaded list of their
     // variant (work = tile area x k summed over the problem's tiles).
     const size_t ni = items.size();
-    std::vector<int32_t> item_v(ni), prob_x(descs.size(), 0);
+    std::vector<int32_t> item_v(ni), prob_x;
     for (size_t i = 0; i < ni; ++i) item_v[i] = variant_of(descs[items[i].prob].flags);
     {
         std::vector<double> pwork(descs.size(), 0.0);
@@ -573,20 +592,7 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
             const double area = (d.flags & F_SMALL) ? 32.0 * 32.0 : 64.0 * 64.0;
             pwork[items[i].prob] += area * std::max<int32_t>(d.k, 1);
         }
-        std::vector<int32_t> porder(descs.size());
-        std::iota(porder.begin(), porder.end(), 0);
-        std::stable_sort(porder.begin(), porder.end(),
-                         [&](int32_t x, int32_t y) { return pwork[x] > pwork[y]; });
-        std::vector<double> load((size_t)NVARIANT * NXCD, 0.0);
-        for (int32_t pi : porder) {
-            if (pwork[pi] == 0.0) continue;
-            const int v = variant_of(descs[pi].flags);
-            int best = 0;
-            for (int x = 1; x < NXCD; ++x)
-                if (load[v * NXCD + x] < load[v * NXCD + best]) best = x;
-            prob_x[pi] = best;
-            load[v * NXCD + best] += pwork[pi];
-        }
+        prob_x = place_problems(pwork, NVARIANT, [&](int32_t pi) { return variant_of(descs[pi].flags); });
     }
     std::vector<int32_t> order(ni);
     std::iota(order.begin(), order.end(), 0);
@@ -618,11 +624,19 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
                                  hipMemcpyHostToDevice, st));
     }
     // Wave-tile items: every 32 x 32 tile of every problem, grouped by layout
-    // variant, then XCD list (same problem placement as above), then
-    // longest-first by k.
+    // variant, then XCD list, then longest-first by k. Each layout is a launch
+    // of its own, so problems are placed on the XCDs by layout.
     {
         std::vector<WorkItem> witems;
-        std::vector<int32_t> wk, wv, wx;
+        std::vector<int32_t> wk, wv, wx, place;
+        {
+            std::vector<double> pwork(descs.size(), 0.0);
+            for (size_t pi = 0; pi < descs.size(); ++pi)
+                if (!(descs[pi].flags & F_GUARDED))
+                    pwork[pi] = (double)descs[pi].tiles_m32 * ((descs[pi].n + 31) / 32) *
+                                std::max<int32_t>(descs[pi].k, 1);
+            place = place_problems(pwork, NLAYOUT, [&](int32_t pi) { return layout_of(descs[pi].flags); });
+        }
         for (size_t pi = 0; pi < descs.size(); ++pi) {
             const BatchDesc& d = descs[pi];
             if (d.flags & F_GUARDED) continue;
@@ -632,7 +646,7 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
                 witems.push_back(WorkItem{(int32_t)pi, (int32_t)ti});
                 wk.push_back(d.k);
                 wv.push_back(lv);
-                wx.push_back(prob_x[pi]);
+                wx.push_back(place[pi]);
             }
         }
         std::vector<int32_t> word(witems.size());
@@ -663,25 +677,14 @@ static BatchPlan* plan_build(Dt dt, const std::vector<BatchProblem>& probs, hipS
     // k slabs of 16 plus two for the epilogue, a 32 x 32 tile at 0.4 of a
     // 64 x 64 one), then longest tile first within each XCD (ties keep the
     // submission order, so a problem's tiles stay together).
-    std::vector<int32_t> dx(descs.size(), 0);
+    std::vector<int32_t> dx;
     {
         auto tile_cost = [&](const BatchDesc& d) {
             return ((d.flags & F_SMALL) ? 0.4 : 1.0) * (double)((std::max<int32_t>(d.k, 0) + 15) / 16 + 2);
         };
         std::vector<double> pwork(descs.size(), 0.0);
         for (size_t i = 0; i < ni; ++i) pwork[items[i].prob] += tile_cost(descs[items[i].prob]);
-        std::vector<int32_t> porder(descs.size());
-        std::iota(porder.begin(), porder.end(), 0);
-        std::stable_sort(porder.begin(), porder.end(),
-                         [&](int32_t x, int32_t y) { return pwork[x] > pwork[y]; });
-        double load[NXCD] = {};
-        for (int32_t pi : porder) {
-            int best = 0;
-            for (int x = 1; x < NXCD; ++x)
-                if (load[x] < load[best]) best = x;
-            dx[pi] = best;
-            load[best] += pwork[pi];
-        }
+        dx = place_problems(pwork, 1, [](int32_t) { return 0; });
         std::vector<int32_t> dord(ni);
         std::iota(dord.begin(), dord.end(), 0);
         std::stable_sort(dord.begin(), dord.end(), [&](int32_t x, int32_t y) {
