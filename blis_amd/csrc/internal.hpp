@@ -62,7 +62,7 @@ BLIS_AMD_HIDDEN void        sync_if_needed();
 // Grow-only device scratch, one buffer per slot: 0-1 GEMM operand packing
 // and transposes, 2-5 split-precision slices and statistics, 5-7 level-1/2
 // partials, 8-10 autotuner operands, 11-12 batch autotuner, 13-16 TRSM,
-// 14, 17 and 18 unused, 19 TRSM composition products, 20-21 dense
+// 17 and 18 unused, 19 TRSM composition products, 20-21 dense
 // copies of structured operands (symm/trmm) and trmm's copy of B, 22-24
 // complex GEMM (A in 1e format, B in 1r format, a column-major copy of C),
 // 25-27 mixed-datatype GEMM (A and B in the computation type, the product).
