@@ -131,13 +131,11 @@ def test_trsm_config2_residual(blis, dtype, uplo):
 @pytest.mark.parametrize("diag", [0, 0x100])
 @pytest.mark.parametrize("size", ["ragged", "whole"])
 def test_trsm_many_leaves(blis, oracle, dtype, side, uplo, ta, diag, size):
-    """Solves with several diagonal blocks and many right-hand sides, where
-    diagonal blocks that pass the dominance check are solved by products with
-    their inverses: a dominant triangle (every block takes the product path)
-    and one whose rows are not dominant (every block falls back to
-    substitution). "ragged": 700 rows, the last block partial (256-row
-    inverses); "whole": 1024 rows, whole 512-row blocks (inverses composed
-    from 64-row ones in the band store). Same bar as the small cases."""
+    """Solves of several leaves (up to 512 rows each, solved by substitution)
+    with updates between them, over many right-hand sides: a dominant triangle
+    and one whose rows are not dominant. "ragged": 700 rows, a last tile of 12
+    rows; "whole": 1024 rows, two full leaves. (Inverted blocks begin at 1536
+    rows: test_gpu_trsm_blocks.py.) Same bar as the small cases."""
     u = unit_roundoff(dtype)
     if size == "ragged":
         m, n = (700, 530) if side == 0 else (530, 700)
@@ -177,8 +175,7 @@ def test_trsm_many_leaves(blis, oracle, dtype, side, uplo, ta, diag, size):
 
 
 def test_trsm_many_leaves_async(blis, oracle):
-    """The same solves with the library in asynchronous mode (the solve waits
-    once, for the check of the diagonal blocks)."""
+    """The same solves with the library in asynchronous mode."""
     import torch
     m, n = 700, 530
     for kind, scale in (("dominant", None), ("not dominant", 2.0)):
@@ -213,10 +210,8 @@ def test_trsm_many_leaves_async(blis, oracle):
 @pytest.mark.parametrize("uplo", [LOWER, UPPER])
 @pytest.mark.parametrize("ta", ["n", "t"])
 def test_trsm_general_stride_dominant(blis, oracle, uplo, ta):
-    """A dominant triangle with neither a unit row nor a unit column stride,
-    large enough for 512-row blocks (700 rows): every diagonal block passes
-    the check, and the composed 512-row inverse, which multiplies
-    off-diagonal blocks in place, must not be used for such a triangle."""
+    """A dominant triangle with neither a unit row nor a unit column stride, of
+    two leaves: the leaves read it in place, the update packs its block."""
     m, n = 700, 530
     say(f"dtrsm general-stride A uplo={uplo:#x} {ta} m={m} n={n}")
     _, full = tri_matrix(m, uplo, False, np.float64, seed=m + 5)

@@ -85,6 +85,17 @@ def _check(blis, dt, left, uplo, trans, unit, q, r, alpha=1.0, tri_gap=0, rows_s
 
 
 @pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+@pytest.mark.parametrize("left", [True, False])
+@pytest.mark.parametrize("uplo", [LOWER, UPPER])
+@pytest.mark.parametrize("trans", [False, True])
+@pytest.mark.parametrize("unit", [False, True])
+def test_blocks_by_product(blis, dt, left, uplo, trans, unit):
+    _check(blis, dt, left, uplo, trans, unit, 1536, 512)
+    _check(blis, dt, left, uplo, trans, unit, 1600, 530, alpha=-0.75, pad=3, rows_stored=left)
+    _check(blis, dt, left, uplo, trans, unit, 2100, 515, alpha=2.0, pad=1, not_dominant=True)
+
+
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
 @pytest.mark.parametrize("uplo", [LOWER, UPPER])
 @pytest.mark.parametrize("trans", [False, True])
 @pytest.mark.parametrize("tri_gap", [1, 2])
@@ -92,3 +103,15 @@ def test_triangle_without_unit_stride(blis, dt, uplo, trans, tri_gap):
     _check(blis, dt, True, uplo, trans, False, 1700, 520, alpha=0.5, tri_gap=tri_gap)
     _check(blis, dt, False, uplo, trans, True, 1536, 513, tri_gap=tri_gap, rows_stored=True)
     _check(blis, dt, True, uplo, trans, False, 1600, 512, tri_gap=tri_gap, not_dominant=True)
+
+
+def test_blocks_by_product_asynchronous(blis):
+    """Calls that return before the device is done (the solve itself waits once,
+    for the check of the diagonal blocks)."""
+    blis.bli_amd_set_stream(None, 0)
+    try:
+        for not_dominant in (False, True):
+            _check(blis, torch.float64, True, LOWER, False, False, 1600, 530,
+                   not_dominant=not_dominant)
+    finally:
+        blis.bli_amd_set_stream(None, 1)
