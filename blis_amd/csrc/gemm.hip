@@ -298,19 +298,20 @@ static void transpose_run(Dt dt, const void* src, int64_t rows, int64_t cols, in
 }
 
 // The FP64 128x128 tile of sixteen 32x32 waves (tile 13) stages a
-// k-contiguous operand into LDS by transposing scalar stores, measured
-// about 4% slower (8192^3 NN vs NT) than its rows-contiguous path. For large
-// problems on that tile it pays to transpose the operand once (rows x k,
-// reused `reuse` times) and take the faster path; the arithmetic is the same
-// either way. The default large FP64 tile (6, eight 64x32 waves) stages it
-// within 1.2% of its rows-contiguous path, less than the transpose costs
-// (8192^3 NN: 16.11 ms as is, 16.23 ms transposed), so it takes the operand
-// as it comes.
+// k-contiguous operand into LDS by transposing scalar stores, which costs
+// about 2% of a large product. On that tile it pays to transpose the operand
+// once (rows x k, reused `reuse` times) and take the faster path; the
+// arithmetic is the same either way. us as is and transposed: A and B
+// k-contiguous at 8192^3 16192 / 16003 and 15770 / 15718, at 8192 x 8192 x
+// 1024 2193 / 2149 and 2148 / 2115; at 4096^3, where the rule says no, 2056 /
+// 2079 and 2002 / 2009. The default large FP64 tile (6, eight 64x32 waves)
+// loses at most 1.8% by it, about what the transpose costs, and takes the
+// operand as it comes.
 static bool transpose_pays(Dt dt, int64_t reuse, int64_t rows, int64_t k) {
     const double es = (double)dt_size(dt);
     const double gemm_s = 2.0 * (double)reuse * rows * k / (dt == Dt::F64 ? 60e12 : 120e12);
     const double tr_s = 2.0 * rows * k * es / 4e12 + 8e-6;
-    return 0.04 * gemm_s > tr_s;
+    return 0.02 * gemm_s > tr_s;
 }
 
 // k-contiguous operands of a large product to the rows-contiguous path, one
@@ -338,7 +339,7 @@ int gemm_default_tile(Dt dt, int64_t m, int64_t n, int64_t k) {
     // tiles so that enough workgroups exist to fill the 256 CUs.
     // Large shapes re-measured with exhaustive autotuning at m, n in
     // 4096..16384 and k in 128..8192: FP64 128x128 tiles of eight 64x32
-    // waves beat sixteen 32x32 waves by 4-8% (8192^3 NN 16.09 vs 16.82 ms);
+    // waves beat sixteen 32x32 waves by 4-8% (8192^3 NN 14.90 vs 15.72 ms);
     // FP32 short-k products prefer 128x64 tiles. Mid-size bands (256 to
     // 1023 tiles of 128x128) take the tile with the least total time over
     // the tuning database's shapes in that band.

@@ -65,10 +65,11 @@ bool launch_sup(const Plan& pl, double alpha, double beta, hipStream_t st) {
 
 } // namespace
 
-// Measured on MI355X (FP64, device time per call): 512^3 12.9 us against
-// 16.3 us on the table's 32 x 32 tile, 256^3 7.6 against 9.6, 128^3 5.8
-// against 6.4. Up to k = 64 the table tile (one 16-deep slab in flight) is
-// as fast or faster (64^3: 4.6 against 4.9 us), so those calls keep it.
+// Measured on MI355X (FP64, device time per call, N/T and N/N): 512^3 10.2
+// and 11.7 us against 11.8 and 11.9 on the table's 32 x 32 tile, 256^3 6.3 and
+// 7.1 against 7.1 and 7.2, 128^3 4.7 and 5.1 against 5.0 and 5.1. Up to k = 64
+// the table tile needs as many slabs (64^3: 3.9 and 4.1 us), so those calls
+// keep it.
 static bool sup_enabled() {
     static const bool on = [] {
         const char* e = std::getenv("BLIS_AMD_SUP");
@@ -83,10 +84,10 @@ bool gemm_sup_applies(int64_t m, int64_t n, int64_t k) {
 }
 
 // Table tile 4 is the 32 x 32 tile of four 16 x 16 waves: the sup kernel
-// computes the same tiles with deeper slabs. Measured (FP64, column-major,
-// ld 4096): 512 x 1024 x 512 20.1 us against 21.3 us; at k = 1024 the
-// 64-deep slabs allow only two workgroups per CU and lose (1024^3: 64.2
-// against 57.8 us), so the substitution stops at k = 512.
+// computes the same tiles with deeper slabs. With more workgroups than two
+// per CU, all that 64-deep slabs allow, it gains nothing any more (FP64, ld 4096,
+// 512 x 1024 x 512: N/T 15.5 us against 15.7, N/N 17.7 against 16.7), and at
+// k = 1024 it had lost (1024^3 64 us against 58), so it stops at k = 512.
 bool gemm_sup_deep_k(int tile, int parts, int64_t k) {
     return sup_enabled() && tile == 4 && parts <= 1 && k > 64 && k <= SMALL_GEMM_MAX_DIM;
 }
