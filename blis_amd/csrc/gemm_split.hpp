@@ -26,8 +26,8 @@ struct SplitChoice {
 // launched than fit the chip (`resident` per CU), and by the CU's matrix
 // cores (full per workgroup on the CU; no less than 2 bm bn bk flops at the
 // card's peak, 78.6 and 157.3 TFLOP/s over 256 CUs). The two overlap in part:
-// their hypotenuse fits plain products best. For parts > 1 the reduction
-// follows: its launch, a chain of `parts` additions, and one pass over the
+// their hypotenuse fits better than the larger of them. For parts > 1 the
+// reduction follows: its launch, a chain of `parts` additions, and one pass over the
 // partitions.
 struct TileCost {
     int tile, bm, bn, bk, resident;
@@ -40,15 +40,18 @@ struct SplitModel {
     // Masked products (gemmt, syrk) launch workgroups for all tiles, and those
     // of the tiles that are not stored end at once, which loads the CUs
     // unevenly: a CU's matrix cores serve this many workgroups more than an
-    // even spread of the others gives it.
+    // even spread of the others gives it (which hides the 64 x 64 tiles' latency).
     double uneven;
+    // Bytes per us at which all workgroups together read their operands (masked
+    // products over a deep k; no bound in sight for plain ones).
+    double operands;
 };
 
 // Fitted to the device times on these tiles with 1 to 64 partitions of 264 GEMM
 // and 98 SYRK shapes per type (m, n in [32, 8192], k in [128, 16384], SYRK to
 // 65536, each operand in both layouts): rms error 8% and 9% over 7,500 FP64
-// and 8,100 FP32 timings of GEMM, 11% and 13% for SYRK. The pair it picks is
-// within 2.4%, 3.1%, 3.8% and 6.9% of the best timing in geometric mean. A fit
+// and 8,100 FP32 timings of GEMM, 10% and 13% for SYRK. The pair it picks is
+// within 2.4%, 3.1%, 3.0% and 5.2% of the best timing in geometric mean. A fit
 // without the floor under `full` had given the 32 x 32 FP64 tile no throughput
 // limit, which sent every split product to it: 12% (GEMM) and 14% (SYRK)
 // from the best, 1024 x 1024 x 8192 at 404 us in place of 281.
@@ -57,18 +60,18 @@ inline const SplitModel& split_model(Dt dt, bool masked) {
         { 3, 64, 64, 16, 4, 0.698, 0.483, 4.4 },
         { 4, 32, 32, 16, 8, 0.420, 0.147, 4.7 },
         { 10, 64, 128, 16, 3, 0.620, 0.931, 5.9 },
-        { 6, 128, 128, 16, 2, 1.020, 1.783, 6.4 } }, 0.5, 0.18, 6.5e6, 0.0 };
+        { 6, 128, 128, 16, 2, 1.020, 1.783, 6.4 } }, 0.5, 0.18, 6.5e6, 0.0, 0.0 };
     static const SplitModel plain32 = { 4, {
         { 3, 64, 64, 32, 4, 0.929, 0.473, 4.3 },
         { 4, 32, 32, 32, 8, 0.468, 0.176, 4.2 },
         { 9, 128, 64, 32, 3, 1.096, 0.925, 4.6 },
-        { 10, 64, 128, 32, 3, 1.117, 0.911, 5.1 } }, 2.0, 0.255, 6.3e6, 0.0 };
+        { 10, 64, 128, 32, 3, 1.117, 0.911, 5.1 } }, 2.0, 0.255, 6.3e6, 0.0, 0.0 };
     static const SplitModel masked64 = { 2, {
-        { 3, 64, 64, 16, 4, 0.680, 0.498, 2.9 },
-        { 4, 32, 32, 16, 8, 0.419, 0.174, 2.5 } }, 3.0, 0.20, 9.5e6, 1.35 };
+        { 3, 64, 64, 16, 4, 0.094, 0.533, 3.2 },
+        { 4, 32, 32, 16, 8, 0.342, 0.165, 2.2 } }, 3.0, 0.20, 9.6e6, 1.19, 10.5e6 };
     static const SplitModel masked32 = { 2, {
-        { 3, 64, 64, 32, 4, 0.854, 0.502, 3.2 },
-        { 4, 32, 32, 32, 8, 0.495, 0.207, 2.1 } }, 3.0, 0.35, 5.7e6, 1.77 };
+        { 3, 64, 64, 32, 4, 0.0, 0.532, 3.4 },
+        { 4, 32, 32, 32, 8, 0.322, 0.200, 2.1 } }, 3.3, 0.33, 6.3e6, 1.59, 9.8e6 };
     return dt == Dt::F64 ? (masked ? masked64 : plain64) : (masked ? masked32 : plain32);
 }
 
@@ -85,7 +88,10 @@ inline double split_cost(Dt dt, const SplitModel& sm, const TileCost& t, int64_t
     const double lat = t.slab * (fits ? 1.0 : wgs / (256.0 * t.resident));
     const double thr = t.full * (masked ? 1.05 * wgs / 256.0 + sm.uneven
                                         : fits ? per_cu : wgs / 256.0 + 0.5);
-    double us = t.fixed + slabs * (masked ? std::max(lat, thr) : std::hypot(lat, thr));
+    double us = slabs * std::hypot(lat, thr);
+    if (sm.operands > 0.0)
+        us = std::max(us, tiles * (t.bm + t.bn) * (double)k * (double)dt_size(dt) / sm.operands);
+    us += t.fixed;
     if (parts > 1) {
         const double bytes = (2.0 * parts + 2.0) * (double)m * (double)n * (double)dt_size(dt);
         us += sm.reduce + sm.reduce_part * parts + (masked ? 0.6 : 1.0) * bytes / sm.rate;
