@@ -195,7 +195,11 @@ void* stream_scratch(size_t bytes, hipStream_t st) {
     it->used = ++s.split_clock;
     if (it->bytes < bytes) {
         // hipFree waits for the device, and so for every product that uses it.
-        if (it->p) HIP_CHECK(hipFree(it->p));
+        if (it->p && hipFree(it->p) != hipSuccess) {
+            (void)hipGetLastError();
+            it->bytes = 0;      // try again next time
+            return nullptr;
+        }
         // Whole 16 MiB steps: a program's shapes settle after a few calls.
         const size_t want = (bytes + ((size_t)16 << 20) - 1) >> 24 << 24;
         it->p = try_malloc(want);

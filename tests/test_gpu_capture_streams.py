@@ -131,3 +131,30 @@ def test_graphs_beside_eager_products(blis, own_stream):
     assert torch.equal(p1.out, want[p1]) and torch.equal(p2.out, want[p2])
     for o in outs:
         assert torch.equal(o, want[p3])
+
+
+def test_eager_product_grows_its_buffer_beside_a_capture(blis, own_stream):
+    """While one stream is captured, a product on another needs more room than
+    its stream has: neither disturbs the other."""
+    say("capture: an eager product on another stream in its midst")
+    st, side = torch.cuda.Stream(), torch.cuda.Stream()
+    small, large = Product(blis, 20, 128, 96, 8192), Product(blis, 21, 900, 850, 4096)
+    want = {p: p.alone(torch.cuda.Stream()) for p in (small, large)}
+    small.alone(side)
+    for p in (small, large):
+        p.out.fill_(7.0)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        blis.bli_amd_set_stream(st.cuda_stream, 0)
+        small.call()
+        blis.bli_amd_set_stream(side.cuda_stream, 0)
+        large.call()
+    torch.cuda.synchronize()
+    assert torch.equal(large.out, want[large])
+    for _ in range(3):
+        small.out.fill_(7.0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(small.out, want[small])
