@@ -571,6 +571,12 @@ hipStream_t check_stream() {
     return cs;
 }
 
+static bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIP_CHECK(hipStreamIsCapturing(st, &cap));
+    return cap != hipStreamCaptureStatusNone;
+}
+
 void trsm_run(Dt dt, side_t side, uplo_t uplo, trans_t trans, diag_t diag, int64_t m,
               int64_t n, double alpha, View a, View b, hipStream_t st) {
     if (m <= 0 || n <= 0) return;
@@ -601,9 +607,10 @@ void trsm_run(Dt dt, side_t side, uplo_t uplo, trans_t trans, diag_t diag, int64
     s.x = bv;
     // A large triangle over many columns: check its whole 512-row diagonal
     // blocks for dominance while they are inverted, and solve them by GEMM
-    // products when all pass.
+    // products when all pass. The host reads the check's flags, so a solve that
+    // is being captured is by substitution.
     const int64_t whole = rows / PB * PB;
-    if (rows >= TRSM_INV_MIN_ROWS && s.n >= TRSM_INV_MIN_N) {
+    if (rows >= TRSM_INV_MIN_ROWS && s.n >= TRSM_INV_MIN_N && !capturing(st)) {
         const size_t es = dt_size(dt);
         const int nblk = (int)(whole / NB);
         int* d_ok = (int*)workspace(sizeof(int) * nblk, 15);

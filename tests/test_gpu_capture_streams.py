@@ -158,3 +158,51 @@ def test_eager_product_grows_its_buffer_beside_a_capture(blis, own_stream):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(small.out, want[small])
+
+
+@pytest.mark.parametrize("rs", [1, 2])
+def test_captured_solve_of_a_large_dominant_triangle(blis, own_stream, rs):
+    """Captured, it is solved by substitution (inverted blocks need a check that
+    the host reads). Bound: as test_gpu_trsm_blocks.py's."""
+    q, r = 1600, 520
+    say(f"capture: large dominant solve rs={rs}")
+    g = torch.Generator(device="cuda").manual_seed(30)
+    a = torch.tril(torch.rand(q, q, generator=g, device="cuda", dtype=torch.float64) - 0.5)
+    a.diagonal().copy_(torch.rand(q, generator=g, device="cuda", dtype=torch.float64) + q)
+    buf = torch.full((q, rs * q), float("nan"), dtype=torch.float64, device="cuda")
+    buf[:, ::rs] = a.T
+    b0 = torch.rand(r, q, generator=g, device="cuda", dtype=torch.float64) - 0.5
+    x = b0.clone()
+
+    def call():
+        blis.bli_dtrsm(0, LOWER, 0, 0, q, r, C.byref(C.c_double(1.0)), buf.data_ptr(), rs, rs * q,
+                       x.data_ptr(), 1, q)
+
+    def check():
+        res = a @ x.T.contiguous() - b0.T
+        assert res.norm() <= 8 * q * 2.0 ** -53 * a.norm() * x.norm()
+
+    st = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    blis.bli_amd_set_stream(st.cuda_stream, 0)
+    # Eager first, by inverted blocks and (a row that is not dominant) by
+    # substitution, which sizes the workspace that a captured update packs into.
+    call()
+    torch.cuda.synchronize()
+    check()
+    off = buf[0, 100 * rs].item()
+    buf[0, 100 * rs] = 1e4
+    x.copy_(b0)
+    torch.cuda.synchronize()
+    call()
+    torch.cuda.synchronize()
+    buf[0, 100 * rs] = off
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        call()
+    for _ in range(3):
+        x.copy_(b0)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        check()
