@@ -70,6 +70,7 @@ BLIS_AMD_HIDDEN void        sync_if_needed();
 // products, constants).
 constexpr int WS_SLOTS = 32;
 BLIS_AMD_HIDDEN void*       workspace(size_t bytes, int slot);
+BLIS_AMD_HIDDEN void*       try_workspace(size_t bytes, int slot);   // nullptr without memory
 // Split-k partitions of products on stream st: a buffer of its own for each
 // of the last eight streams and for each stream of a capture, so that products
 // on several streams and in graphs replayed beside them do not share one.

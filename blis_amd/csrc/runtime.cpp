@@ -107,7 +107,14 @@ void sync_if_needed() {
     if (S().sync) HIP_CHECK(hipStreamSynchronize(S().stream));
 }
 
-void* workspace(size_t bytes, int slot) {
+static void* try_malloc(size_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+
+void* try_workspace(size_t bytes, int slot) {
     State& s = S();
     if (slot < 0 || slot >= WS_SLOTS) abort_with(BLIS_INVALID_UKR_ID, "workspace slot");
     std::lock_guard<std::mutex> g(s.ws_mutex);
@@ -122,16 +129,18 @@ void* workspace(size_t bytes, int slot) {
         }
         size_t want = bytes + bytes / 4;
         want = (want + 4095) & ~(size_t)4095;
-        void* p = nullptr;
-        hipError_t e = hipMalloc(&p, want);
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            abort_with(BLIS_MALLOC_RETURNED_NULL, "workspace allocation");
-        }
+        void* p = try_malloc(want);
+        if (p == nullptr) return nullptr;
         s.ws[slot] = p;
         s.ws_bytes[slot] = want;
     }
     return s.ws[slot];
+}
+
+void* workspace(size_t bytes, int slot) {
+    void* p = try_workspace(bytes, slot);
+    if (p == nullptr) abort_with(BLIS_MALLOC_RETURNED_NULL, "workspace allocation");
+    return p;
 }
 
 // hipMalloc and hipFree are refused while a stream is captured in a mode other
@@ -142,13 +151,6 @@ struct RelaxedCapture {
     RelaxedCapture() { HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode)); }
     ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
-
-static void* try_malloc(size_t bytes) {
-    void* p = nullptr;
-    if (hipMalloc(&p, bytes) == hipSuccess) return p;
-    (void)hipGetLastError();
-    return nullptr;
-}
 
 // Partitions of a product that is being captured. The graph holds the address
 // and may be replayed at any time on any stream, beside eager products and

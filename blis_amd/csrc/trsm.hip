@@ -610,11 +610,18 @@ void trsm_run(Dt dt, side_t side, uplo_t uplo, trans_t trans, diag_t diag, int64
     // products when all pass. The host reads the check's flags, so a solve that
     // is being captured is by substitution.
     const int64_t whole = rows / PB * PB;
+    const int nblk = (int)(whole / NB);
+    const size_t es = dt_size(dt);
+    const bool gather = s.a.rs != 1 && s.a.cs != 1;
+    int* d_ok = nullptr;
+    void *band = nullptr, *blocks = nullptr;
     if (rows >= TRSM_INV_MIN_ROWS && s.n >= TRSM_INV_MIN_N && !capturing(st)) {
-        const size_t es = dt_size(dt);
-        const int nblk = (int)(whole / NB);
-        int* d_ok = (int*)workspace(sizeof(int) * nblk, 15);
-        void* band = workspace((size_t)(whole + 1) * BAND_LD * es, 13);
+        d_ok = (int*)try_workspace(sizeof(int) * nblk, 15);
+        band = try_workspace((size_t)(whole + 1) * BAND_LD * es, 13);
+        if (gather) blocks = try_workspace((size_t)whole * (PB + 1) * es, 14);
+    }
+    // Substitution needs none of these, and is what is left without memory.
+    if (d_ok && band && (blocks || !gather)) {
         // The check runs on a side stream, beside the inversion on the main
         // stream; only the host reads its flags (pinned memory, one wait).
         hipStream_t cs = check_stream();
@@ -655,23 +662,22 @@ void trsm_run(Dt dt, side_t side, uplo_t uplo, trans_t trans, diag_t diag, int64
         // GPU stays busy while the host reads the flags.
         s.band = band;
         s.tri = s.a;
-        if (s.a.rs != 1 && s.a.cs != 1) {
+        if (gather) {
             // The composition's products need a unit stride. The updates pack
             // their blocks of the triangle themselves, as every GEMM does.
             // FP64 4096 x 1024 with strides 2 and 8192: 582 us, by
             // substitution 895.
-            void* w = workspace((size_t)whole * (PB + 1) * es, 14);
             const dim3 grid(28, (unsigned)(whole / PB)), block(256);
             if (dt == Dt::F64)
                 hipLaunchKernelGGL(trsm_gather_kernel<double>, grid, block, 0, st,
-                                   (const double*)s.a.ptr, s.a.rs, s.a.cs, (double*)w,
+                                   (const double*)s.a.ptr, s.a.rs, s.a.cs, (double*)blocks,
                                    (int)s.lower);
             else
                 hipLaunchKernelGGL(trsm_gather_kernel<float>, grid, block, 0, st,
-                                   (const float*)s.a.ptr, s.a.rs, s.a.cs, (float*)w,
+                                   (const float*)s.a.ptr, s.a.rs, s.a.cs, (float*)blocks,
                                    (int)s.lower);
             HIP_CHECK(hipGetLastError());
-            s.tri = { w, 1, PB };
+            s.tri = { blocks, 1, PB };
         }
         if (dt == Dt::F64) inverse_launch<double>(s, (int)(whole / LB));
         else inverse_launch<float>(s, (int)(whole / LB));
@@ -683,10 +689,11 @@ void trsm_run(Dt dt, side_t side, uplo_t uplo, trans_t trans, diag_t diag, int64
         HIP_CHECK(hipEventDestroy(ready));
         bool all = true;
         for (int i = 0; i < nblk; ++i) all = all && flags[i];
-        if (all) {
+        void* xbuf = all ? try_workspace((size_t)rows * s.n * es, 16) : nullptr;
+        if (xbuf) {
             // The right-hand side is updated in place and X is built in a
             // separate column-major buffer, copied over B once at the end.
-            s.x = { workspace((size_t)rows * s.n * es, 16), 1, rows };
+            s.x = { xbuf, 1, rows };
             solve(s, 0, rows, alpha);
             if (bv.rs == 1 && bv.cs == rows) {
                 // Column-stored without padding: one contiguous span, which

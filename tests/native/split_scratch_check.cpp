@@ -1,6 +1,6 @@
-// split_scratch_check.cpp — the pool of split-k partition buffers
-// (stream_scratch, runtime.cpp) on the CPU, against a model of the HIP calls it
-// makes. The model refuses what HIP refuses while a stream is captured:
+// split_scratch_check.cpp — the pool of split-k partition buffers and the
+// workspace that may fail (stream_scratch, try_workspace, runtime.cpp) on the
+// CPU, against a model of the HIP calls they make. The model refuses what HIP refuses while a stream is captured:
 // allocating and freeing unless the thread's capture mode is relaxed, and any
 // wait for a captured stream or the device. Prints "ok", or what went wrong.
 #include "../../blis_amd/csrc/runtime.cpp"
@@ -130,12 +130,15 @@ int main() {
     end(30);
     // No memory: the caller makes one pass; later calls ask again.
     memory_left = false;
+    if (blis_amd::try_workspace(4 << 20, 13) != nullptr) fail("a workspace without memory");
     if (take(4, 40) != nullptr) fail("a buffer without memory");
     begin(41, 11);
     if (take(4, 41) != nullptr) fail("a captured buffer without memory");
     end(41);
     memory_left = true;
-    if (take(4, 40) == nullptr) fail("memory is back");
+    if (take(4, 40) == nullptr || blis_amd::try_workspace(4 << 20, 13) == nullptr)
+        fail("memory is back");
+    hipFree(blis_amd::workspace(4 << 20, 13));
     // What graphs hold is bounded, and so are the streams' buffers.
     bool refused_one = false;
     for (unsigned long long id = 100; id < 200; ++id) {
