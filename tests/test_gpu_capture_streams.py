@@ -160,6 +160,23 @@ def test_eager_product_grows_its_buffer_beside_a_capture(blis, own_stream):
         assert torch.equal(small.out, want[small])
 
 
+def test_products_in_flight_on_more_streams_than_buffers(blis, own_stream):
+    """A stream beyond the eighth takes the longest unused buffer, whose product
+    may still run: nothing is waited for between the calls."""
+    say("streams: products in flight on twelve streams")
+    p = Product(blis, 22, 600, 550, 6000)
+    want = p.alone(torch.cuda.Stream())
+    streams = [torch.cuda.Stream() for _ in range(12)]
+    outs = [torch.empty_like(want) for _ in range(36)]
+    torch.cuda.synchronize()
+    for i, o in enumerate(outs):
+        blis.bli_amd_set_stream(streams[i % 12].cuda_stream, 0)
+        p.call(o)
+    torch.cuda.synchronize()
+    for o in outs:
+        assert torch.equal(o, want)
+
+
 @pytest.mark.parametrize("rs", [1, 2])
 def test_captured_solve_of_a_large_dominant_triangle(blis, own_stream, rs):
     """Captured, it is solved by substitution (inverted blocks need a check that
